@@ -52,23 +52,23 @@ def fgp_traffic(kernel: str):
     return float(m.group(1)) if m else None
 
 
+def fgp_passes(inner: int) -> list[int]:
+    """FGP steps of each pass of one prox call: as few passes of at most four steps as it needs, of
+    nearly equal length, the longer ones first (TvState::prox)."""
+    passes = (inner + 3) // 4
+    return [inner // passes + (k < inner % passes) for k in range(passes)]
+
+
 def fgp_pass_volumes(inner: int) -> list[int]:
-    """Volumes (b, dual components) each FGP launch of one prox call must read and write, in the
-    order TvState::prox issues them: two steps per pass, a single last step for odd counts. A
-    pass reads b and p_k (3), plus p_{k-1} (3) except on the first step of the call (r = p
-    there); it writes p_{k+1} (3, skipped by a last pass of two steps) and p_{k+2} (3)."""
+    """Volumes (b, dual components, output) each FGP launch of one prox call must read and write.
+    A pass of T steps reads b and p_k (3), plus p_{k-1} (3) except in the first (r = p there); it
+    writes p_{k+T-1} (3; not the last pass, nor one of a single step) and p_{k+T} (3), the last
+    pass the output as well."""
     out = []
-    k = 0
-    while k < inner:
-        first = k == 0
-        reads = 1 + 3 + (0 if first else 3)
-        if k + 1 < inner:
-            last = k + 2 == inner
-            out.append(reads + (3 if last else 6))
-            k += 2
-        else:
-            out.append(reads + 3)
-            k += 1
+    steps = fgp_passes(inner)
+    for k, t in enumerate(steps):
+        last = k + 1 == len(steps)
+        out.append(1 + 3 + (3 if k else 0) + 3 + (1 if last else 3 if t > 1 else 0))
     return out
 
 
@@ -79,7 +79,7 @@ def reconstruction_bytes(count: int, holo: int, n: int, nz: int, iterations: int
     one write of its array however many passes it takes. Front end as the algorithmic model of
     the reference's stages (hologram R2C, crop, inverse, ratio, unwrap, Rytov, 2D FFT); mapping
     with uint16 hit counts; per outer iteration the five transform kernels (momentum fused into
-    the first, the data restore into the z pass), the FGP passes and the primal."""
+    the first, the data restore into the z pass) and the FGP passes (the last forms the output)."""
     a, nh, m = count, holo, n
     v = nz * n * n
     h = nz * n * (n // 2 + 1)
@@ -96,7 +96,7 @@ def reconstruction_bytes(count: int, holo: int, n: int, nz: int, iterations: int
              + 10 * v + 9 * h                            # Hermitian data and hits
              + 8 * h + 4 * v)                            # initial C2R
     transforms = (8 * v + 8 * h) + 16 * h + 25 * h + 16 * h + (8 * h + 4 * v)
-    prox = (sum(fgp_pass_volumes(inner)) + 5) * 4 * v
+    prox = sum(fgp_pass_volumes(inner)) * 4 * v
     return int(front + iterations * (transforms + prox))
 
 
@@ -230,8 +230,8 @@ def streaming_reference(torch, mib=256, reps=20):
 
 
 def fgp_traffic_run(qh, torch, n: int = N) -> int:
-    """One TV prox of 10 FGP steps on an n^3 volume (five two-step passes, plus the prox's fill
-    and primal kernels) and one copy of a 256 MiB buffer (reads and writes exactly 256 MiB) as
+    """One TV prox of 10 FGP steps on an n^3 volume (three passes, plus the prox's fill) and one
+    copy of a 256 MiB buffer (reads and writes exactly 256 MiB) as
     the counter calibration."""
     from qoraholo_amd import _native
 
@@ -249,7 +249,7 @@ def fgp_traffic_run(qh, torch, n: int = N) -> int:
     b = torch.full_like(src, 3.0)
     torch.addcmul(src, a, b, out=dst)
     torch.cuda.synchronize()
-    log(f"fgp traffic run: 10 FGP steps in 5 passes at {n}^3, a 268435456-byte copy and an "
+    log(f"fgp traffic run: 10 FGP steps in 3 passes at {n}^3, a 268435456-byte copy and an "
         "addcmul of three 268435456-byte inputs")
     return 0
 
@@ -860,17 +860,17 @@ def main() -> int:
     vol_bytes = N * N * N * 4
     launches = max(1, t["fgp_launches"])
     steps_per_launch = t["fgp_steps"] / launches
-    kernel = "fgp_pair" if steps_per_launch == 2 else "fgp_step"
+    kernel = "fgp_steps"
     passes = fgp_pass_volumes(INNER)
     assert len(passes) * ITERATIONS == launches, (passes, launches)
     # What the launches must move: per pass b and the dual iterates it reads, the iterates it
-    # writes (13 volumes for a two-step pass inside a prox call, 10 for its first and last).
+    # writes and the output (10, 13 and 11 volumes for the passes of 4, 3 and 3 steps).
     alg_bytes = ITERATIONS * sum(passes) * vol_bytes
     fgp_avg_ms = t["fgp_ms"] / launches
     per_launch = alg_bytes / launches
     achieved = per_launch / (fgp_avg_ms * 1e-3) / 1e9
     # The reference's model: 13 volumes per step (read b, r(3), p(3); write p(3), r(3)). A pass
-    # of two steps moves half of that, so its rate on this model can exceed the peak.
+    # of several steps moves that once, so its rate on this model can exceed the peak.
     ref_bytes = int(13 * vol_bytes * steps_per_launch)
     roofline = {
         "bound": "hbm",
@@ -890,8 +890,7 @@ def main() -> int:
     }
     if roofline["traffic"]:
         # The physical rate: measured HBM bytes of the average launch of a prox call (the mean
-        # over its passes, which move 10, 13, 13, 13 and 10 volumes) over the mean launch
-        # duration of the same passes.
+        # over its passes) over the mean launch duration of the same passes.
         roofline["traffic_gbs"] = round(roofline["traffic"] / (fgp_avg_ms * 1e-3) / 1e9, 1)
         roofline["traffic_frac"] = round(roofline["traffic_gbs"] / HBM_PEAK_GBS, 4)
     roofline["streaming_reference"] = streaming_reference(torch)

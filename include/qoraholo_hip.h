@@ -82,8 +82,8 @@ typedef struct {
 } qh_odt_options;
 
 /* src/backends.hpp:31-42 (OdtTimings), device event intervals in milliseconds, plus the summed
- * duration of the FGP dual-step kernels, the steps and the kernel passes they took (two steps
- * per pass where the row width allows; FISTA-TV only). */
+ * duration of the FGP dual-step kernels, the steps and the kernel passes they took (up to four
+ * steps per pass, the last of which forms the output; FISTA-TV only). */
 typedef struct {
   size_t bytes;
   double setup;
@@ -432,8 +432,8 @@ int qh_hip_fft_c2c(qh_c64* data, int d0, int d1, int d2, unsigned axes, int forw
 int qh_hip_rfft3(const float* x, int nz, int ny, int nx, qh_c64* out);
 int qh_hip_irfft3(const qh_c64* in, int nz, int ny, int nx, float scale, float* x);
 /* One TV prox call from a zero dual: argmin 0.5 |x - b|^2 + lambda TV(x), x >= 0
- * (src/cpu/tv.cpp:7-44). fused: 1 runs the FGP steps two per pass where the row width allows
- * (what the solvers do), 0 one per pass; the results are the same bits. */
+ * (src/cpu/tv.cpp:7-44). fused: 1 runs up to four FGP steps per pass (what the solvers do),
+ * 0 one per pass; the results are the same bits. */
 int qh_hip_tv_prox(const float* b, int nz, int ny, int nx, float lambda, int inner, int fused,
                    float* x);
 /* qh_hip_tv_prox of `batch` volumes at once (no counterpart in the reference, whose tv_prox

@@ -18,7 +18,7 @@ Array3<cfloat> extract_fields(const Array3<float>& holograms, const CropPlan& pl
 Array3<float> unwrap(const Array3<float>& wrapped);
 Array3<cfloat> rytov(const Array3<cfloat>& ratio);
 // tv_kernel selects among the CUDA backend's FGP kernels for its benchmark (all do the same
-// arithmetic); the HIP backend has one FGP implementation, two steps per pass and equal to
+// arithmetic); the HIP backend has one FGP implementation, up to four steps per pass and equal to
 // single steps bit for bit, which every value runs.
 OdtResult reconstruct(const Array3<cfloat>& rytov_fields, std::span<const Illumination> illum,
                       const detail::OdtGrid& grid, const Geometry& geometry,

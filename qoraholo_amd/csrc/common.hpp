@@ -70,31 +70,6 @@ QH_HD void hermitian_restore(float are, float aim, int hits, float& re, float& i
   im = aim + b * im;
 }
 
-// Primal point of the TV dual: max(b - lambda L(p), 0). common.hpp:121-124.
-QH_HD float tv_primal(float b, float lambda, float adjoint) {
-  const float x = b - lambda * adjoint;
-  return x > 0.0f ? x : 0.0f;
-}
-
-// One FGP dual step at a voxel: q = r + step g, p' = q / max(1, |q|), r' = p' + m (p' - p).
-// common.hpp:128-141.
-QH_HD void tv_dual_step(const float g[3], float step, float momentum, float p[3], float r[3]) {
-  float q[3];
-  float norm2 = 0.0f;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    q[a] = r[a] + step * g[a];
-    norm2 += q[a] * q[a];
-  }
-  const float scale = norm2 > 1.0f ? 1.0f / sqrtf(norm2) : 1.0f;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const float next = q[a] * scale;
-    r[a] = next + momentum * (next - p[a]);
-    p[a] = next;
-  }
-}
-
 // t_{k+1} of FISTA and FGP. common.hpp:153.
 QH_HD float fista_t(float t) { return 0.5f * (1.0f + sqrtf(1.0f + 4.0f * t * t)); }
 
@@ -103,6 +78,12 @@ QH_HD float index_from_potential(float re, float im, float nm2, float inv_k02) {
   const float a = nm2 + re * inv_k02;
   const float b = im * inv_k02;
   return sqrtf(0.5f * (hypotf(a, b) + a));
+}
+
+// The same for a real potential, whose modulus is |a|: the bits of index_from_potential(re, 0).
+QH_HD float index_from_real(float re, float nm2, float inv_k02) {
+  const float a = nm2 + re * inv_k02;
+  return sqrtf(0.5f * (fabsf(a) + a));
 }
 
 // One slice of the multi-slice BPM on a spectrum bin and its adjoint. common.hpp:158-176.

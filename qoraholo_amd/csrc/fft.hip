@@ -223,8 +223,8 @@ __global__ void __launch_bounds__(kThreads) k_irfft_rows(RowsArgs a) {
     float u0 = v.x * a.op.a;
     float u1 = v.y * a.op.a;
     if (a.op.out == RealOut::index) {
-      u0 = index_from_potential(u0, 0.0f, a.op.nm2, a.op.inv_k02);
-      u1 = index_from_potential(u1, 0.0f, a.op.nm2, a.op.inv_k02);
+      u0 = index_from_real(u0, a.op.nm2, a.op.inv_k02);
+      u1 = index_from_real(u1, a.op.nm2, a.op.inv_k02);
     }
     float* px = a.xo + (r0 + line) * a.x_pitch + 2 * j;
     px[0] = u0;
@@ -527,8 +527,8 @@ __global__ void __launch_bounds__((Shape4<N1, N2>::BLOCK)) k_irfft4s_rows(RowsAr
       float u0 = w[k1].x * a.op.a;
       float u1 = w[k1].y * a.op.a;
       if (a.op.out == RealOut::index) {
-        u0 = index_from_potential(u0, 0.0f, a.op.nm2, a.op.inv_k02);
-        u1 = index_from_potential(u1, 0.0f, a.op.nm2, a.op.inv_k02);
+        u0 = index_from_real(u0, a.op.nm2, a.op.inv_k02);
+        u1 = index_from_real(u1, a.op.nm2, a.op.inv_k02);
       }
       *reinterpret_cast<float2*>(a.xo + row * a.x_pitch + 2 * m) = float2{u0, u1};
     }

@@ -208,6 +208,7 @@ OdtSolver::OdtSolver(const OdtGrid& g, int count, const OdtConfig& c, int batch)
       x_[1].resize(nb * vol_);
       x_[2].resize(nb * vol_);
       tv_state_ = std::make_unique<TvState>(g.nz, g.n, g.n, batch);
+      tv_state_->set_exact(false);
       fgp_events_.resize(2 * c.iterations);
     }
   } else if (c.iterations > 0) {

@@ -1,21 +1,32 @@
 // Total-variation proximal step by fast gradient projection on the dual (FGP), the inner loop
 // of FISTA-TV, on gfx950.
 //
-// One wavefront per block owns a strip of TY rows of the volume, each lane VX consecutive x
-// positions of every row (a whole 256-wide row is 64 lanes x 4 floats, loaded as float4), and
-// marches along z through a chunk of planes. y neighbours are in the lane's own registers, x
-// neighbours one lane away (shuffles), z neighbours in the registers of the previous plane; only
-// one halo row above and below the strip (and one plane at the chunk start) is read twice.
+// k_fgp_steps runs up to four FGP steps per pass over the volume. The extrapolated dual
+// r_k = p_k + m_{k-1} (p_k - p_{k-1}) is not stored: a pass of T steps reads b and the two latest
+// dual iterates p_k, p_{k-1} and writes p_{k+T-1} and p_{k+T}, 7 volumes in and 6 out. The first
+// pass of a prox starts from r = p_k (src/cpu/tv.cpp:10) and reads no p_{k-1}; the last one forms
+// the prox output as it goes and writes no p_{k+T-1}.
 //
-// The extrapolated dual r_k = p_k + m_{k-1} (p_k - p_{k-1}) is not stored: each step reads the
-// two latest dual iterates and forms r with the same float operations the reference's dual step
-// uses to produce it (src/common.hpp:128-141), so a step reads b, p_k, p_{k-1} and writes p_{k+1}
-// (10 volumes instead of 13 with r stored). The first step of a prox uses r = p_k
-// (src/cpu/tv.cpp:10).
+// The dual is the library's own, laid out for these accesses: within each plane of a component,
+// rows go in groups of four ("quads"), stored column by column, so that the four rows of a column
+// are 16 consecutive bytes and a 128-byte line holds 4 rows of 8 columns. A wave loads or stores
+// its 64 columns x 4 rows as one 16-byte access per lane, and tiles cut at multiples of 8 columns
+// and 4 rows share no line they write. With plain rows a tile of 64 columns wrote parts of lines
+// and the 256^3 pass of three steps took 290-350 us against 220 us (a kernel that only moves the
+// same data in that pattern took 326 us cut at 58 columns, 231 us cut at 48, and 186-202 us in
+// quads).
+//
+// Per prox of 10 steps, output included (4 + 3 + 3 steps), against two steps per pass and a kernel
+// for the output before: 671 against 837 us at 256^3, 1131 against 2635 us at 320^3, 1952 against
+// 3183 us at 384^3, 158 against 184 us at 128^3 and 73 against 131 us at 64^3. What bounds it: a
+// middle pass moves its 13 volumes at 4-5 TB/s with the halo re-reads (a device copy reaches 4.9),
+// a first or last pass of four stages is near its vector work (42 instructions a point and step,
+// and only 24 of 32 rows and 56 of 64 columns of a tile are its own).
 #include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
+#include "fft_core.hpp"
 #include "runtime.hpp"
 #include "tv.hpp"
 
@@ -23,755 +34,386 @@ namespace qh {
 
 namespace {
 
-constexpr int kZChunk = 16;
+// The arithmetic of a step, in two forms. EXACT: every operation rounded on its own, in the order
+// of the reference's expressions (src/common.hpp:121-141), and the projection's 1 / sqrt(n) the
+// float nearest to 1 / (float nearest to sqrt(n)); the bits of the reference's expressions, which
+// the data terms of the BPM inversion are compared by. Otherwise multiply-adds are fused and
+// 1 / sqrt(n) takes one Newton step from the hardware's: nearer to real arithmetic by itself and 11%
+// faster over a 256^3 prox of 10 steps (744 -> 670 us).
+template <bool EXACT>
+__device__ __forceinline__ float multiply_add(float a, float x, float y) {
+  return EXACT ? y + a * x : fmaf(a, x, y);
+}
 
-struct TvArgs {
-  const float* b;       // primal data, dense (nz, ny, nx)
-  const float* p_in;    // dual p_k, three components `vol` floats apart
-  const float* p_prev;  // dual p_{k-1} (unused on the first step)
-  float* p_out;         // dual p_{k+1}, a third buffer
-  long vol;
-  int nz, ny, nx;
-  float lambda;
-  float step;
-  float momentum;  // m_{k-1}, the momentum of the step that produced p_k
-  int first;       // r = p_k exactly
-  int zlen = kZChunk;  // planes per chunk of the strip kernels (strip_grid)
+// max(b - lambda L(r), 0) from the components of r at a point and at its lower neighbours, added
+// in the order of the negative divergence L(r)(i) = sum_a r_a(i) - r_a(i - e_a), axes z, y, x. A
+// component is zero on the last plane, row or column along its axis (its difference is), and the
+// neighbour before the first counts as zero, so the faces need no case of their own.
+template <bool EXACT>
+__device__ __forceinline__ float primal_value(float b, float lambda, float rz, float rz_below,
+                                              float ry, float ry_up, float rx, float rx_left) {
+  float s = rz - rz_below;
+  s += ry;
+  s -= ry_up;
+  s += rx;
+  s -= rx_left;
+  return fmaxf(multiply_add<EXACT>(-lambda, s, b), 0.0f);
+}
+
+// 1 / max(1, sqrt(norm2)) from the hardware's reciprocal square root y. EXACT: g = n y corrected
+// once is the nearest float to sqrt(n), and y corrected once against that the nearest to its
+// reciprocal: the bits of 1.0f / sqrtf(n) for every float n from 1 up to the last 128 before
+// overflow (all of them compared on the device), in 8 operations instead of the compiler's 25. The
+// bounds keep the limits of the division: 0 for an infinite norm, whose residuals are NaN; a NaN
+// norm counts as below one, as in norm2 > 1 ? ... : 1.
+template <bool EXACT>
+__device__ __forceinline__ float ball_scale(float norm2) {
+  const float n = fmaxf(norm2, 1.0f);
+  const float y = __builtin_amdgcn_rsqf(n);
+  const float g = n * y;
+  const float h = 0.5f * y;
+  if constexpr (EXACT) {
+    const float root = fmaf(fmaf(-g, g, n), h, g);
+    return fmaxf(fmaf(fmaf(-root, y, 1.0f), y, y), 0.0f);
+  } else {
+    return fmaf(h, fmaxf(fmaf(-g, y, 1.0f), -1.0f), y);
+  }
+}
+
+// The value of the lane below (lane 0: zero) and of the lane above (lane 63: zero).
+__device__ __forceinline__ float lane_below(float v) {
+  constexpr int kWaveShr1 = 0x138;
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kWaveShr1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_above(float v) {
+  constexpr int kWaveShl1 = 0x130;
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kWaveShl1, 0xf, 0xf, true));
+}
+
+// A window of device memory in scalar registers: an access at a byte offset past its end loads
+// zero or stores nothing. So faces, halos and arrays that a pass does without need no branch, and
+// the compiler knows how many accesses are in flight (with stores in branches it waits for all of
+// them where it needs the loads before them).
+constexpr unsigned kOutside = 0x80000000u;  // past the end of every window
+struct Window {
+  typedef unsigned quad __attribute__((ext_vector_type(4)));
+  static constexpr int kNonTemporal = 2;
+  __amdgpu_buffer_rsrc_t rsrc;
+  // `bytes` from p, or nothing where not `on` (the same for the whole wave).
+  __device__ __forceinline__ Window(const float* p, int bytes, bool on)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, on ? bytes : 0,
+                                               0x00020000)) {}
+  __device__ __forceinline__ float load(unsigned at) const {
+    return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, 0));
+  }
+  __device__ __forceinline__ void store(float v, unsigned at) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), rsrc, at, 0, 0);
+  }
+  __device__ __forceinline__ void load4(float (&v)[4], unsigned at) const {
+    const quad q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(q[j]);
+  }
+  // Non-temporal: the dual iterates are all written before the next pass reads them.
+  __device__ __forceinline__ void stream4(const float (&v)[4], unsigned at) const {
+    quad q;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q[j] = __float_as_uint(v[j]);
+    __builtin_amdgcn_raw_buffer_store_b128(q, rsrc, at, 0, kNonTemporal);
+  }
+  __device__ __forceinline__ void stream(float v, unsigned at) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), rsrc, at, 0, kNonTemporal);
+  }
 };
 
-// Volume blockIdx.y of a batch of volumes that lie one after another: its primal data and
-// output start blockIdx.y vol floats in, its duals (three components each) 3 blockIdx.y vol in.
-// Kernels apply the offsets only in their BATCH instantiations, which single volumes never run:
-// the offsets cost the 256^3 two-step pass 1.3% (154.7 -> 156.8 us) when always applied.
-__device__ __forceinline__ long batch_volume() { return static_cast<long>(blockIdx.y); }
-template <class T>
-__device__ __forceinline__ T* shifted(T* p, long by) {
-  return p == nullptr ? p : p + by;
-}
-
-// Block b runs tile t: with a grid that is a multiple of 8, blocks b, b+8, b+16, ... (which the
-// dispatcher places on the same XCD) get consecutive tiles, so the halo rows and the planes
-// shared by neighbouring tiles are read through the same L2.
-__device__ __forceinline__ int xcd_tile() {
-  const int nb = static_cast<int>(gridDim.x);
-  const int b = static_cast<int>(blockIdx.x);
-  return (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
-}
-
-// Row access. VEC: nx is a multiple of VX and VX of 2, so a lane's VX values are all inside the
-// row or all outside it and every access is whole float4s (float2s when VX is not a multiple of
-// 4) under one predicate per lane; otherwise element by element.
-// XNEG: xb may be negative (the left halo of an x tile); other callers start rows at column 0.
-template <int VX, bool VEC, bool XNEG = false, bool NT = false>
-__device__ __forceinline__ void load_row(const float* base, const TvArgs& a, int z, int y, int xb,
-                                         float (&out)[VX]) {
-  const bool inside = z >= 0 && z < a.nz && y >= 0 && y < a.ny;
-  if constexpr (VEC) {
-    static_assert(VX % 2 == 0, "whole float2s");
-    if (inside && (!XNEG || xb >= 0) && xb < a.nx) {
-      const float* p = base + (static_cast<long>(z) * a.ny + y) * a.nx + xb;
-      if constexpr (VX % 4 == 0) {
-#pragma unroll
-        for (int v = 0; v < VX; v += 4) {
-          typedef float vec4 __attribute__((ext_vector_type(4)));
-          const vec4 q = NT ? __builtin_nontemporal_load(reinterpret_cast<const vec4*>(p + v))
-                            : *reinterpret_cast<const vec4*>(p + v);
-          out[v] = q.x;
-          out[v + 1] = q.y;
-          out[v + 2] = q.z;
-          out[v + 3] = q.w;
-        }
-      } else {
-#pragma unroll
-        for (int v = 0; v < VX; v += 2) {
-          typedef float vec2 __attribute__((ext_vector_type(2)));
-          const vec2 q = NT ? __builtin_nontemporal_load(reinterpret_cast<const vec2*>(p + v))
-                            : *reinterpret_cast<const vec2*>(p + v);
-          out[v] = q.x;
-          out[v + 1] = q.y;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int v = 0; v < VX; ++v) out[v] = 0.0f;
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < VX; ++v) out[v] = 0.0f;
-    if (!inside) return;
-    const long row = (static_cast<long>(z) * a.ny + y) * a.nx;
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      if ((!XNEG || xb + v >= 0) && xb + v < a.nx) out[v] = base[row + xb + v];
-    }
-  }
-}
-
-// NT: non-temporal stores, for the dual iterates. A pass writes them (400 MB at 256^3) long
-// before the next pass reads them, so kept in the caches they only displace the halo rows and
-// columns that neighbouring tiles of the same pass read back (measured: 169 -> 165 us per pass
-// at 256^3, 657 -> 620 us at 384^3 together with 64-plane z chunks).
-template <int VX, bool VEC, bool NT = false>
-__device__ __forceinline__ void store_row(float* base, const TvArgs& a, int z, int y, int xb,
-                                          const float (&in)[VX]) {
-  if (z >= a.nz || y >= a.ny) return;
-  float* p = base + (static_cast<long>(z) * a.ny + y) * a.nx + xb;
-  if constexpr (VEC) {
-    static_assert(VX % 2 == 0, "whole float2s");
-    typedef float vec4 __attribute__((ext_vector_type(4)));
-    typedef float vec2 __attribute__((ext_vector_type(2)));
-    if (xb < a.nx) {
-      if constexpr (VX % 4 == 0) {
-#pragma unroll
-        for (int v = 0; v < VX; v += 4) {
-          const vec4 q = {in[v], in[v + 1], in[v + 2], in[v + 3]};
-          if constexpr (NT) {
-            __builtin_nontemporal_store(q, reinterpret_cast<vec4*>(p + v));
-          } else {
-            *reinterpret_cast<vec4*>(p + v) = q;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int v = 0; v < VX; v += 2) {
-          const vec2 q = {in[v], in[v + 1]};
-          if constexpr (NT) {
-            __builtin_nontemporal_store(q, reinterpret_cast<vec2*>(p + v));
-          } else {
-            *reinterpret_cast<vec2*>(p + v) = q;
-          }
-        }
-      }
-    }
-  } else {
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      if (xb + v < a.nx) p[v] = in[v];
-    }
-  }
-}
-
-// Primal point z = max(b - lambda L(r), 0) of plane zp for the strip's rows y0..y0+TY (the
-// last one is the halo row below the strip). R holds r at plane zp, ry_top the y component of
-// r on row y0 - 1, rz_below the z component on plane zp - 1. The additions run in the order of
-// the negative divergence L(r)(i) = sum_a r_a(i) - r_a(i - e_a), axes z, y, x.
-template <int VX, int TY>
-__device__ __forceinline__ void primal_plane(const TvArgs& a, int zp, int y0, int xb,
-                                             const float (&R)[3][TY + 1][VX],
-                                             const float (&ry_top)[VX],
-                                             const float (&rz_below)[TY + 1][VX],
-                                             const float (&B)[TY + 1][VX],
-                                             float (&Z)[TY + 1][VX]) {
-#pragma unroll
-  for (int j = 0; j <= TY; ++j) {
-    const int y = y0 + j;
-    const float left = __shfl_up(R[2][j][VX - 1], 1);
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      const int x = xb + v;
-      float s = 0.0f;
-      if (zp < a.nz - 1) s += R[0][j][v];
-      if (zp > 0) s -= rz_below[j][v];
-      if (y < a.ny - 1) s += R[1][j][v];
-      if (y > 0) s -= (j == 0 ? ry_top[v] : R[1][j - 1][v]);
-      if (x < a.nx - 1) s += R[2][j][v];
-      if (x > 0) s -= (v == 0 ? left : R[2][j][v - 1]);
-      Z[j][v] = (y < a.ny && x < a.nx && zp < a.nz) ? tv_primal(B[j][v], a.lambda, s) : 0.0f;
-    }
-  }
-}
-
-// r = p_k + m (p_k - p_{k-1}) on one row (or p_k on the first step of a prox).
-template <int VX>
-__device__ __forceinline__ void extrapolate(const TvArgs& a, const float (&pk)[VX],
-                                            const float (&pm)[VX], float (&r)[VX]) {
-#pragma unroll
-  for (int v = 0; v < VX; ++v) r[v] = a.first ? pk[v] : pk[v] + a.momentum * (pk[v] - pm[v]);
-}
-
-// r of plane z on the strip rows and the halo row below (R), its y component on the row above
-// (ry_top), and b on the strip rows and the halo row. P keeps p_k of the strip rows for the
-// dual step of this plane.
-template <int VX, int TY, bool VEC>
-__device__ __forceinline__ void load_plane(const TvArgs& a, int z, int y0, int xb,
-                                           float (&R)[3][TY + 1][VX], float (&ry_top)[VX],
-                                           float (&B)[TY + 1][VX], float (&P)[3][TY][VX]) {
-#pragma unroll
-  for (int j = 0; j <= TY; ++j) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      float pk[VX], pm[VX];
-      load_row<VX, VEC>(a.p_in + c * a.vol, a, z, y0 + j, xb, pk);
-      if (!a.first) {
-        load_row<VX, VEC>(a.p_prev + c * a.vol, a, z, y0 + j, xb, pm);
-      } else {
-#pragma unroll
-        for (int v = 0; v < VX; ++v) pm[v] = 0.0f;
-      }
-      extrapolate<VX>(a, pk, pm, R[c][j]);
-      if (j < TY) {
-#pragma unroll
-        for (int v = 0; v < VX; ++v) P[c][j][v] = pk[v];
-      }
-    }
-    load_row<VX, VEC>(a.b, a, z, y0 + j, xb, B[j]);
-  }
-  float pk[VX], pm[VX];
-  load_row<VX, VEC>(a.p_in + a.vol, a, z, y0 - 1, xb, pk);
-  if (!a.first) {
-    load_row<VX, VEC>(a.p_prev + a.vol, a, z, y0 - 1, xb, pm);
-  } else {
-#pragma unroll
-    for (int v = 0; v < VX; ++v) pm[v] = 0.0f;
-  }
-  extrapolate<VX>(a, pk, pm, ry_top);
-}
-
-template <int VX, int TY, bool VEC, bool BATCH>
-__global__ void __launch_bounds__(64) k_fgp_step(TvArgs a, int chunks) {
-  if constexpr (BATCH) {
-    a.b = shifted(a.b, batch_volume() * a.vol);
-    a.p_in = shifted(a.p_in, 3 * batch_volume() * a.vol);
-    a.p_prev = shifted(a.p_prev, 3 * batch_volume() * a.vol);
-    a.p_out = shifted(a.p_out, 3 * batch_volume() * a.vol);
-  }
-  const int t = xcd_tile();
-  const int y0 = (t / chunks) * TY;
-  const int z0 = (t % chunks) * a.zlen;
-  const int z1 = min(z0 + a.zlen, a.nz);
-  const int xb = static_cast<int>(threadIdx.x) * VX;
-
-  float r[3][TY + 1][VX];  // r at plane z, rows y0..y0+TY
-  float pc[3][TY][VX];     // p_k at plane z, strip rows
-  float zc[TY + 1][VX];    // primal at plane z
-  {
-    // Warm-up: the primal on plane z0 needs the z component of r on plane z0 - 1.
-    float rz_below[TY + 1][VX];
-#pragma unroll
-    for (int j = 0; j <= TY; ++j) {
-      float pk[VX], pm[VX];
-      load_row<VX, VEC>(a.p_in, a, z0 - 1, y0 + j, xb, pk);
-      if (!a.first) {
-        load_row<VX, VEC>(a.p_prev, a, z0 - 1, y0 + j, xb, pm);
-      } else {
-#pragma unroll
-        for (int v = 0; v < VX; ++v) pm[v] = 0.0f;
-      }
-      extrapolate<VX>(a, pk, pm, rz_below[j]);
-    }
-    float ry_top[VX], bb[TY + 1][VX];
-    load_plane<VX, TY, VEC>(a, z0, y0, xb, r, ry_top, bb, pc);
-    primal_plane<VX, TY>(a, z0, y0, xb, r, ry_top, rz_below, bb, zc);
-  }
-  for (int z = z0; z < z1; ++z) {
-    float rn[3][TY + 1][VX], ryn[VX], bn[TY + 1][VX], pn[3][TY][VX], zn[TY + 1][VX];
-    load_plane<VX, TY, VEC>(a, z + 1, y0, xb, rn, ryn, bn, pn);
-    primal_plane<VX, TY>(a, z + 1, y0, xb, rn, ryn, r[0], bn, zn);
-#pragma unroll
-    for (int j = 0; j < TY; ++j) {
-      const int y = y0 + j;
-      const float right = __shfl_down(zc[j][0], 1);
-      float po[3][VX];
-#pragma unroll
-      for (int v = 0; v < VX; ++v) {
-        const int x = xb + v;
-        const float c = zc[j][v];
-        float g[3];
-        g[0] = z < a.nz - 1 ? c - zn[j][v] : 0.0f;
-        g[1] = y < a.ny - 1 ? c - zc[j + 1][v] : 0.0f;
-        g[2] = x < a.nx - 1 ? c - (v == VX - 1 ? right : zc[j][v + 1]) : 0.0f;
-        float p3[3] = {pc[0][j][v], pc[1][j][v], pc[2][j][v]};
-        float r3[3] = {r[0][j][v], r[1][j][v], r[2][j][v]};
-        tv_dual_step(g, a.step, 0.0f, p3, r3);
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) po[cc][v] = p3[cc];
-      }
-#pragma unroll
-      for (int cc = 0; cc < 3; ++cc) store_row<VX, VEC, true>(a.p_out + cc * a.vol, a, z, y, xb, po[cc]);
-    }
-#pragma unroll
-    for (int j = 0; j <= TY; ++j) {
-#pragma unroll
-      for (int v = 0; v < VX; ++v) {
-        zc[j][v] = zn[j][v];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) r[c][j][v] = rn[c][j][v];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < TY; ++j) {
-#pragma unroll
-      for (int v = 0; v < VX; ++v) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) pc[c][j][v] = pn[c][j][v];
-      }
-    }
-  }
-}
-
-// ---- two FGP steps per pass ----
+// A block of NW waves holds a tile of 64 columns (one per lane) by NW quads of rows (one per
+// wave) and marches z. Stage s = 0 .. T-1 runs step k+s+1 on the planes as they come: with plane f
+// of the inputs loaded, stage s forms z_{k+s} on plane f - s from r_{k+s} there, then p_{k+s+1} and
+// r_{k+s+1} on plane f - s - 1, which stage s + 1 takes. Each stage keeps one plane of r, p and z of
+// the tile in registers (7 floats a point); the last planes of b wait in LDS. x neighbours come
+// by DPP from the next lane, y neighbours from the thread's own registers except at the edges of
+// a wave's quad (a row of r_y and one of z per wave and stage through LDS), z neighbours from the
+// registers of the plane before. Every step makes one column, row and plane on either side of the
+// tile invalid, so tiles overlap by kHalo columns and rows on each side and a chunk of planes
+// starts T planes early. FINAL adds a stage that forms max(b - lambda L(p_{k+T}), 0).
 //
-// A block of NW waves owns NW - 4 output rows; wave w holds row y0 - 2 + w across its 64 lanes
-// (VX floats each) and the block marches z through a chunk of planes. Per plane t the waves
-// load b, p_k, p_{k-1} of plane t + 2, form r_k and z_k there, the dual p_{k+1} of plane t + 1
-// and its r_{k+1}, z_{k+1} of plane t + 1, and p_{k+2} of plane t. y neighbours come through
-// LDS (one row buffer per quantity, read back before the owner overwrites it), x neighbours by
-// shuffles, z neighbours from the registers of the previous plane. The two halo rows on each
-// side make step one available where step two needs it; their results are not stored. Every
-// value is formed with the float operations of k_fgp_step, so a pass equals two single steps
-// bit for bit, while HBM sees 7 volumes read and 6 written per two steps instead of 20.
-// Planes per block: at most 64 and at least 4, chosen per volume by pair_chunk; each chunk
-// starts two planes early, so longer chunks read fewer warm-up planes (384^3 pass with x tiles
-// of 2 columns per lane 675 -> 637 us from 32 to 64 planes).
-constexpr int kPairChunk = 64;
-constexpr int kPairChunkMin = 4;
+// Eight waves of up to 256 registers make one block per CU. Twelve waves (48 rows a tile) leave 168
+// registers, which T = 3 just fits and the other passes spill: 209 against 220 us for a 256^3 pass
+// of three steps but 330 against 232 us for one with the output, and no gain at 384^3 (665 against
+// 643 us) or 128^3 (56 against 44 us), where fewer, larger tiles fill the CUs less evenly.
+constexpr int kRows = 4;   // rows of a quad
+constexpr int kWaves = 8;  // quads of a tile
+constexpr int kHalo = 4;   // columns and rows of a tile, on each side, that are not its own
+constexpr int kMaxSteps = 4;
 
-struct PairArgs {
+struct StepArgs {
   const float* b;
   const float* p_k;    // p_k (r_k is formed from it)
-  const float* p_km1;  // p_{k-1} (unused on the first step of a prox)
-  float* p_k1;         // out: p_{k+1}
-  float* p_k2;         // out: p_{k+2}
+  const float* p_km1;  // p_{k-1} (not read on the first step of a prox)
+  float* p_prev;       // out: p_{k+T-1}, or null
+  float* p_last;       // out: p_{k+T}, or null
+  float* x;            // out with FINAL: the prox output
   long vol;
   int nz, ny, nx;
   float lambda;
   float step;
-  float m1;  // momentum of r_k = p_k + m1 (p_k - p_{k-1})
+  float m[kMaxSteps];  // m[s]: momentum of r_{k+s}; 0 on the first step of a prox
   int first;
-  float m2;  // momentum of r_{k+1} = p_{k+1} + m2 (p_{k+1} - p_k)
-  int zlen;  // planes per chunk
-  int xt;       // output columns per x tile (nx when one tile spans the row)
-  int tiles_x;  // x tiles per row
+  int zlen;              // planes per chunk
+  int tiles_x, tiles_y;
+  int tile_x, tile_y;    // columns and rows a tile writes
+  int halo_x, halo_y;    // kHalo, or 0 where one tile holds the volume's side
+  int to_index;          // the output as refractive index
+  float nm2, inv_k02;
 };
 
-// Whether column xb + v of a lane can lie on the volume's x faces. Rows that start at column 0
-// (not XNEG) with whole-vector access (VEC: nx a multiple of VX, xb a multiple of VX) put the
-// faces only in a lane's first (x = 0) and last (x = nx - 1) element, so the middle elements of
-// an active lane (xb < nx) never need the x tests.
-template <int VX, bool XNEG, bool VEC>
-__device__ __forceinline__ constexpr bool x_left_face(int v) {
-  return XNEG || !VEC || v == 0;
-}
-template <int VX, bool XNEG, bool VEC>
-__device__ __forceinline__ constexpr bool x_right_face(int v) {
-  return XNEG || !VEC || v == VX - 1;
-}
+// The march, unrolled over T + 1 planes: the r and p a stage hands on take the registers of the
+// plane it has done with, so the register sets rotate through the T stages and the loads, and after
+// T + 1 planes are back in place (a rolled loop moves 7 floats a point and stage back by v_mov). The
+// unrolled planes are numbered U = 0 .. T.
+//
+// QUADS: ny is a multiple of 4. Otherwise the rows of the last quad are stored column by column
+// like the others (h floats a column for h rows), which takes accesses of 4 bytes. FIRST: the first
+// pass of a prox, which needs no p_{k-1}.
+template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
+struct StepMarch {
+  static constexpr int NW = kWaves;
+  static constexpr int HL = T + (FINAL ? 1 : 0);  // planes in front of a chunk
+  static constexpr int S = T + (FINAL ? 1 : 0);   // stages that exchange rows
+  static constexpr int TS = T > 0 ? T : 1;
+  static constexpr int kUnroll = T + 1;
+  // Row exchange buffers: planes that follow one another use different ones, as a wave may be one
+  // barrier ahead of its neighbours, never a plane.
+  static constexpr int kBufs = kUnroll % 2 == 0 ? 2 : 3;
+  static constexpr int buf(int u) { return u == kUnroll - 1 && kBufs == 3 ? 2 : u % 2; }
 
-// z = max(b - lambda L(r), 0) on one row of plane zp (the expression order of primal_plane).
-// zp and y are the same for every lane of the wave: on planes and rows off the volume's z and y
-// faces every z and y term is taken, so that branch runs the same float operations without the
-// per-element selects (the kernel's time is set by its VALU issue rate, not only by its bytes).
-template <int VX, bool XNEG, bool VEC>
-__device__ __forceinline__ void pair_primal(const PairArgs& a, int zp, int y, int xb,
-                                            const float (&R)[3][VX], const float (&rz_below)[VX],
-                                            const float (&ry_up)[VX], const float (&B)[VX],
-                                            float (&Z)[VX]) {
-  const float left = __shfl_up(R[2][VX - 1], 1);
-  if (zp > 0 && zp < a.nz - 1 && y > 0 && y < a.ny - 1) {
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      const int x = xb + v;
-      float s = 0.0f;
-      s += R[0][v];
-      s -= rz_below[v];
-      s += R[1][v];
-      s -= ry_up[v];
-      if (!x_right_face<VX, XNEG, VEC>(v) || x < a.nx - 1) s += R[2][v];
-      if (!x_left_face<VX, XNEG, VEC>(v) || x > 0) s -= (v == 0 ? left : R[2][v - 1]);
-      // Without XNEG and with VEC every element of an active lane is inside the row; inactive
-      // lanes (xb >= nx) are never stored and feed no active lane's result.
-      Z[v] = (XNEG || !VEC) ? (((!XNEG || x >= 0) && x < a.nx) ? tv_primal(B[v], a.lambda, s) : 0.0f)
-                            : tv_primal(B[v], a.lambda, s);
-    }
-    return;
-  }
-#pragma unroll
-  for (int v = 0; v < VX; ++v) {
-    const int x = xb + v;
-    float s = 0.0f;
-    if (zp < a.nz - 1) s += R[0][v];
-    if (zp > 0) s -= rz_below[v];
-    if (y < a.ny - 1) s += R[1][v];
-    if (y > 0) s -= ry_up[v];
-    if (x < a.nx - 1) s += R[2][v];
-    if (x > 0) s -= (v == 0 ? left : R[2][v - 1]);
-    Z[v] = (y >= 0 && y < a.ny && (!XNEG || x >= 0) && x < a.nx && zp >= 0 && zp < a.nz)
-               ? tv_primal(B[v], a.lambda, s)
-               : 0.0f;
-  }
-}
+  struct Lds {
+    float ry[kBufs][S][NW + 1][64];  // r_y of the last row of wave w at w + 1; zero at 0
+    float z[kBufs][TS][NW + 1][64];  // z of the first row of wave w at w; zero at NW
+    float4 b[kUnroll][NW][64];       // the last planes of b; read back by the thread that wrote
+  };
 
-// p' = P(r + step g) on one row of plane zp, g from z of this plane (zc), the plane above (zn)
-// and the row below (zdn): the dual step of k_fgp_step. Off the last plane and the last row
-// (wave-uniform) the z and y differences are taken without selects.
-template <int VX, bool XNEG, bool VEC>
-__device__ __forceinline__ void pair_dual(const PairArgs& a, int zp, int y, int xb,
-                                          const float (&zc)[VX], const float (&zn)[VX],
-                                          const float (&zdn)[VX], const float (&R)[3][VX],
-                                          float (&P)[3][VX]) {
-  const float right = __shfl_down(zc[0], 1);
-  const bool inner = zp < a.nz - 1 && y < a.ny - 1;
-#pragma unroll
-  for (int v = 0; v < VX; ++v) {
-    const int x = xb + v;
-    const float c = zc[v];
-    float g[3];
-    if (inner) {
-      g[0] = c - zn[v];
-      g[1] = c - zdn[v];
-    } else {
-      g[0] = zp < a.nz - 1 ? c - zn[v] : 0.0f;
-      g[1] = y < a.ny - 1 ? c - zdn[v] : 0.0f;
-    }
-    g[2] = (!x_right_face<VX, XNEG, VEC>(v) || x < a.nx - 1)
-               ? c - (v == VX - 1 ? right : zc[v + 1])
-               : 0.0f;
-    float p3[3] = {0.0f, 0.0f, 0.0f};
-    float r3[3] = {R[0][v], R[1][v], R[2][v]};
-    tv_dual_step(g, a.step, 0.0f, p3, r3);
-#pragma unroll
-    for (int c3 = 0; c3 < 3; ++c3) P[c3][v] = p3[c3];
-  }
-}
+  const StepArgs& a;
+  Lds& l;
+  int w, lane, z0, z1, yw, last_plane;
+  bool gx_on;
+  long plane, wave_row;
+  int rows;      // of the wave's quad inside the volume (0: none)
+  bool wave_on;  // the wave's rows are the tile's to write
+  // Byte offsets of the thread's column in a quad of the dual and in a row of b, or kOutside; and
+  // the same where the column is the tile's to write. (Rows outside the volume end past a window.)
+  unsigned xq, xr, xq_out, xr_out;
+  float R[TS][kRows][3], P[TS][kRows][3], Z[TS][kRows], PZ[kRows];
+  // p_k, p_{k-1} (zero on the first step of a prox, whose m[0] is zero: r = p) and b of the next
+  // plane, loaded a plane ahead.
+  float pk[3][kRows], pm[3][kRows], bb[kRows];
 
-// Rows in LDS (row r of a buffer at r * nx), with the access rules of load_row.
-template <int VX, bool VEC>
-__device__ __forceinline__ void lds_put(float* buf, int row, int nx, int xb, const float (&v)[VX]) {
-  if constexpr (VEC && VX % 4 == 0) {
-    if (xb < nx) {
+  __device__ __forceinline__ void load_dual(float (&v)[3][kRows], const float* p, long at,
+                                            bool on) {
 #pragma unroll
-      for (int i = 0; i < VX; i += 4) {
-        *reinterpret_cast<float4*>(buf + row * nx + xb + i) = float4{v[i], v[i + 1], v[i + 2], v[i + 3]};
+    for (int c = 0; c < 3; ++c) {
+      const Window q(p + c * a.vol + at, 4 * rows * a.nx, on);
+      if constexpr (QUADS) {
+        q.load4(v[c], xq);
+      } else {
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) v[c][j] = q.load(j < rows ? xq + 4u * j : kOutside);
       }
     }
-  } else if constexpr (VEC && VX % 2 == 0) {
-    if (xb < nx) {
-#pragma unroll
-      for (int i = 0; i < VX; i += 2) {
-        *reinterpret_cast<float2*>(buf + row * nx + xb + i) = float2{v[i], v[i + 1]};
-      }
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < VX; ++i) {
-      if (xb + i < nx) buf[row * nx + xb + i] = v[i];
-    }
   }
-}
+  __device__ __forceinline__ void load(int f) {
+    const long at = static_cast<long>(min(f, a.nz - 1)) * plane + wave_row;
+    load_dual(pk, a.p_k, at, true);
+    if constexpr (!FIRST) load_dual(pm, a.p_km1, at, a.first == 0);
+    const Window b(a.b + at, 4 * rows * a.nx, true);
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) bb[j] = b.load(xr + 4u * static_cast<unsigned>(j * a.nx));
+  }
 
-template <int VX, bool VEC>
-__device__ __forceinline__ void lds_get(const float* buf, int row, int nx, int xb, float (&v)[VX]) {
-  if constexpr (VEC && VX % 4 == 0) {
-    if (xb < nx) {
+  // Component-wise rows of p on plane z, where that is the tile's to write.
+  __device__ __forceinline__ void store(float* p, int z, const float (&v)[kRows][3]) {
+    const bool on = p != nullptr && wave_on && z >= z0 && z < z1;
+    const long at = static_cast<long>(max(z, 0)) * plane + wave_row;
 #pragma unroll
-      for (int i = 0; i < VX; i += 4) {
-        const float4 q = *reinterpret_cast<const float4*>(buf + row * nx + xb + i);
-        v[i] = q.x;
-        v[i + 1] = q.y;
-        v[i + 2] = q.z;
-        v[i + 3] = q.w;
+    for (int c = 0; c < 3; ++c) {
+      const Window q(p + c * a.vol + at, 4 * rows * a.nx, on);
+      if constexpr (QUADS) {
+        const float r[kRows] = {v[0][c], v[1][c], v[2][c], v[3][c]};
+        q.stream4(r, xq_out);
+      } else {
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) q.stream(v[j][c], j < rows ? xq_out + 4u * j : kOutside);
       }
-    } else {
-#pragma unroll
-      for (int i = 0; i < VX; ++i) v[i] = 0.0f;
     }
-  } else if constexpr (VEC && VX % 2 == 0) {
-    if (xb < nx) {
-#pragma unroll
-      for (int i = 0; i < VX; i += 2) {
-        const float2 q = *reinterpret_cast<const float2*>(buf + row * nx + xb + i);
-        v[i] = q.x;
-        v[i + 1] = q.y;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < VX; ++i) v[i] = 0.0f;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < VX; ++i) v[i] = (xb + i < nx) ? buf[row * nx + xb + i] : 0.0f;
   }
-}
 
-// VEC: see load_row. XT: rows are cut into x tiles (more than one per row).
-template <int VX, int NW, bool VEC, bool XT, bool BATCH>
-__global__ void __launch_bounds__(NW * 64) k_fgp_pair(PairArgs a, int chunks) {
-  if constexpr (BATCH) {
-    a.b = shifted(a.b, batch_volume() * a.vol);
-    a.p_k = shifted(a.p_k, 3 * batch_volume() * a.vol);
-    a.p_km1 = shifted(a.p_km1, 3 * batch_volume() * a.vol);
-    a.p_k1 = shifted(a.p_k1, 3 * batch_volume() * a.vol);
-    a.p_k2 = shifted(a.p_k2, 3 * batch_volume() * a.vol);
+  __device__ __forceinline__ void planes_of_b(int u, float (&v)[kRows]) {
+    const float4 q = l.b[u][w][lane];
+    v[0] = q.x;
+    v[1] = q.y;
+    v[2] = q.z;
+    v[3] = q.w;
   }
-  constexpr int TOP = 2;  // halo rows above the output rows (and two below)
-  constexpr int T = NW - 4;
-  // LDS row width: the row when a wave holds it whole, else the columns one wave holds.
-  const int LW = XT ? 64 * VX : a.nx;
-  extern __shared__ float4 lds4[];
-  float* lds = reinterpret_cast<float*>(lds4);
-  float* ry = lds;              // y component of r_k of each row
-  float* rqy = ry + NW * LW;    // y component of r_{k+1}
-  float* zk = rqy + NW * LW;    // z_k
-  float* zq = zk + NW * LW;     // z_{k+1}
-  TvArgs bd{};
-  bd.nz = a.nz;
-  bd.ny = a.ny;
-  bd.nx = a.nx;
+
+  // Stage s on plane f - s: takes r and p of that plane, leaves p and r of the step on the plane
+  // below it.
+  template <int U, int s>
+  __device__ __forceinline__ void stage(int f, float (&rn)[kRows][3], float (&pn)[kRows][3]) {
+    constexpr int kBuf = buf(U);
+    constexpr int kLast = buf((U + kUnroll - 1) % kUnroll);  // of the plane before
+    float bs[kRows];
+    planes_of_b((U + kUnroll - s) % kUnroll, bs);
+    l.ry[kBuf][s][w + 1][lane] = rn[kRows - 1][1];
+    __syncthreads();
+    const float ry_edge = l.ry[kBuf][s][w][lane];
+    const float z_edge = l.z[kLast][s][w + 1][lane];
+    const int zo = f - s - 1;  // plane of p_{k+s+1}
+    const bool gz_on = zo >= 0 && zo < a.nz - 1;
+    float z_first = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const float ry_up = j > 0 ? R[s][j > 0 ? j - 1 : 0][1] : ry_edge;
+      const float zn = primal_value<EXACT>(bs[j], a.lambda, rn[j][0], R[s][j][0], rn[j][1],
+                                           ry_up, rn[j][2], lane_below(rn[j][2]));
+      const float zc = Z[s][j];
+      const float z_dn = j < kRows - 1 ? Z[s][j < kRows - 1 ? j + 1 : j] : z_edge;
+      const float qz = multiply_add<EXACT>(a.step, zc - zn, R[s][j][0]);
+      const float qy = multiply_add<EXACT>(a.step, zc - z_dn, R[s][j][1]);
+      const float qx = multiply_add<EXACT>(a.step, zc - lane_above(zc), R[s][j][2]);
+      // A point outside the volume differs from one inside only in that no step updates its
+      // component along the axis it is outside of, so it never reaches a point inside.
+      const float q[3] = {gz_on ? qz : 0.0f,
+                          yw + j >= 0 && yw + j < a.ny - 1 ? qy : 0.0f, gx_on ? qx : 0.0f};
+      const float scale = ball_scale<EXACT>(multiply_add<EXACT>(
+          q[2], q[2], multiply_add<EXACT>(q[1], q[1], q[0] * q[0])));
+      if (j == 0) z_first = zn;
+      Z[s][j] = zn;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float next = q[c] * scale;
+        const float old = P[s][j][c];
+        R[s][j][c] = rn[j][c];
+        P[s][j][c] = pn[j][c];
+        pn[j][c] = next;
+        if constexpr (s + 1 < T) rn[j][c] = multiply_add<EXACT>(a.m[s + 1], next - old, next);
+      }
+    }
+    l.z[kBuf][s][w][lane] = z_first;
+    if constexpr (s == T - 2) store(a.p_prev, zo, pn);
+    if constexpr (s == T - 1) store(a.p_last, zo, pn);
+    if constexpr (s + 1 < T) stage<U, s + 1>(f, rn, pn);
+  }
+
+  // The prox output on plane f - T from p_{k+T} there.
+  template <int U>
+  __device__ __forceinline__ void output(int f, const float (&pn)[kRows][3]) {
+    constexpr int kBuf = buf(U);
+    float bs[kRows];
+    planes_of_b((U + kUnroll - T) % kUnroll, bs);
+    l.ry[kBuf][S - 1][w + 1][lane] = pn[kRows - 1][1];
+    __syncthreads();
+    const float py_edge = l.ry[kBuf][S - 1][w][lane];
+    const int zp = f - T;
+    const Window x(a.x + static_cast<long>(max(zp, 0)) * plane + wave_row, 4 * rows * a.nx,
+                   wave_on && zp >= z0 && zp < z1);
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const float py_up = j > 0 ? pn[j > 0 ? j - 1 : 0][1] : py_edge;
+      float v = primal_value<EXACT>(bs[j], a.lambda, pn[j][0], PZ[j], pn[j][1], py_up, pn[j][2],
+                                    lane_below(pn[j][2]));
+      PZ[j] = pn[j][0];
+      if (a.to_index) v = index_from_real(v, a.nm2, a.inv_k02);
+      x.store(v, xr_out + 4u * static_cast<unsigned>(j * a.nx));
+    }
+  }
+
+  template <int U>
+  __device__ __forceinline__ void planes(int f) {
+    float rn[kRows][3], pn[kRows][3];
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        pn[j][c] = pk[c][j];
+        rn[j][c] = FIRST ? pk[c][j]
+                         : multiply_add<EXACT>(a.m[0], pk[c][j] - pm[c][j], pk[c][j]);
+      }
+    }
+    l.b[U][w][lane] = float4{bb[0], bb[1], bb[2], bb[3]};
+    load(f + 1);
+    if constexpr (T > 0) stage<U, 0>(f, rn, pn);
+    if constexpr (FINAL) output<U>(f, pn);
+    if constexpr (U + 1 < kUnroll) {
+      // The longer passes with the output end within a turn (128^3: 53 against 61 us); in the others
+      // the test costs more, in scheduling across planes, than the planes it saves (256^3: 236
+      // against 218 us).
+      if (FINAL && f >= last_plane) return;
+      planes<U + 1>(f + 1);
+    }
+  }
+};
+
+template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
+__global__ void __launch_bounds__(kWaves * 64)
+    __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) k_fgp_steps(StepArgs a) {
+  using M = StepMarch<T, FIRST, FINAL, QUADS, EXACT>;
+  __shared__ typename M::Lds lds;
+  // Volume blockIdx.y of a batch of volumes that lie one after another.
+  const long batch = static_cast<long>(blockIdx.y);
+  a.b += batch * a.vol;
+  a.p_k += 3 * batch * a.vol;
+  if (a.p_km1) a.p_km1 += 3 * batch * a.vol;
+  if (a.p_prev) a.p_prev += 3 * batch * a.vol;
+  if (a.p_last) a.p_last += 3 * batch * a.vol;
+  if (a.x) a.x += batch * a.vol;
+  M m{a, lds};
   // The wave index is uniform across the wave: as a scalar it keeps the row arithmetic, the
-  // row addresses and the y tests off the vector ALU.
-  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  // Tiles of one z chunk are consecutive (x fastest, then y), so the neighbours that share halo
-  // rows and columns run on the same XCD. Rows wider than a wave are cut into x tiles of xt
-  // output columns; each tile's wave also holds one lane of columns on either side, which two
-  // steps of the 7-point stencil need, and stores only its own columns.
-  const int tile = xcd_tile();
-  const int tx = XT ? tile % a.tiles_x : 0;
-  const int rest = XT ? tile / a.tiles_x : tile;
-  const int tiles_y = static_cast<int>(gridDim.x) / (chunks * (XT ? a.tiles_x : 1));
-  const int y0 = (rest % tiles_y) * T;
-  const int z0 = (rest / tiles_y) * a.zlen;
-  const int z1 = min(z0 + a.zlen, a.nz);
-  const int y = y0 - TOP + w;
-  const int xo = tx * a.xt;            // first output column of the tile
-  const int x0 = XT ? xo - VX : 0;     // column of lane 0
-  const int xl = lane * VX;            // column within the LDS row
-  const int xb = x0 + xl;
-  const bool out_col = !XT || (xb >= xo && xb < min(xo + a.xt, a.nx));
-  const int wu = w > 0 ? w - 1 : 0;       // the first and last waves read their own row: their
-  const int wd = w < NW - 1 ? w + 1 : w;  // results only feed other halo values, never a store
-  const bool out_row = w >= TOP && w < TOP + T && y < a.ny;
-  const int pre = 2;  // planes of warm-up before z0
-  // p_k, p_{k-1} and b of this row on plane f, as loaded.
-  auto load_raw_as = [&]<bool NT>(int f, float (&Pk)[3][VX], float (&Pm)[3][VX], float (&B)[VX]) {
+  // windows and the y tests off the vector ALU.
+  m.w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  m.lane = static_cast<int>(threadIdx.x) & 63;
+  // Tiles of one chunk are consecutive (x fastest), so that tiles that share halos run on one
+  // XCD and share its L2.
+  const int tile = static_cast<int>(xcd_block());
+  const int tx = tile % a.tiles_x;
+  const int rest = tile / a.tiles_x;
+  const int ty = rest % a.tiles_y;
+  m.z0 = (rest / a.tiles_y) * a.zlen;
+  m.z1 = min(m.z0 + a.zlen, a.nz);
+  const int x = tx * a.tile_x - a.halo_x + m.lane;
+  m.yw = ty * a.tile_y - a.halo_y + m.w * kRows;
+  m.rows = m.yw < 0 ? 0 : max(0, min(kRows, a.ny - m.yw));
+  m.wave_on = m.yw >= ty * a.tile_y && m.yw < (ty + 1) * a.tile_y;
+  m.gx_on = x >= 0 && x < a.nx - 1;
+  m.plane = static_cast<long>(a.ny) * a.nx;
+  m.wave_row = m.rows > 0 ? static_cast<long>(m.yw) * a.nx : 0;
+  const bool in_x = x >= 0 && x < a.nx;
+  const bool out_x = in_x && x >= tx * a.tile_x && x < (tx + 1) * a.tile_x;
+  m.xq = in_x ? 4u * static_cast<unsigned>(x * m.rows) : kOutside;
+  m.xr = in_x ? 4u * static_cast<unsigned>(x) : kOutside;
+  m.xq_out = out_x ? m.xq : kOutside;
+  m.xr_out = out_x ? m.xr : kOutside;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      load_row<VX, VEC, XT, NT>(a.p_k + c * a.vol, bd, f, y, xb, Pk[c]);
-      if (!a.first) {
-        load_row<VX, VEC, XT, NT>(a.p_km1 + c * a.vol, bd, f, y, xb, Pm[c]);
-      } else {
+  for (int j = 0; j < kRows; ++j) {
+    m.PZ[j] = 0.0f;
 #pragma unroll
-        for (int v = 0; v < VX; ++v) Pm[c][v] = 0.0f;
-      }
+    for (int s = 0; s < T; ++s) {
+      m.Z[s][j] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) m.R[s][j][c] = m.P[s][j][c] = 0.0f;
     }
-    load_row<VX, VEC, XT, NT>(a.b, bd, f, y, xb, B);
-  };
-  // Rows that no other tile reads (waves 4 .. NW-5 of an untiled row: the halo rows of the
-  // tiles above and below are this tile's first and last two output rows) are loaded
-  // non-temporally, which keeps them from displacing the rows that neighbouring tiles read back
-  // (256^3 pass 153.6 -> 147.8 us). In x tiles every row's edge columns are a neighbouring
-  // tile's halo, and the same hint made the 384^3 pass slower (587 -> 608 us); so did loading
-  // every row non-temporally (256^3: 165 us).
-  const bool stream_row = !XT && w >= 4 && w <= NW - 5;
-  auto load_raw = [&](int f, float (&Pk)[3][VX], float (&Pm)[3][VX], float (&B)[VX]) {
-    if (stream_row) {
-      load_raw_as.template operator()<true>(f, Pk, Pm, B);
-    } else {
-      load_raw_as.template operator()<false>(f, Pk, Pm, B);
-    }
-  };
-  // r_k = p_k + m1 (p_k - p_{k-1}), or p_k on the first step.
-  auto extrapolate_k = [&](const float (&Pk)[3][VX], const float (&Pm)[3][VX], float (&R)[3][VX]) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-      for (int v = 0; v < VX; ++v) R[c][v] = a.first ? Pk[c][v] : Pk[c][v] + a.m1 * (Pk[c][v] - Pm[c][v]);
-    }
-  };
-  // r_k, p_k and b of this row on plane f.
-  auto load_step1 = [&](int f, float (&R)[3][VX], float (&Pk)[3][VX], float (&B)[VX]) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      float pm[VX];
-      load_row<VX, VEC, XT>(a.p_k + c * a.vol, bd, f, y, xb, Pk[c]);
-      if (!a.first) {
-        load_row<VX, VEC, XT>(a.p_km1 + c * a.vol, bd, f, y, xb, pm);
-      } else {
-#pragma unroll
-        for (int v = 0; v < VX; ++v) pm[v] = 0.0f;
-      }
-#pragma unroll
-      for (int v = 0; v < VX; ++v) R[c][v] = a.first ? Pk[c][v] : Pk[c][v] + a.m1 * (Pk[c][v] - pm[v]);
-    }
-    load_row<VX, VEC, XT>(a.b, bd, f, y, xb, B);
-  };
-
-  // Prologue: r_k on plane z0 - pre (z component) and z_k on plane z0 - pre + 1.
-  const int zs = z0 - pre + 1;
-  float rz_m2[VX];
-  {
-    float pk[VX], pm[VX];
-    load_row<VX, VEC, XT>(a.p_k, bd, zs - 1, y, xb, pk);
-    if (!a.first) {
-      load_row<VX, VEC, XT>(a.p_km1, bd, zs - 1, y, xb, pm);
-    } else {
-#pragma unroll
-      for (int v = 0; v < VX; ++v) pm[v] = 0.0f;
-    }
-#pragma unroll
-    for (int v = 0; v < VX; ++v) rz_m2[v] = a.first ? pk[v] : pk[v] + a.m1 * (pk[v] - pm[v]);
   }
-  float rk1[3][VX], pk1[3][VX], b1[VX], zk1[VX];
-  load_step1(zs, rk1, pk1, b1);
-  lds_put<VX, VEC>(ry, w, LW, xl, rk1[1]);
-  __syncthreads();
-  {
-    float up[VX];
-    lds_get<VX, VEC>(ry, wu, LW, xl, up);
-    pair_primal<VX, XT, VEC>(a, zs, y, xb, rk1, rz_m2, up, b1, zk1);
-  }
-  lds_put<VX, VEC>(zk, w, LW, xl, zk1);
-  float rq0[3][VX], zq0[VX], zdn_k[VX], zdn_q[VX];
-#pragma unroll
-  for (int v = 0; v < VX; ++v) {
-    zq0[v] = 0.0f;
-    zdn_q[v] = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) rq0[c][v] = 0.0f;
+  float* const words = reinterpret_cast<float*>(&lds);
+  for (int i = static_cast<int>(threadIdx.x); i < static_cast<int>(sizeof(lds) / 4);
+       i += kWaves * 64) {
+    words[i] = 0.0f;
   }
   __syncthreads();
-  lds_get<VX, VEC>(zk, wd, LW, xl, zdn_k);  // z_k of the row below on plane zs
-
-  // The loads of the next plane are issued once the first dual step is done, before the second
-  // barrier, so that their latency overlaps the second primal and the last dual step instead
-  // of stalling the block at the next barrier (issued after the third barrier the pass took 6%
-  // longer at 256 and 7% at 384; any earlier, the registers spill); r_k is formed from them at
-  // the top of the next iteration.
-  // What each wave's row feeds: the output rows (waves 2 .. NW-3) need p_{k+2}, which needs
-  // z_{k+1} one row further down (waves 2 .. NW-2), which needs r_{k+1} one row up (waves
-  // 1 .. NW-2), which needs z_k one row down (waves 1 .. NW-1); wave 0 only supplies r_k. A
-  // wave skips the quantities no output depends on (wave-uniform branches; the variant with
-  // element-wise row access keeps computing them, which holds it below the register limit).
-  const bool need_zk = !VEC || w >= 1;
-  const bool need_pk1 = !VEC || (w >= 1 && w <= NW - 2);
-  const bool need_zq = !VEC || (w >= 2 && w <= NW - 2);
-  const bool need_pk2 = !VEC || (w >= TOP && w < TOP + T);
-  float pk2[3][VX], pm2[3][VX], b2[VX];
-  load_raw(z0 - pre + 2, pk2, pm2, b2);
-  for (int t = z0 - pre; t < z1; ++t) {
-    const int f = t + 2;
-    float rk2[3][VX];
-    extrapolate_k(pk2, pm2, rk2);
-    lds_put<VX, VEC>(ry, w, LW, xl, rk2[1]);
-    __syncthreads();  // (1) r_k of plane f visible
-    float zk2[VX] = {};
-    if (need_zk) {
-      float up[VX];
-      lds_get<VX, VEC>(ry, wu, LW, xl, up);
-      pair_primal<VX, XT, VEC>(a, f, y, xb, rk2, rk1[0], up, b2, zk2);
-    }
-    // p_{k+1} and r_{k+1} on plane t + 1.
-    float rq1[3][VX] = {};
-    if (need_pk1) {
-      float pq1[3][VX];
-      pair_dual<VX, XT, VEC>(a, t + 1, y, xb, zk1, zk2, zdn_k, rk1, pq1);
-      if (a.p_k1 && out_row && out_col && t + 1 >= z0 && t + 1 < z1) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) store_row<VX, VEC, true>(a.p_k1 + c * a.vol, bd, t + 1, y, xb, pq1[c]);
-      }
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-#pragma unroll
-        for (int v = 0; v < VX; ++v) rq1[c][v] = pq1[c][v] + a.m2 * (pq1[c][v] - pk1[c][v]);
-      }
-    }
-    float pk3[3][VX], pm3[3][VX], b3[VX];
-    load_raw(f + 1, pk3, pm3, b3);
-    lds_put<VX, VEC>(zk, w, LW, xl, zk2);
-    lds_put<VX, VEC>(rqy, w, LW, xl, rq1[1]);
-    __syncthreads();  // (2) z_k of plane f and r_{k+1} of plane t + 1 visible
-    lds_get<VX, VEC>(zk, wd, LW, xl, zdn_k);  // for the next plane's dual step
-    float zq1[VX] = {};
-    if (need_zq) {
-      float up[VX];
-      lds_get<VX, VEC>(rqy, wu, LW, xl, up);
-      pair_primal<VX, XT, VEC>(a, t + 1, y, xb, rq1, rq0[0], up, b1, zq1);
-    }
-    lds_put<VX, VEC>(zq, w, LW, xl, zq1);
-    __syncthreads();  // (3) z_{k+1} of plane t + 1 visible
-    // p_{k+2} on plane t.
-    if (t >= z0 && need_pk2) {
-      float p2[3][VX];
-      pair_dual<VX, XT, VEC>(a, t, y, xb, zq0, zq1, zdn_q, rq0, p2);
-      if (out_row && out_col) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) store_row<VX, VEC, true>(a.p_k2 + c * a.vol, bd, t, y, xb, p2[c]);
-      }
-    }
-    lds_get<VX, VEC>(zq, wd, LW, xl, zdn_q);  // z_{k+1} of the row below on plane t + 1
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      b1[v] = b2[v];
-      b2[v] = b3[v];
-      zk1[v] = zk2[v];
-      zq0[v] = zq1[v];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        rk1[c][v] = rk2[c][v];
-        pk1[c][v] = pk2[c][v];
-        pk2[c][v] = pk3[c][v];
-        pm2[c][v] = pm3[c][v];
-        rq0[c][v] = rq1[c][v];
-      }
-    }
-  }
-}
-
-// out = max(b - lambda L(p), 0) (optionally its refractive index), same strip layout.
-template <int VX, int TY, bool VEC, bool BATCH>
-__global__ void __launch_bounds__(64) k_tv_primal(TvArgs a, int chunks, float* out, int to_index,
-                                                  float nm2, float inv_k02) {
-  if constexpr (BATCH) {
-    a.b = shifted(a.b, batch_volume() * a.vol);
-    a.p_in = shifted(a.p_in, 3 * batch_volume() * a.vol);
-    out += batch_volume() * a.vol;
-  }
-  const int t = xcd_tile();
-  const int y0 = (t / chunks) * TY;
-  const int z0 = (t % chunks) * a.zlen;
-  const int z1 = min(z0 + a.zlen, a.nz);
-  const int xb = static_cast<int>(threadIdx.x) * VX;
-  float p[3][TY + 1][VX];
-  float pz_below[TY + 1][VX];
-  float py_top[VX];
-  float bb[TY + 1][VX];
-  float x3[TY + 1][VX];
-#pragma unroll
-  for (int j = 0; j < TY; ++j) load_row<VX, VEC>(a.p_in, a, z0 - 1, y0 + j, xb, pz_below[j]);
-#pragma unroll
-  for (int v = 0; v < VX; ++v) pz_below[TY][v] = 0.0f;
-  for (int z = z0; z < z1; ++z) {
-#pragma unroll
-    for (int j = 0; j < TY; ++j) {
-      // Read once (non-temporal), except the y component of the strip's last row, which the
-      // strip below reads as its row above (256^3 FISTA-TV request 20.33 -> 20.17 ms).
-      load_row<VX, VEC, false, true>(a.p_in, a, z, y0 + j, xb, p[0][j]);
-      if (j == TY - 1) {
-        load_row<VX, VEC>(a.p_in + a.vol, a, z, y0 + j, xb, p[1][j]);
-      } else {
-        load_row<VX, VEC, false, true>(a.p_in + a.vol, a, z, y0 + j, xb, p[1][j]);
-      }
-      load_row<VX, VEC, false, true>(a.p_in + 2 * a.vol, a, z, y0 + j, xb, p[2][j]);
-      load_row<VX, VEC, false, true>(a.b, a, z, y0 + j, xb, bb[j]);
-    }
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      p[0][TY][v] = p[1][TY][v] = p[2][TY][v] = 0.0f;
-      bb[TY][v] = 0.0f;
-    }
-    load_row<VX, VEC>(a.p_in + a.vol, a, z, y0 - 1, xb, py_top);
-    primal_plane<VX, TY>(a, z, y0, xb, p, py_top, pz_below, bb, x3);
-#pragma unroll
-    for (int j = 0; j < TY; ++j) {
-      float o[VX];
-#pragma unroll
-      for (int v = 0; v < VX; ++v) {
-        o[v] = to_index ? index_from_potential(x3[j][v], 0.0f, nm2, inv_k02) : x3[j][v];
-        pz_below[j][v] = p[0][j][v];
-      }
-      store_row<VX, VEC>(out, a, z, y0 + j, xb, o);
-    }
-  }
+  const int first_plane = max(m.z0 - M::HL, 0);
+  m.last_plane = m.z1 - 1 + T;
+  m.load(first_plane);
+  for (int f = first_plane; f <= m.last_plane; f += M::kUnroll) m.template planes<0>(f);
 }
 
 __global__ void k_fill(float* d, long n, float v) {
@@ -789,18 +431,6 @@ void fill(float* d, long n, float v, hipStream_t s) {
 
 namespace {
 
-constexpr int kRows = 2;
-
-int lanes_x(int nx) {
-  const int vx = (nx + 63) / 64;
-  if (vx <= 1) return 1;
-  if (vx <= 2) return 2;
-  if (vx <= 4) return 4;
-  if (vx <= 6) return 6;
-  if (vx <= 8) return 8;
-  throw InvalidArgument("tv: volume side above 512");
-}
-
 // CUs of the current device, queried once per device.
 int device_cus() {
   static std::atomic<int> cache[64];
@@ -817,144 +447,17 @@ int device_cus() {
   return cus;
 }
 
-// One wave per strip of kRows rows and z chunk: chunks of kZChunk planes, halved (down to 2)
-// while the grid holds fewer than two waves per SIMD (128^3: 4 planes and 2048 waves, where
-// 16-plane chunks gave 512 waves for 1024 SIMDs).
-dim3 strip_grid(int ny, int nz, TvArgs& a, int* chunks, int batch) {
-  const long strips = (ny + kRows - 1) / kRows;
-  const long want = 8L * device_cus();
-  int zlen = kZChunk;
-  while (zlen > 2 && strips * ((nz + zlen - 1) / zlen) * batch < want) zlen /= 2;
-  a.zlen = zlen;
-  *chunks = (nz + zlen - 1) / zlen;
-  return dim3(static_cast<unsigned>(strips * *chunks), static_cast<unsigned>(batch));
-}
-
-// Whole-vector row access (see load_row) when the row splits into whole lane chunks.
-template <int VX>
-bool rows_vec(int nx) {
-  return VX % 2 == 0 && nx % VX == 0;
-}
-
-template <int VX, bool BATCH>
-void launch_step_as(const TvArgs& a, int chunks, dim3 grid, hipStream_t s) {
-  if constexpr (VX % 2 == 0) {
-    if (rows_vec<VX>(a.nx)) {
-      hipLaunchKernelGGL((k_fgp_step<VX, kRows, true, BATCH>), grid, dim3(64), 0, s, a, chunks);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((k_fgp_step<VX, kRows, false, BATCH>), grid, dim3(64), 0, s, a, chunks);
-}
-
-// A grid with a second dimension runs a batch of volumes (strip_grid).
-template <int VX>
-void launch_step(const TvArgs& a, int chunks, dim3 grid, hipStream_t s) {
-  if (grid.y > 1) {
-    launch_step_as<VX, true>(a, chunks, grid, s);
-  } else {
-    launch_step_as<VX, false>(a, chunks, grid, s);
-  }
-}
-
-template <int VX, bool BATCH>
-void launch_primal_as(const TvArgs& a, int chunks, dim3 grid, float* out, int ti, float nm2,
-                      float inv_k02, hipStream_t s) {
-  if constexpr (VX % 2 == 0) {
-    if (rows_vec<VX>(a.nx)) {
-      hipLaunchKernelGGL((k_tv_primal<VX, kRows, true, BATCH>), grid, dim3(64), 0, s, a, chunks,
-                         out, ti, nm2, inv_k02);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((k_tv_primal<VX, kRows, false, BATCH>), grid, dim3(64), 0, s, a, chunks, out,
-                     ti, nm2, inv_k02);
-}
-
-template <int VX>
-void launch_primal(const TvArgs& a, int chunks, dim3 grid, float* out, int ti, float nm2,
-                   float inv_k02, hipStream_t s) {
-  if (grid.y > 1) {
-    launch_primal_as<VX, true>(a, chunks, grid, out, ti, nm2, inv_k02, s);
-  } else {
-    launch_primal_as<VX, false>(a, chunks, grid, out, ti, nm2, inv_k02, s);
-  }
-}
-
-}  // namespace
-
-void fgp_step(const float* b, const float* p_in, const float* p_prev, float* p_out, int nz,
-              int ny, int nx, float lambda, float step, float momentum, bool first,
-              hipStream_t s, int batch) {
-  require(batch >= 1 && batch <= 65535, "fgp_step: batch must be 1 to 65535");
-  TvArgs a{b, p_in, p_prev, p_out, static_cast<long>(nz) * ny * nx, nz, ny, nx,
-           lambda, step, momentum, first ? 1 : 0};
-  int chunks = 0;
-  const dim3 grid = strip_grid(ny, nz, a, &chunks, batch);
-  switch (lanes_x(nx)) {
-    case 1: launch_step<1>(a, chunks, grid, s); break;
-    case 2: launch_step<2>(a, chunks, grid, s); break;
-    case 4: launch_step<4>(a, chunks, grid, s); break;
-    case 6: launch_step<6>(a, chunks, grid, s); break;
-    default: launch_step<8>(a, chunks, grid, s); break;
-  }
-  check_launch("fgp_step");
-}
-
-void tv_primal(const float* b, const float* p, int nz, int ny, int nx, float lambda, float* out,
-               bool to_index, float nm2, float inv_k02, hipStream_t s, int batch) {
-  require(batch >= 1 && batch <= 65535, "tv_primal: batch must be 1 to 65535");
-  TvArgs a{b, p, nullptr, nullptr, static_cast<long>(nz) * ny * nx, nz, ny, nx,
-           lambda, 0.0f, 0.0f, 1};
-  int chunks = 0;
-  const dim3 grid = strip_grid(ny, nz, a, &chunks, batch);
-  const int ti = to_index ? 1 : 0;
-  switch (lanes_x(nx)) {
-    case 1: launch_primal<1>(a, chunks, grid, out, ti, nm2, inv_k02, s); break;
-    case 2: launch_primal<2>(a, chunks, grid, out, ti, nm2, inv_k02, s); break;
-    case 4: launch_primal<4>(a, chunks, grid, out, ti, nm2, inv_k02, s); break;
-    case 6: launch_primal<6>(a, chunks, grid, out, ti, nm2, inv_k02, s); break;
-    default: launch_primal<8>(a, chunks, grid, out, ti, nm2, inv_k02, s); break;
-  }
-  check_launch("tv_primal");
-}
-
-namespace {
-
-// Rows per block of the two-step kernel: NW waves, NW - 4 output rows, as many waves as the
-// registers of VX floats per lane leave room for in one block per CU. Rows up to 256 wide are
-// held whole by a wave; wider rows are cut into x tiles of at most 62 VX output columns (one
-// lane of VX columns of halo on either side), balanced. Tiles of 4 columns per lane (12 waves,
-// 8 output rows) when the row width is a multiple of 4, so that every access is a float4: at
-// 384^3, 2 tiles of 192 columns ran a pass in 593 us against 618 us for 4 tiles of 96 at 2
-// columns per lane (16 waves, 12 output rows), which leave fewer lanes and rows idle; at 512^3
-// and 320^3 the two were equal (1667 against 1658 us, 417 against 420 us). Other widths take
-// tiles of 2 columns per lane, whole float2s for even widths.
-int pair_waves(int vx) { return vx == 1 ? 16 : (vx == 2 ? 16 : 12); }
-int pair_tile_vx(int nx) { return nx % 4 == 0 ? 4 : 2; }
-
-// Planes per z chunk for a grid of `tiles` row tiles: the length from kPairChunkMin to
-// kPairChunk that minimises the rounds of blocks each CU runs times the planes a block marches
-// (its chunk and two warm-up planes), the longest on ties. 256^3: 32 planes, 256 blocks, one
-// round; 384^3 in x tiles of 4 columns per lane: 48 planes, 768 blocks, three full rounds (64
-// planes would leave the third round a quarter full; tiles of 2 columns per lane took 64);
-// 128^3: 6 planes and 242 blocks (8-plane chunks left 80 CUs idle and spent a fifth of each
-// block on warm-up).
-int pair_chunk(const void* kernel, std::atomic<int>& per_cu_cache, int threads, std::size_t lds,
-               int tiles, int nz) {
-  int per_cu = per_cu_cache.load(std::memory_order_relaxed);
-  if (per_cu == 0) {
-    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, lds),
-          "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-    per_cu = std::max(per_cu, 1);
-    per_cu_cache.store(per_cu, std::memory_order_relaxed);
-  }
-  const long slots = static_cast<long>(device_cus()) * per_cu;
-  int best = kPairChunk;
+// Planes per z chunk for a grid of `tiles` tiles (one block per CU): the length that minimises the
+// rounds of blocks per CU times the planes a block marches (its chunk and a halo of planes on
+// either side, in turns of `turn` planes); the longest on ties.
+int step_chunk(int steps, int halo, int turn, long tiles, int nz) {
+  const long slots = device_cus();
+  int best = nz;
   long best_cost = -1;
-  for (int zl = kPairChunk; zl >= kPairChunkMin; --zl) {
-    const long blocks = static_cast<long>(tiles) * ((nz + zl - 1) / zl);
-    const long cost = (blocks + slots - 1) / slots * (zl + 2);
+  for (int zl = nz; zl >= 1; --zl) {
+    const long chunks = (nz + zl - 1) / zl;
+    const long planes = (std::min(zl + halo, nz + steps) + turn - 1) / turn * turn;
+    const long cost = (tiles * chunks + slots - 1) / slots * planes;
     if (best_cost < 0 || cost < best_cost) {
       best_cost = cost;
       best = zl;
@@ -963,82 +466,54 @@ int pair_chunk(const void* kernel, std::atomic<int>& per_cu_cache, int threads, 
   return best;
 }
 
-// Volumes of a batch are the grid's second dimension; their blocks count in the chunk choice.
-template <int VX, int NW, bool VEC, bool XT, bool BATCH>
-void launch_pair_kernel_as(PairArgs a, int tiles, std::size_t lds, hipStream_t s, int batch) {
-  // Blocks per CU of this kernel (its registers and LDS; the same on every gfx950 device).
-  static std::atomic<int> per_cu{0};
-  a.zlen = pair_chunk(reinterpret_cast<const void*>(&k_fgp_pair<VX, NW, VEC, XT, BATCH>), per_cu,
-                      NW * 64, lds, tiles * batch, a.nz);
+template <int T, bool FIRST, bool FINAL>
+void launch_steps(StepArgs a, hipStream_t s, int batch, bool exact) {
+  const auto cut = [](int n, int width, int& own, int& halo) {
+    halo = n <= width ? 0 : kHalo;
+    own = width - 2 * halo;
+    return (n + own - 1) / own;
+  };
+  a.tiles_x = cut(a.nx, 64, a.tile_x, a.halo_x);
+  a.tiles_y = cut(a.ny, kWaves * kRows, a.tile_y, a.halo_y);
+  const int tiles = a.tiles_x * a.tiles_y;
+  a.zlen = step_chunk(T, 2 * T + (FINAL ? 1 : 0), FINAL ? 1 : T + 1,
+                      static_cast<long>(tiles) * batch, a.nz);
   const int chunks = (a.nz + a.zlen - 1) / a.zlen;
-  hipLaunchKernelGGL((k_fgp_pair<VX, NW, VEC, XT, BATCH>),
-                     dim3(static_cast<unsigned>(tiles * chunks), static_cast<unsigned>(batch)),
-                     dim3(NW * 64), lds, s, a, chunks);
-}
-
-template <int VX, int NW, bool VEC, bool XT>
-void launch_pair_kernel(PairArgs a, int tiles, std::size_t lds, hipStream_t s, int batch) {
-  if (batch > 1) {
-    launch_pair_kernel_as<VX, NW, VEC, XT, true>(a, tiles, lds, s, batch);
+  const dim3 grid(static_cast<unsigned>(tiles * chunks), static_cast<unsigned>(batch));
+  const dim3 block(kWaves * 64);
+  if (a.ny % kRows != 0) {
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, false, true>), grid, block, 0, s, a);
+  } else if (exact) {
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, true, true>), grid, block, 0, s, a);
   } else {
-    launch_pair_kernel_as<VX, NW, VEC, XT, false>(a, tiles, lds, s, batch);
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, true, false>), grid, block, 0, s, a);
   }
 }
 
-template <int VX, int NW, bool XT>
-void launch_pair(const PairArgs& a, int tiles, hipStream_t s, int batch) {
-  // Four row buffers of NW rows of nx floats (64 VX per x tile): at most 48 KiB.
-  const std::size_t lds = 4 * static_cast<std::size_t>(NW) * (XT ? 64 * VX : a.nx) * sizeof(float);
-  if constexpr (VX % 2 == 0) {
-    if (rows_vec<VX>(a.nx)) {
-      launch_pair_kernel<VX, NW, true, XT>(a, tiles, lds, s, batch);
-      return;
-    }
-  }
-  launch_pair_kernel<VX, NW, false, XT>(a, tiles, lds, s, batch);
-}
-
-}  // namespace
-
-bool fgp_pair_supported(int nx) { return nx >= 1 && nx <= 512; }
-
-void fgp_pair(const float* b, const float* p_k, const float* p_km1, float* p_k1, float* p_k2,
-              int nz, int ny, int nx, float lambda, float step, float m1, bool first, float m2,
-              hipStream_t s, int batch) {
-  require(fgp_pair_supported(nx), "fgp_pair: rows up to 512 wide");
-  require(batch >= 1 && batch <= 65535, "fgp_pair: batch must be 1 to 65535");
-  int vx = std::min(lanes_x(nx), 4);
-  int tiles_x = 1;
-  int xt = nx;
-  if (nx > 64 * 4) {
-    vx = pair_tile_vx(nx);
-    const int widest = 62 * vx;
-    tiles_x = (nx + widest - 1) / widest;
-    xt = ((nx + tiles_x - 1) / tiles_x + vx - 1) / vx * vx;  // balanced tiles, whole lanes
-  }
-  const int nw = pair_waves(vx);
-  const int rows = nw - 4;
-  const int tiles_y = (ny + rows - 1) / rows;
-  const int tiles = tiles_x * tiles_y;
-  PairArgs a{b,  p_k,    p_km1, p_k1, p_k2,          static_cast<long>(nz) * ny * nx,
-             nz, ny,     nx,    lambda, step,        m1, first ? 1 : 0, m2, 0, xt, tiles_x};
-  if (tiles_x > 1) {
-    if (vx == 4) {
-      launch_pair<4, 12, true>(a, tiles, s, batch);
-    } else {
-      launch_pair<2, 16, true>(a, tiles, s, batch);
-    }
+template <int T>
+void launch_steps_of(const StepArgs& a, hipStream_t s, int batch, bool exact) {
+  if (a.x) {
+    launch_steps<T, false, true>(a, s, batch, exact);
+  } else if (T == kMaxSteps && a.first) {
+    // The first of several passes, the longest: without p_{k-1} at all (256^3: 219 against 240 us).
+    launch_steps<T, T == kMaxSteps, false>(a, s, batch, exact);
   } else {
-    switch (vx) {
-      case 1: launch_pair<1, 16, false>(a, tiles, s, batch); break;
-      case 2: launch_pair<2, 16, false>(a, tiles, s, batch); break;
-      default: launch_pair<4, 12, false>(a, tiles, s, batch); break;
-    }
+    launch_steps<T, false, false>(a, s, batch, exact);
   }
-  check_launch("fgp_pair");
 }
 
-namespace {
+// `steps` FGP steps in one pass; with x set, the prox output after them (0 steps: of p_k). Only
+// whole quads have kernels with fused arithmetic.
+void fgp_steps(int steps, const StepArgs& a, hipStream_t s, int batch, bool exact) {
+  switch (steps) {
+    case 0: launch_steps<0, true, true>(a, s, batch, exact); break;
+    case 1: launch_steps_of<1>(a, s, batch, exact); break;
+    case 2: launch_steps_of<2>(a, s, batch, exact); break;
+    case 3: launch_steps_of<3>(a, s, batch, exact); break;
+    default: launch_steps_of<4>(a, s, batch, exact); break;
+  }
+  check_launch("fgp_steps");
+}
 
 // Floats of one dual buffer (three components per volume of the batch, one volume's after
 // another's), rounded up to 256 bytes so that every buffer of a workspace starts 256-byte
@@ -1076,67 +551,73 @@ void TvState::reset(hipStream_t s, int batch) {
 std::size_t TvState::bytes() const { return owned_.bytes(); }
 
 // tv_prox of the reference (src/cpu/tv.cpp:7-44): r <- p, `inner` FGP steps, out = primal(p).
-// The dual iterates rotate through four buffers: a pass reads p_k and p_{k-1} (r is formed
-// inside it) and writes p_{k+1} (and p_{k+2} for a two-step pass) to buffers nobody reads in
-// that pass. Steps go in pairs where the row width allows, with an odd last step on its own; the
-// momentum sequence is that of single steps. A last pass that is a pair skips p_{k+1}, which the
-// next call does not read (its first step uses r = p). The prox leaves p in buffer cur_ for the
-// next call.
+// The steps go in as few passes as they need, the last of which forms the output. The dual
+// iterates rotate through four buffers: a pass of T steps reads p_k and p_{k-1} (r is formed
+// inside it) and writes p_{k+T-1} and p_{k+T} to buffers nobody reads in that pass; the last pass
+// skips p_{k+T-1}, which the next call does not read (its first step uses r = p). The prox leaves
+// p in buffer cur_ for the next call.
 void TvState::prox(const float* b, float* out, float lambda, int inner, hipStream_t s,
                    bool to_index, float nm2, float inv_k02, Event* t0, Event* t1) {
+  if (nx_ > 512) throw InvalidArgument("tv: volume side above 512");
   const float step = 1.0f / (12.0f * lambda);
-  const bool pairs = fused_ && fgp_pair_supported(nx_);
+  // An output that overlaps b is written only by a pass without steps: the stages of the others
+  // read b beyond their own points, its last stage at them alone.
+  const bool apart = out + vol_ * batch_ <= b || b + vol_ * batch_ <= out;
+  const bool joined = fused_ && apart && inner > 0;
+  const int most = fused_ ? kMaxSteps : 1;
+  const int passes = (inner + most - 1) / most;
+  StepArgs a{};
+  a.b = b;
+  a.vol = vol_;
+  a.nz = nz_;
+  a.ny = ny_;
+  a.nx = nx_;
+  a.lambda = lambda;
+  a.step = step;
+  a.to_index = to_index ? 1 : 0;
+  a.nm2 = nm2;
+  a.inv_k02 = inv_k02;
   float t = 1.0f;
   float m_prev = 0.0f;
   int cur = cur_;
   int prev = (cur_ + 1) % 4;
-  launches_ = 0;
-  const auto free_buffers = [&](int& f1, int& f2) {
-    f1 = -1;
-    f2 = -1;
-    for (int i = 0; i < 4; ++i) {
-      if (i == cur || i == prev) continue;
-      if (f1 < 0) {
-        f1 = i;
-      } else {
-        f2 = i;
-      }
-    }
-  };
+  int left = inner;
+  launches_ = passes;
   if (t0) t0->record(s);
-  for (int k = 0; k < inner;) {
-    int f1 = 0, f2 = 0;
-    free_buffers(f1, f2);
-    if (pairs && k + 1 < inner) {
-      const float m1 = m_prev;
-      float tn = fista_t(t);
-      const float m2 = (t - 1.0f) / tn;
-      t = tn;
-      // The last pass skips p_{k+1}: the next prox starts from p alone.
-      const bool last = k + 2 == inner;
-      fgp_pair(b, p_[cur], p_[prev], last ? nullptr : p_[f1], p_[f2],
-               nz_, ny_, nx_, lambda, step, m1, k == 0, m2, s, batch_);
-      tn = fista_t(t);
-      m_prev = (t - 1.0f) / tn;
-      t = tn;
-      prev = f1;
-      cur = f2;
-      k += 2;
-    } else {
-      fgp_step(b, p_[cur], p_[prev], p_[f1], nz_, ny_, nx_, lambda, step,
-               m_prev, k == 0, s, batch_);
+  for (int k = 0; k < passes; ++k) {
+    // Nearly equal shares of what is left, the larger ones first.
+    const int steps = (left + passes - k - 1) / (passes - k);
+    const bool last = k + 1 == passes;
+    left -= steps;
+    int f[2] = {0, 0};
+    for (int i = 0, n = 0; i < 4; ++i) {
+      if (i != cur && i != prev && n < 2) f[n++] = i;
+    }
+    a.p_k = p_[cur];
+    a.p_km1 = p_[prev];
+    // A pass of one step leaves p_k as the previous iterate.
+    a.p_prev = last || steps == 1 ? nullptr : p_[f[0]];
+    a.p_last = p_[f[1]];
+    a.x = last && joined ? out : nullptr;
+    a.first = k == 0 ? 1 : 0;
+    for (int i = 0; i < steps; ++i) {
+      a.m[i] = m_prev;
       const float tn = fista_t(t);
       m_prev = (t - 1.0f) / tn;
       t = tn;
-      prev = cur;
-      cur = f1;
-      k += 1;
     }
-    ++launches_;
+    fgp_steps(steps, a, s, batch_, exact_);
+    prev = steps == 1 ? cur : f[0];
+    cur = f[1];
   }
   if (t1) t1->record(s);
   cur_ = cur;
-  tv_primal(b, p_[cur_], nz_, ny_, nx_, lambda, out, to_index, nm2, inv_k02, s, batch_);
+  if (joined) return;
+  a.p_k = p_[cur_];
+  a.p_km1 = a.p_prev = a.p_last = nullptr;
+  a.x = out;
+  a.first = 1;
+  fgp_steps(0, a, s, batch_, exact_);
 }
 
 }  // namespace qh

@@ -12,30 +12,10 @@ namespace qh {
 // d[0, n) = v, by a kernel (safe inside captured graphs, unlike a memset node).
 void fill(float* d, long n, float v, hipStream_t s);
 
-// One fused FGP dual step over a dense (nz, ny, nx) volume: r = p_k + m (p_k - p_prev) (r = p_k
-// on the first step), z = max(b - lambda L(r), 0) at each voxel and its upper neighbours,
-// g = L^T z, and the projected dual update p_out = P(r + step g). p_out is a third buffer.
-// With batch > 1, every array holds that many volumes one after another (b, out: nz ny nx
-// floats apart; duals: three components, 3 nz ny nx floats apart), all in one launch.
-void fgp_step(const float* b, const float* p_in, const float* p_prev, float* p_out, int nz,
-              int ny, int nx, float lambda, float step, float momentum, bool first,
-              hipStream_t s, int batch = 1);
-
-// Two FGP steps in one pass (rows up to 256 wide): from p_k, p_{k-1} to p_{k+1} and p_{k+2},
-// bit for bit what two fgp_step calls with momenta m1 then m2 give. The four buffers are
-// distinct; p_k1 may be null (not written).
-bool fgp_pair_supported(int nx);
-void fgp_pair(const float* b, const float* p_k, const float* p_km1, float* p_k1, float* p_k2,
-              int nz, int ny, int nx, float lambda, float step, float m1, bool first, float m2,
-              hipStream_t s, int batch = 1);
-
-// out = max(b - lambda L(p), 0); with to_index the refractive index of that potential.
-void tv_primal(const float* b, const float* p, int nz, int ny, int nx, float lambda, float* out,
-               bool to_index, float nm2, float inv_k02, hipStream_t s, int batch = 1);
-
 // Dual state of the TV prox, kept across calls (FISTA warm start): four rotating dual buffers
-// of three components each. Steps run two per pass where the row width allows (set_fused(false)
-// runs them one per pass, for comparisons).
+// of three components each. Steps run up to four per pass, the last of which forms the output
+// (set_fused(false) runs them one per pass and the output in a kernel of its own, for
+// comparisons; the results are the same bits).
 class TvState {
  public:
   // The dual buffers in device memory of its own, for up to `batch` volumes proxed together.
@@ -48,12 +28,14 @@ class TvState {
   // next reset takes together: b and out then hold that many volumes one after another.
   void reset(hipStream_t s, int batch = 1);
   // out = prox_{lambda TV, x >= 0}(b) by `inner` FGP steps from the current dual.
-  // Events t0 and t1, when given, bracket the FGP steps (not the final primal kernel).
+  // out may be b itself. Events t0 and t1, when given, bracket the passes of FGP steps.
   void prox(const float* b, float* out, float lambda, int inner, hipStream_t s,
             bool to_index = false, float nm2 = 0.0f, float inv_k02 = 0.0f, Event* t0 = nullptr,
             Event* t1 = nullptr);
   std::size_t bytes() const;
   void set_fused(bool on) { fused_ = on; }
+  // Whether every operation of a step rounds on its own (the default), or multiply-adds are fused.
+  void set_exact(bool on) { exact_ = on; }
   // Kernel passes of the last prox call.
   int launches() const { return launches_; }
 
@@ -66,6 +48,7 @@ class TvState {
   float* p_[4];  // dual buffers of three components each, inside owned_ or the workspace
   int cur_ = 0;
   bool fused_ = true;
+  bool exact_ = true;
   int launches_ = 0;
 };
 

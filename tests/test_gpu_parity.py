@@ -218,6 +218,43 @@ def test_tv_two_step_passes_equal_single_steps(device, shape, inner):
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("shape", [(9, 32, 64), (5, 33, 65), (7, 31, 57), (3, 25, 120), (40, 49, 113),
+                                   (2, 1, 1), (1, 24, 56), (12, 56, 121)])
+@pytest.mark.parametrize("inner", [0, 1, 3, 4, 9])
+def test_tv_tile_edges_match_oracle(device, oracle, shape, inner):
+    """Rows and columns at, below and above one tile (32 x 64) and the two that overlapping tiles
+    own (24 x 56), row counts that leave 1 to 3 rows in the last group of four, one to three passes
+    and none. Bound: a step rounds each dual component (at most 1) a few times at 2^-24, and the
+    output adds six of them times lambda: under inner 6 lambda 2^-22 < 3e-7 for these."""
+    from qoraholo_amd import _native
+
+    rng = np.random.default_rng(shape[1] + inner)
+    b = (rng.standard_normal(shape) * 0.1 + 0.05).astype(np.float32)
+    want = oracle.tv_prox(b, 0.02, inner)
+    got = np.empty_like(b)
+    _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *shape, 0.02, inner, 1,
+                                               _native.ptr(got)))
+    assert np.max(np.abs(got - want)) < 1e-6
+
+
+def test_tv_infinities_and_nans_stay_where_the_oracle_has_them(device, oracle):
+    """One voxel that is infinite or NaN, inside and on the faces and tile seams."""
+    from qoraholo_amd import _native
+
+    rng = np.random.default_rng(5)
+    base = (rng.standard_normal((10, 40, 70)) * 0.1 + 0.05).astype(np.float32)
+    for value in (np.inf, -np.inf, np.nan):
+        for at in ((4, 20, 30), (0, 0, 0), (9, 39, 69), (5, 24, 56), (5, 23, 55), (0, 20, 69)):
+            b = base.copy()
+            b[at] = value
+            want = oracle.tv_prox(b, 0.02, 5)
+            got = np.empty_like(b)
+            _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *b.shape, 0.02, 5, 1,
+                                                       _native.ptr(got)))
+            np.testing.assert_allclose(got, want, rtol=0, atol=1e-6, equal_nan=True,
+                                       err_msg=f"{value} at {at}")
+
+
 @pytest.mark.parametrize("shape,inner,batch", [((9, 20, 64), 5, 3), ((16, 16, 128), 4, 3),
                                                ((20, 30, 300), 3, 3), ((12, 18, 302), 5, 3),
                                                ((40, 64, 256), 4, 3), ((256, 256, 256), 4, 2)])

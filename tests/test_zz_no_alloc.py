@@ -44,6 +44,25 @@ def test_noalloc_prox_equals_allocating_prox(device):
         assert np.all(got >= 0)
 
 
+def test_noalloc_prox_in_place(device):
+    """The output may be the input: tiles read b beyond their own points while others write."""
+    import torch
+    from qoraholo_amd import _native
+
+    lib = _native.lib()
+    rng = np.random.default_rng(12)
+    stream = torch.cuda.current_stream()
+    for shape, inner in [((20, 70, 130), 10), ((9, 33, 65), 3), ((4, 8, 16), 0)]:
+        b = (rng.standard_normal(shape) * 0.2 + 0.3).astype(np.float32)
+        want = _prox_allocating(lib, _native, b, 0.03, inner, 1)
+        bd = torch.from_numpy(b).cuda()
+        _native.check(lib.qh_hip_tv_prox_dev_noalloc(
+            _native.ptr(bd.data_ptr()), *shape, 0.03, inner, 1, _native.ptr(bd.data_ptr()),
+            _native.ptr(stream.cuda_stream)))
+        torch.cuda.synchronize()
+        assert np.array_equal(bd.cpu().numpy().view(np.uint32), want.view(np.uint32)), shape
+
+
 def test_noalloc_prox_refuses_volumes_above_the_limit(device):
     import torch
     from qoraholo_amd import _native
