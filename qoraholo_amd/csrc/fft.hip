@@ -10,6 +10,7 @@
 #include "common.hpp"
 #include "fft.hpp"
 #include "fft4s.hpp"
+#include "fft_args.hpp"
 #include "runtime.hpp"
 
 namespace qh {
@@ -41,23 +42,6 @@ const float2* table(int kind, int n) {
   }
   return buf.get();
 }
-
-__device__ __forceinline__ long line_base(long l, const Lines& g) {
-  return (l / g.inner) * g.outer + (l % g.inner) * g.inner_stride;
-}
-
-struct LinesArgs {
-  const float2* in;
-  float2* out;
-  Lines g;
-  int n;
-  int lines_per_block;
-  FftFactors f;
-  const float2* tw;
-  int inverse;
-  float scale;
-  int alt_mod;
-};
 
 // CONTIG: lines contiguous in memory (stride 1), LDS line-major, threads walk along lines.
 // Otherwise lines are adjacent (inner_stride 1): each row of the block is one coalesced
@@ -106,21 +90,6 @@ __global__ void __launch_bounds__(kThreads) k_fft_lines(LinesArgs a) {
     a.out[base[line] + i * a.g.stride] = v;
   }
 }
-
-struct RowsArgs {
-  const float* x;
-  const float* x2;
-  float* xo;
-  long x_pitch;
-  float2* c;
-  long c_pitch;
-  long rows;
-  int n;
-  int rows_per_block;
-  FftFactors f;      // of n / 2
-  const float2* tw;  // exp(-2 pi i t / n), t in [0, n)
-  RealOp op;
-};
 
 // Real rows of even length n through a complex transform of n/2 packed samples
 // z[j] = x[2j] + i x[2j+1]; X[k] = (Z[k] + conj Z[-k]) / 2 - i/2 w^k (Z[k] - conj Z[-k]).
@@ -230,24 +199,6 @@ __global__ void __launch_bounds__(kThreads) k_irfft_rows(RowsArgs a) {
     px[0] = u0;
     px[1] = u1;
   }
-}
-
-struct ZArgs {
-  float2* e;
-  const float2* a;
-  const std::uint8_t* hits;
-  long lines;
-  long plane;
-  int nz;
-  int lines_per_block;
-  FftFactors f;
-  const float2* tw;
-  long vol;  // elements between the volumes of a batch (0: one volume, lines == plane)
-};
-
-// First element of z line l: lines past a plane's belong to the next volumes of the batch.
-__device__ __forceinline__ long z_line_base(const ZArgs& a, long l) {
-  return a.vol == 0 ? l : (l / a.plane) * a.vol + l % a.plane;
 }
 
 __global__ void __launch_bounds__(kThreads) k_z_roundtrip_restore(ZArgs a) {
@@ -643,7 +594,7 @@ void fft_lines(const float2* in, float2* out, int n, const Lines& l, bool invers
   if (l.count == 0) return;
   LinesArgs a{in, out, l, n, 0, fft_factors(n), fft_twiddles(n), inverse ? 1 : 0, scale, alt_mod};
   if (l.stride != 1) require(l.inner_stride == 1, "fft: strided lines must be adjacent");
-  if (with_four_step<LaunchLines>(n, a, l.stride == 1, s)) {
+  if (with_four_step<LaunchLines>(n, a, l.stride == 1, s) || split_fft_lines(a, l.stride == 1, s)) {
     check_launch("fft_lines");
     return;
   }
@@ -669,7 +620,8 @@ void rfft_rows(const float* x, const float* x2, long x_pitch, float2* out, long 
   const int m = n / 2;
   RowsArgs a{x, x2, nullptr, x_pitch, out, out_pitch, rows, n, contig_lines_per_block(m),
              fft_factors(m), fft_twiddles(n), op};
-  if (x_pitch % 2 == 0 && with_four_step<LaunchRows>(m, a, false, s)) {
+  if (x_pitch % 2 == 0 &&
+      (with_four_step<LaunchRows>(m, a, false, s) || split_rfft_rows(a, false, s))) {
     check_launch("rfft_rows");
     return;
   }
@@ -687,7 +639,8 @@ void irfft_rows(const float2* in, long in_pitch, float* x, long x_pitch, long ro
   const int m = n / 2;
   RowsArgs a{nullptr, nullptr, x, x_pitch, const_cast<float2*>(in), in_pitch, rows, n,
              contig_lines_per_block(m), fft_factors(m), fft_twiddles(n), op};
-  if (x_pitch % 2 == 0 && with_four_step<LaunchRows>(m, a, true, s)) {
+  if (x_pitch % 2 == 0 &&
+      (with_four_step<LaunchRows>(m, a, true, s) || split_rfft_rows(a, true, s))) {
     check_launch("irfft_rows");
     return;
   }
@@ -704,7 +657,7 @@ void z_roundtrip_restore(float2* e, const float2* a, const std::uint8_t* hits, i
   const long plane = static_cast<long>(ny) * h;
   ZArgs z{e, a, hits, plane * batch, plane, nz, strided_lines_per_block(nz), fft_factors(nz),
           fft_twiddles(nz), batch > 1 ? plane * nz : 0};
-  if (with_four_step<LaunchZrt>(nz, z, s)) {
+  if (with_four_step<LaunchZrt>(nz, z, s) || split_z_roundtrip(z, s)) {
     check_launch("z_roundtrip_restore");
     return;
   }

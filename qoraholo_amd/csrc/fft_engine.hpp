@@ -23,7 +23,8 @@
 // cheap barriers); column blocks hold at least 16 lines so that each load spans whole 128-byte
 // lines.
 // LdsLines: any length that factors into 2, 3 and 5 (up to 2048), lines held in LDS between
-// radix passes, 256 threads.
+// radix passes, 256 threads; for the lengths that neither RegLines nor SplitLines
+// (split_lines.hpp) hold in registers.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -104,6 +104,18 @@ def test_jvp_matches_oracle(device, qh, oracle, nz, n, count):
     assert np.array_equal(qh.bpm_jvp(x, h, il, g, chunk=1), got)
 
 
+@pytest.mark.parametrize("nz,n", [(6, 36), (5, 50), (4, 90), (4, 108), (3, 162), (3, 250), (2, 320)])
+def test_two_group_lengths_match_oracle(device, qh, oracle, nz, n):
+    """The forward model and its adjoint on lines of the two-group register engine."""
+    g, il, ri, x = case(qh, nz, n)
+    got = qh.bpm_forward(ri, il, g)
+    want = oracle.bpm_forward(x, il, GEOM)
+    assert rel_l2(got - 1, want - 1) < 5e-5
+    rng = np.random.default_rng(n)
+    r = (rng.standard_normal(want.shape) + 1j * rng.standard_normal(want.shape)).astype(np.complex64)
+    assert rel_l2(qh.bpm_vjp(x, r, il, g), oracle.bpm_vjp(x, r, il, GEOM)) < 2e-5
+
+
 def test_jvp_adjoint_identity_and_difference_on_device(device, qh):
     """<J h, r> = <h, J^T r> with both sides from the device, and J h against a central
     difference of the device forward model (the checks of the reference's
