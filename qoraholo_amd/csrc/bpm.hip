@@ -24,6 +24,7 @@
 
 #include "bpm.hpp"
 #include "bpm_kernels.hpp"
+#include "bpm_plane.hpp"
 #include "common.hpp"
 #include "fft.hpp"
 #include "fft_engine.hpp"
@@ -268,10 +269,33 @@ void BpmModel::set_screen(const float* x, hipStream_t s) {
   check_launch("bpm_screen");
 }
 
+// Arguments of the one-launch march of small planes (bpm_plane.hip).
+BpmPlaneArgs BpmModel::plane_args(int a0, int chunk_count, bool keep) const {
+  BpmPlaneArgs p{};
+  p.tw = fft_twiddles(n_);
+  p.nz = nz_;
+  p.screen = screen_.get();
+  p.step = step_.get() + a0 * plane_;
+  p.last = last_.get() + a0 * plane_;
+  p.q = q_.get() + a0 * plane_;
+  p.w = keep ? w_.get() : nullptr;
+  p.w_slice = static_cast<long>(chunk_count) * plane_;
+  p.in = a_.get();
+  p.out = f_.get();
+  p.inv = 1.0f / static_cast<float>(plane_);
+  p.phase = phase_;
+  return p;
+}
+
 // Slices 0 .. nz-1 of illuminations [a0, a0 + chunk_count); the final T is left in f_. With
 // keep, (S, T) in front of every segment after the first go to the checkpoints and the last
-// segment's envelopes to w_.
+// segment's envelopes to w_. Small planes march through the slices in one launch; not to
+// checkpoints, which leave few slices to a launch and are asked for where memory is short.
 void BpmModel::forward_pass(int a0, int chunk_count, bool keep, hipStream_t s) {
+  if (bpm_plane_supported(n_) && (!keep || nseg_ == 1)) {
+    bpm_plane_forward(n_, chunk_count, plane_args(a0, chunk_count, keep), s);
+    return;
+  }
   const long cp = static_cast<long>(chunk_count) * plane_;
   for (int k = 0; k < nz_; ++k) {
     const int seg = k / seg_len_;
@@ -323,6 +347,10 @@ void BpmModel::recompute(int seg, int a0, int chunk_count, hipStream_t s) {
 // reduction blocks), those of slice 0 by a launch of their own; with init (the first chunk)
 // the sums start from zero, and grad needs no clearing.
 void BpmModel::adjoint(int a0, int chunk_count, float* grad, bool init, hipStream_t s) {
+  if (bpm_plane_supported(n_) && nseg_ == 1) {
+    bpm_plane_adjoint(n_, chunk_count, plane_args(a0, chunk_count, true), grad, init, s);
+    return;
+  }
   const long cp = static_cast<long>(chunk_count) * plane_;
   int pending = -1;  // slice whose terms are in p_, not yet summed
   for (int seg = nseg_ - 1; seg >= 0; --seg) {

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/qoraholo_hip.h"
+#include "bpm_plane.hpp"
 #include "runtime.hpp"
 #include "tv.hpp"
 
@@ -74,6 +75,7 @@ class BpmModel {
 
  private:
   Args base(int chunk_count) const;
+  BpmPlaneArgs plane_args(int a0, int chunk_count, bool keep) const;
   void ensure_adjoint();
   void set_screen(const float* x, hipStream_t s);
   void forward_pass(int a0, int chunk_count, bool keep, hipStream_t s);

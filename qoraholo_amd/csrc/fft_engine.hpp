@@ -13,6 +13,7 @@
 //   reduce_lines(f, out)  out[l] = sum over k of f(l, k, v), summed in a fixed order
 //   second(inverse)  transform every line again
 //   store1(f) / store2(f)  f(l, m, v) receives element m after the first / second transform
+//   bins(f)          (register engines) mid with the number i of the bin within its thread
 // Lines of a block that lie beyond `lines` are neither read nor written.
 //
 // RegLines: lengths N = N1 N2 of the form 2^a 3^b (32 .. 512) as register-resident four-step
@@ -89,22 +90,41 @@ struct RegLines {
   __device__ explicit RegLines(const LineGeom& g) { init<false>(g, 0); }
   // The grid's first nb blocks run the lines (its later blocks run other work).
   __device__ RegLines(const LineGeom& g, int nb) { init<true>(g, nb); }
+  // The block's own LINES lines, numbered from 0, with LDS of the caller's (kLds and kTw values);
+  // table is exp(-2 pi i t / N). The caller synchronises before the first transform.
+  static constexpr int kBins = N1;  // bins a thread holds after a transform
+  __device__ RegLines(float2* lds, float2* lds_table, const float2* table) : t(lds), tw(lds_table) {
+    fill(table);
+    l = line;
+    valid = true;
+  }
+  // f(i, l, k, v&) for the thread's i-th bin k.
+  template <class F>
+  __device__ void bins(F f) {
+    if (valid && j < N2) {
+#pragma unroll
+      for (int k1 = 0; k1 < N1; ++k1) f(k1, l, N2 * k1 + j, w[k1]);
+    }
+  }
   // The block's line index is formed after the twiddle fill has been issued, so that the fill's
   // loads do not wait for the grid size (a short kernel's start is on its critical path).
   template <bool PART>
   __device__ void init(const LineGeom& g, int nb) {
     t = lds_t();
     tw = lds_tw();
+    fill(g.tw);
+    l = (PART ? xcd_block(nb) : xcd_block()) * LINES + line;
+    valid = l < g.lines;
+  }
+  __device__ __forceinline__ void fill(const float2* table) {
     const int tid = static_cast<int>(threadIdx.x);
     if constexpr (kMatrix) {
-      fill_twiddle_matrix<N2, N1, kTwPitch>(tw, g.tw, 1, tid, BLOCK);
+      fill_twiddle_matrix<N2, N1, kTwPitch>(tw, table, 1, tid, BLOCK);
     } else {
-      for (int i = tid; i < N; i += BLOCK) tw[i] = g.tw[i];
+      for (int i = tid; i < N; i += BLOCK) tw[i] = table[i];
     }
     line = LINE_FAST ? tid % LINES : tid / T;
     j = LINE_FAST ? tid / LINES : tid % T;
-    l = (PART ? xcd_block(nb) : xcd_block()) * LINES + line;
-    valid = l < g.lines;
   }
 
   template <class F>

@@ -131,16 +131,38 @@ struct SplitLines {
   __device__ explicit SplitLines(const LineGeom& g) { init<false>(g, 0); }
   // The grid's first nb blocks run the lines (its later blocks run other work).
   __device__ SplitLines(const LineGeom& g, int nb) { init<true>(g, nb); }
+  // The block's own LINES lines, numbered from 0, with LDS of the caller's (kLds and kTw values);
+  // table is exp(-2 pi i t / N). The caller synchronises before the first transform.
+  static constexpr int kLds = kLine * LINES;
+  static constexpr int kTw = N;
+  static constexpr int kBins = N2;  // bins a thread holds after a transform
+  __device__ SplitLines(float2* lds, float2* lds_table, const float2* table)
+      : t(lds), tw(lds_table) {
+    fill(table);
+    l = line;
+    valid = true;
+  }
   template <bool PART>
   __device__ void init(const LineGeom& g, int nb) {
     t = lds_t();
     tw = lds_tw();
-    const int tid = static_cast<int>(threadIdx.x);
-    for (int i = tid; i < N; i += kBlock) tw[i] = g.tw[i];
-    line = LINE_FAST ? tid % LINES : tid / T;
-    j = LINE_FAST ? tid / LINES : tid % T;
+    fill(g.tw);
     l = (PART ? xcd_block(nb) : xcd_block()) * LINES + line;
     valid = l < g.lines;
+  }
+  __device__ __forceinline__ void fill(const float2* table) {
+    const int tid = static_cast<int>(threadIdx.x);
+    for (int i = tid; i < N; i += kBlock) tw[i] = table[i];
+    line = LINE_FAST ? tid % LINES : tid / T;
+    j = LINE_FAST ? tid / LINES : tid % T;
+  }
+  // f(i, l, k, v&) for the thread's i-th bin k.
+  template <class F>
+  __device__ void bins(F f) {
+    if (valid && j < N1) {
+#pragma unroll
+      for (int i = 0; i < N2; ++i) f(i, l, j + N1 * i, w[i]);
+    }
   }
   __device__ __forceinline__ float2& at(int i) { return LINE_FAST ? t[i * LINES + line] : t[line * kLine + i]; }
 

@@ -116,6 +116,23 @@ def test_two_group_lengths_match_oracle(device, qh, oracle, nz, n):
     assert rel_l2(qh.bpm_vjp(x, r, il, g), oracle.bpm_vjp(x, r, il, GEOM)) < 2e-5
 
 
+@pytest.mark.parametrize("nz,n,count", [(1, 32, 3), (2, 36, 1), (5, 40, 3), (4, 48, 3), (3, 50, 2),
+                                        (3, 54, 2), (4, 60, 3), (5, 64, 270)])
+def test_plane_march_matches_slices_and_oracle(device, qh, oracle, nz, n, count):
+    """Planes that one block marches through all slices: the bits of the launches per slice
+    (which a checkpointed adjoint takes), and the oracle's values."""
+    g, il, ri, x = case(qh, nz, n, count)
+    r = residual_pattern(count, n)
+    got = qh.bpm_vjp(x, r, il, g, checkpoint=0)
+    assert np.array_equal(qh.bpm_vjp(x, r, il, g, checkpoint=0, chunk=1 + count // 2), got)
+    if nz > 1:
+        assert np.array_equal(qh.bpm_vjp(x, r, il, g, checkpoint=1), got)
+    few = il[:3]
+    want = oracle.bpm_forward(x, few, GEOM)
+    assert rel_l2(qh.bpm_forward(ri, few, g) - 1, want - 1) < 5e-5
+    assert rel_l2(qh.bpm_vjp(x, r[:3], few, g), oracle.bpm_vjp(x, r[:3], few, GEOM)) < 2e-5
+
+
 def test_jvp_adjoint_identity_and_difference_on_device(device, qh):
     """<J h, r> = <h, J^T r> with both sides from the device, and J h against a central
     difference of the device forward model (the checks of the reference's
