@@ -11,6 +11,7 @@
 #include "fft.hpp"
 #include "fft4s.hpp"
 #include "fft_args.hpp"
+#include "fft_rows_roundtrip.hpp"
 #include "runtime.hpp"
 
 namespace qh {
@@ -114,10 +115,7 @@ __global__ void __launch_bounds__(kThreads) k_rfft_rows(RowsArgs a) {
     const long at = (r0 + line) * a.x_pitch + 2 * j;
     float u = a.x[at];
     float v = a.x[at + 1];
-    if (a.op.in == RealIn::nonneg) {
-      u = u < 0.0f ? 0.0f : u;
-      v = v < 0.0f ? 0.0f : v;
-    } else if (a.op.in == RealIn::momentum) {
+    if (a.op.in == RealIn::momentum) {
       const float pu = a.x2[at];
       const float pv = a.x2[at + 1];
       u = u + a.op.a * (u - pu);
@@ -130,19 +128,8 @@ __global__ void __launch_bounds__(kThreads) k_rfft_rows(RowsArgs a) {
   for (int e = threadIdx.x; e < nl * (m + 1); e += blockDim.x) {
     const int line = e / (m + 1);
     const int k = e - line * (m + 1);
-    const float2 zk = z[line * m + (k == m ? 0 : k)];
-    const float2 zm = cconj(z[line * m + (k == 0 ? 0 : m - k)]);
-    const float2 ev = {0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y)};
-    const float2 d = {0.5f * (zk.x - zm.x), 0.5f * (zk.y - zm.y)};
-    const float2 od = cmul(tw[k], d);
-    const float2 o = {od.y, -od.x};
-    float2 out;
-    if (k == 0 || k == m) {
-      out = {ev.x + o.x, 0.0f};
-    } else {
-      out = cadd(ev, o);
-    }
-    a.c[(r0 + line) * a.c_pitch + k] = out;
+    a.c[(r0 + line) * a.c_pitch + k] =
+        real_bin(z[line * m + (k == m ? 0 : k)], z[line * m + (k == 0 ? 0 : m - k)], tw[k], k, m);
   }
 }
 
@@ -172,16 +159,8 @@ __global__ void __launch_bounds__(kThreads) k_irfft_rows(RowsArgs a) {
   for (int e = threadIdx.x; e < nl * m; e += blockDim.x) {
     const int line = e / m;
     const int k = e - line * m;
-    float2 xk = b0[line * (m + 1) + k];
-    float2 xm = b0[line * (m + 1) + m - k];
-    if (k == 0) {
-      xk.y = 0.0f;
-      xm.y = 0.0f;
-    }
-    const float2 s = cadd(xk, cconj(xm));
-    const float2 d = csub(xk, cconj(xm));
-    const float2 wd = cmul(cconj(tw[k]), d);
-    b1[line * m + k] = cadd(s, float2{-wd.y, wd.x});
+    const float2* row = b0 + line * (m + 1);
+    b1[line * m + k] = real_pack(row[k], row[m - k], tw[k], k);
   }
   __syncthreads();
   const float2* z = lds_fft(b1, b0, m, 1, nl, a.f, twm, true, false);
@@ -198,6 +177,47 @@ __global__ void __launch_bounds__(kThreads) k_irfft_rows(RowsArgs a) {
     float* px = a.xo + (r0 + line) * a.x_pitch + 2 * j;
     px[0] = u0;
     px[1] = u1;
+  }
+}
+
+// k_irfft_rows, max(., 0) and k_rfft_rows on rows that stay in LDS.
+__global__ void __launch_bounds__(kThreads) k_rows_roundtrip(RowsArgs a) {
+  extern __shared__ float2 smem[];
+  const int n = a.n;
+  const int m = n / 2;
+  float2* tw = smem;
+  float2* twm = tw + n;
+  float2* b0 = twm + m;
+  float2* b1 = b0 + a.rows_per_block * (m + 1);
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const float2 w = a.tw[i];
+    tw[i] = w;
+    if ((i & 1) == 0) twm[i >> 1] = w;
+  }
+  const long r0 = xcd_block() * a.rows_per_block;
+  const int nl = static_cast<int>(min(static_cast<long>(a.rows_per_block), a.rows - r0));
+  for (int e = threadIdx.x; e < nl * (m + 1); e += blockDim.x) {
+    const int line = e / (m + 1);
+    const int k = e - line * (m + 1);
+    b0[e] = a.c[(r0 + line) * a.c_pitch + k];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < nl * m; e += blockDim.x) {
+    const int line = e / m;
+    const int k = e - line * m;
+    const float2* row = b0 + line * (m + 1);
+    b1[line * m + k] = real_pack(row[k], row[m - k], tw[k], k);
+  }
+  __syncthreads();
+  float2* x = lds_fft(b1, b0, m, 1, nl, a.f, twm, true, false);
+  for (int e = threadIdx.x; e < nl * m; e += blockDim.x) x[e] = scale_nonneg(x[e], a.op.a);
+  __syncthreads();
+  const float2* z = lds_fft(x, x == b0 ? b1 : b0, m, 1, nl, a.f, twm, false, false);
+  for (int e = threadIdx.x; e < nl * (m + 1); e += blockDim.x) {
+    const int line = e / (m + 1);
+    const int k = e - line * (m + 1);
+    a.c[(r0 + line) * a.c_pitch + k] =
+        real_bin(z[line * m + (k == m ? 0 : k)], z[line * m + (k == 0 ? 0 : m - k)], tw[k], k, m);
   }
 }
 
@@ -316,6 +336,18 @@ __global__ void __launch_bounds__((Shape4<N1, N2, true>::BLOCK)) k_fft4s_zrt(ZAr
   for (int n2 = 0; n2 < N2; ++n2) {
     v[n2] = (valid && j < N1) ? a.e[static_cast<long>(j + N1 * n2) * a.plane + lb] : float2{0.0f, 0.0f};
   }
+  // The restore operands of the shorter lines are loaded before the transform.
+  constexpr bool kSkip = N1 == 16 && (N2 == 16 || N2 == 24);
+  [[maybe_unused]] float2 d[N1];
+  [[maybe_unused]] std::uint8_t h[N1];
+  if constexpr (!kSkip) {
+    if (valid && j < N2) {
+#pragma unroll
+      for (int k1 = 0; k1 < N1; ++k1) d[k1] = a.a[static_cast<long>(N2 * k1 + j) * a.plane + lb];
+#pragma unroll
+      for (int k1 = 0; k1 < N1; ++k1) h[k1] = a.hits[static_cast<long>(N2 * k1 + j) * a.plane + lb];
+    }
+  }
   __syncthreads();
   fft_4step<N1, N2, S::LINES, true>(v, w, j, line, t, tw, false);
   if (valid && j < N2) {
@@ -323,23 +355,18 @@ __global__ void __launch_bounds__((Shape4<N1, N2, true>::BLOCK)) k_fft4s_zrt(ZAr
     // cleared potential folded: 0.5 (+0 + +0), 0.5 (+0 - +0)), so it need not be read there:
     // most of the half spectrum lies outside the measured caps. The compiler then holds more of
     // the loads in registers; the lengths whose occupancy that leaves unchanged (256, 384) skip.
-    if constexpr (N1 == 16 && (N2 == 16 || N2 == 24)) {
-      std::uint8_t h[N1];
+    if constexpr (kSkip) {
 #pragma unroll
       for (int k1 = 0; k1 < N1; ++k1) h[k1] = a.hits[static_cast<long>(N2 * k1 + j) * a.plane + lb];
 #pragma unroll
       for (int k1 = 0; k1 < N1; ++k1) {
         const long g = static_cast<long>(N2 * k1 + j) * a.plane + lb;
-        const float2 d = h[k1] != 0 ? a.a[g] : float2{0.0f, 0.0f};
-        hermitian_restore(d.x, d.y, h[k1], w[k1].x, w[k1].y);
+        d[k1] = h[k1] != 0 ? a.a[g] : float2{0.0f, 0.0f};
+        hermitian_restore(d[k1].x, d[k1].y, h[k1], w[k1].x, w[k1].y);
       }
     } else {
 #pragma unroll
-      for (int k1 = 0; k1 < N1; ++k1) {
-        const long g = static_cast<long>(N2 * k1 + j) * a.plane + lb;
-        const float2 d = a.a[g];
-        hermitian_restore(d.x, d.y, a.hits[g], w[k1].x, w[k1].y);
-      }
+      for (int k1 = 0; k1 < N1; ++k1) hermitian_restore(d[k1].x, d[k1].y, h[k1], w[k1].x, w[k1].y);
     }
   }
   // Thread j now holds X[j + N2 k1]: the input layout of the transform with the factors swapped.
@@ -384,13 +411,7 @@ __global__ void __launch_bounds__((Shape4<N1, N2>::BLOCK)) k_rfft4s_rows(RowsArg
     q[n2] = (live && momentum) ? *reinterpret_cast<const float2*>(a.x2 + at0 + 2 * N1 * n2)
                                : float2{0.0f, 0.0f};
   }
-  if (a.op.in == RealIn::nonneg) {
-#pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) {
-      v[n2].x = v[n2].x < 0.0f ? 0.0f : v[n2].x;
-      v[n2].y = v[n2].y < 0.0f ? 0.0f : v[n2].y;
-    }
-  } else if (momentum) {
+  if (momentum) {
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) {
       v[n2].x = v[n2].x + a.op.a * (v[n2].x - q[n2].x);
@@ -407,13 +428,8 @@ __global__ void __launch_bounds__((Shape4<N1, N2>::BLOCK)) k_rfft4s_rows(RowsArg
   __syncthreads();
   if (valid) {
     for (int k = j; k <= M; k += S::T) {
-      const float2 zk = zrow[k == M ? 0 : k];
-      const float2 zm = cconj(zrow[k == 0 ? 0 : M - k]);
-      const float2 ev = {0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y)};
-      const float2 d = {0.5f * (zk.x - zm.x), 0.5f * (zk.y - zm.y)};
-      const float2 od = cmul(twn[k], d);
-      const float2 o = {od.y, -od.x};
-      a.c[row * a.c_pitch + k] = (k == 0 || k == M) ? float2{ev.x + o.x, 0.0f} : cadd(ev, o);
+      a.c[row * a.c_pitch + k] =
+          real_bin(zrow[k == M ? 0 : k], zrow[k == 0 ? 0 : M - k], twn[k], k, M);
     }
   }
 }
@@ -455,18 +471,7 @@ __global__ void __launch_bounds__((Shape4<N1, N2>::BLOCK)) k_irfft4s_rows(RowsAr
   for (int n2 = 0; n2 < N2; ++n2) {
     const int k = j + N1 * n2;
     float2 z{0.0f, 0.0f};
-    if (j < N1) {
-      float2 xk = xrow[k];
-      float2 xm = xrow[M - k];
-      if (k == 0) {
-        xk.y = 0.0f;
-        xm.y = 0.0f;
-      }
-      const float2 s = cadd(xk, cconj(xm));
-      const float2 d = csub(xk, cconj(xm));
-      const float2 wd = cmul(cconj(twn[k]), d);
-      z = cadd(s, float2{-wd.y, wd.x});
-    }
+    if (j < N1) z = real_pack(xrow[k], xrow[M - k], twn[k], k);
     v[n2] = z;
   }
   __syncthreads();
@@ -485,6 +490,13 @@ __global__ void __launch_bounds__((Shape4<N1, N2>::BLOCK)) k_irfft4s_rows(RowsAr
     }
   }
 }
+
+template <int N1, int N2>
+struct LaunchRowsRoundtrip {
+  static void run(const RowsArgs& a, hipStream_t s) {
+    launch_rows_roundtrip<RegLines<N1, N2, false, Shape4<N1, N2>::BLOCK>>(a, s);
+  }
+};
 
 // Runs F<N1, N2> for the lengths with a four-step kernel; false for the others.
 template <template <int, int> class F, class... Args>
@@ -649,6 +661,23 @@ void irfft_rows(const float2* in, long in_pitch, float* x, long x_pitch, long ro
   const unsigned grid = static_cast<unsigned>((rows + a.rows_per_block - 1) / a.rows_per_block);
   hipLaunchKernelGGL(k_irfft_rows, dim3(grid), dim3(kThreads), lds, s, a);
   check_launch("irfft_rows");
+}
+
+void rows_roundtrip(float2* e, long pitch, long rows, int n, float scale, hipStream_t s) {
+  require(n % 2 == 0, "rows_roundtrip: even length required");
+  if (rows == 0) return;
+  const int m = n / 2;
+  RealOp op;
+  op.a = scale;
+  RowsArgs a{nullptr, nullptr, nullptr, 0, e, pitch, rows, n, contig_lines_per_block(m),
+             fft_factors(m), fft_twiddles(n), op};
+  if (!with_four_step<LaunchRowsRoundtrip>(m, a, s) && !split_rows_roundtrip(a, s)) {
+    const std::size_t lds =
+        (n + m + static_cast<std::size_t>(a.rows_per_block) * (2 * m + 1)) * sizeof(float2);
+    const unsigned grid = static_cast<unsigned>((rows + a.rows_per_block - 1) / a.rows_per_block);
+    hipLaunchKernelGGL(k_rows_roundtrip, dim3(grid), dim3(kThreads), lds, s, a);
+  }
+  check_launch("rows_roundtrip");
 }
 
 void z_roundtrip_restore(float2* e, const float2* a, const std::uint8_t* hits, int nz, int ny,

@@ -42,8 +42,7 @@ void fft_lines(const float2* in, float2* out, int n, const Lines& l, bool invers
 // Elementwise operation fused into the real input of a row transform.
 enum class RealIn : int {
   plain = 0,     // x
-  nonneg = 1,    // max(x, 0)
-  momentum = 2,  // x + m (x - x2)
+  momentum = 1,  // x + m (x - x2)
 };
 // Elementwise operation fused into the real output of an inverse row transform.
 enum class RealOut : int {
@@ -66,6 +65,9 @@ void rfft_rows(const float* x, const float* x2, long x_pitch, float2* out, long 
 // Half-spectrum rows -> real rows; the imaginary parts of bins 0 and n/2 are ignored.
 void irfft_rows(const float2* in, long in_pitch, float* x, long x_pitch, long rows, int n,
                 const RealOp& op, hipStream_t s);
+
+// Half-spectrum solver step along x, in place: e <- R2C(max(C2R(e) * scale, 0)) of every row.
+void rows_roundtrip(float2* e, long pitch, long rows, int n, float scale, hipStream_t s);
 
 // Half-spectrum solver step along z: forward transform of each z line of e, restore
 // e <- a + (1 - hits / 2) e, inverse transform. e, a, hits are (nz, ny, h) arrays, or `batch`

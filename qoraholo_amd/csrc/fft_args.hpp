@@ -54,6 +54,36 @@ struct ZArgs {
   long vol;  // elements between the volumes of a batch (0: one volume, lines == plane)
 };
 
+// Bin k of a real row of 2m samples from bins k and m - k (k = 0, m: bin 0 twice) of its packed
+// transform: X[k] = (Z[k] + conj Z[m-k]) / 2 - i/2 w (Z[k] - conj Z[m-k]), w = exp(-i pi k / m).
+__device__ __forceinline__ float2 real_bin(float2 zk, float2 zmk, float2 w, int k, int m) {
+  const float2 zm = cconj(zmk);
+  const float2 ev = {0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y)};
+  const float2 d = {0.5f * (zk.x - zm.x), 0.5f * (zk.y - zm.y)};
+  const float2 od = cmul(w, d);
+  const float2 o = {od.y, -od.x};
+  return (k == 0 || k == m) ? float2{ev.x + o.x, 0.0f} : cadd(ev, o);
+}
+
+// The way back: Z[k] = (X[k] + conj X[m-k]) + i conj(w) (X[k] - conj X[m-k]); imaginary parts of
+// X[0] and X[m] are dropped.
+__device__ __forceinline__ float2 real_pack(float2 xk, float2 xm, float2 w, int k) {
+  if (k == 0) {
+    xk.y = 0.0f;
+    xm.y = 0.0f;
+  }
+  const float2 s = cadd(xk, cconj(xm));
+  const float2 d = csub(xk, cconj(xm));
+  const float2 wd = cmul(cconj(w), d);
+  return cadd(s, float2{-wd.y, wd.x});
+}
+
+__device__ __forceinline__ float2 scale_nonneg(float2 v, float scale) {
+  const float x = v.x * scale;
+  const float y = v.y * scale;
+  return {x < 0.0f ? 0.0f : x, y < 0.0f ? 0.0f : y};
+}
+
 // First element of z line l: lines past a plane's belong to the next volumes of the batch.
 __device__ __forceinline__ long z_line_base(const ZArgs& a, long l) {
   return a.vol == 0 ? l : (l / a.plane) * a.vol + l % a.plane;
@@ -62,6 +92,7 @@ __device__ __forceinline__ long z_line_base(const ZArgs& a, long l) {
 // The kernel for a length of split_lines.hpp (lines and z: n; rows: n / 2); false for other lengths.
 bool split_fft_lines(const LinesArgs& a, bool contig, hipStream_t s);
 bool split_rfft_rows(const RowsArgs& a, bool inverse, hipStream_t s);
+bool split_rows_roundtrip(const RowsArgs& a, hipStream_t s);
 bool split_z_roundtrip(const ZArgs& a, hipStream_t s);
 
 }  // namespace qh

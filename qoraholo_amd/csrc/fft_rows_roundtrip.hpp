@@ -1,0 +1,63 @@
+// Row round trip of the Gerchberg-Papoulis step on the register engines: inverse real transform,
+// max(., 0), forward real transform of each half-spectrum row, in one pass.
+//
+// What bounds it: one read and one write of the half spectrum, instead of two of it and of the
+// real volume (MEASURED).
+#pragma once
+
+#include "fft.hpp"
+#include "fft_args.hpp"
+#include "fft_engine.hpp"
+#include "runtime.hpp"
+
+namespace qh {
+
+inline LineGeom row_geometry(int n, long lines) {
+  return LineGeom{fft_twiddles(n), FftFactors{}, n, lines, 0};
+}
+
+template <class E>
+__global__ void __launch_bounds__(E::kBlock) k_rows_roundtrip_reg(RowsArgs a, LineGeom g) {
+  constexpr int M = E::N;
+  __shared__ float2 twn[M + 1];
+  E e(g);
+  for (int i = static_cast<int>(threadIdx.x); i <= M; i += E::kBlock) twn[i] = a.tw[i];
+  // The bins of a row lie in the engine's exchange buffer, which holds at least M + 1 of them.
+  float2* const row = e.t + e.line * (M + 1);
+  constexpr int kPer = (M + E::T) / E::T;
+  float2 c[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int k = e.j + i * E::T;
+    c[i] = (e.valid && k <= M) ? a.c[e.l * a.c_pitch + k] : float2{0.0f, 0.0f};
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int k = e.j + i * E::T;
+    if (k <= M) row[k] = c[i];
+  }
+  __syncthreads();
+  e.load([&](long, int k) { return real_pack(row[k], row[M - k], twn[k], k); });
+  e.first(true);
+  e.mid([&](long, int, float2& v) { v = scale_nonneg(v, a.op.a); });
+  e.second(false);
+  __syncthreads();
+  e.store2([&](long, int k, float2 v) { row[k] = v; });
+  __syncthreads();
+  if (!e.valid) return;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int k = e.j + i * E::T;
+    if (k <= M) {
+      a.c[e.l * a.c_pitch + k] = real_bin(row[k == M ? 0 : k], row[k == 0 ? 0 : M - k], twn[k], k, M);
+    }
+  }
+}
+
+template <class E>
+void launch_rows_roundtrip(const RowsArgs& a, hipStream_t s) {
+  const LineGeom g = row_geometry(E::N, a.rows);
+  hipLaunchKernelGGL(k_rows_roundtrip_reg<E>, dim3(E::grid(g.lines)), dim3(E::kBlock), 0, s, a, g);
+}
+
+}  // namespace qh

@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 #include "fft_args.hpp"
+#include "fft_rows_roundtrip.hpp"
 #include "runtime.hpp"
 #include "split_lines.hpp"
 
@@ -20,13 +21,7 @@ __global__ void __launch_bounds__(E::kBlock) k_split_rfft_rows(RowsArgs a, LineG
   E e(g);
   // All loads of a thread before the first use (the operation is uniform over the grid).
   e.load([&](long l, int i) { return *reinterpret_cast<const float2*>(a.x + l * a.x_pitch + 2 * i); });
-  if (a.op.in == RealIn::nonneg) {
-#pragma unroll
-    for (int i = 0; i < E::N1; ++i) {
-      e.v[i].x = e.v[i].x < 0.0f ? 0.0f : e.v[i].x;
-      e.v[i].y = e.v[i].y < 0.0f ? 0.0f : e.v[i].y;
-    }
-  } else if (a.op.in == RealIn::momentum) {
+  if (a.op.in == RealIn::momentum) {
     float2 q[E::N1];
 #pragma unroll
     for (int i = 0; i < E::N1; ++i) {
@@ -47,13 +42,8 @@ __global__ void __launch_bounds__(E::kBlock) k_split_rfft_rows(RowsArgs a, LineG
   __syncthreads();
   if (!e.valid) return;
   for (int k = e.j; k <= M; k += E::T) {
-    const float2 zk = row[k == M ? 0 : k];
-    const float2 zm = cconj(row[k == 0 ? 0 : M - k]);
-    const float2 ev = {0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y)};
-    const float2 d = {0.5f * (zk.x - zm.x), 0.5f * (zk.y - zm.y)};
-    const float2 od = cmul(a.tw[k], d);
-    const float2 o = {od.y, -od.x};
-    a.c[e.l * a.c_pitch + k] = (k == 0 || k == M) ? float2{ev.x + o.x, 0.0f} : cadd(ev, o);
+    a.c[e.l * a.c_pitch + k] =
+        real_bin(row[k == M ? 0 : k], row[k == 0 ? 0 : M - k], a.tw[k], k, M);
   }
 }
 
@@ -67,16 +57,7 @@ __global__ void __launch_bounds__(E::kBlock) k_split_irfft_rows(RowsArgs a, Line
   }
   __syncthreads();
   e.load([&](long, int k) {
-    float2 xk = row[k];
-    float2 xm = row[M - k];
-    if (k == 0) {
-      xk.y = 0.0f;
-      xm.y = 0.0f;
-    }
-    const float2 s = cadd(xk, cconj(xm));
-    const float2 d = csub(xk, cconj(xm));
-    const float2 wd = cmul(cconj(a.tw[k]), d);
-    return cadd(s, float2{-wd.y, wd.x});
+    return real_pack(row[k], row[M - k], a.tw[k], k);
   });
   e.first(true);
   e.store1([&](long l, int m, float2 v) {
@@ -90,8 +71,6 @@ __global__ void __launch_bounds__(E::kBlock) k_split_irfft_rows(RowsArgs a, Line
   });
 }
 
-LineGeom geometry(int n, long lines) { return LineGeom{fft_twiddles(n), FftFactors{}, n, lines, 0}; }
-
 // About 256 threads a block.
 template <int N>
 using RowEngine = SplitLines<N, false, std::max(1, 256 / SplitLines<N, false, 1>::T)>;
@@ -100,7 +79,7 @@ template <int N>
 struct LaunchRows {
   static void run(const RowsArgs& a, bool inverse, hipStream_t s) {
     using E = RowEngine<N>;
-    const LineGeom g = geometry(N, a.rows);
+    const LineGeom g = row_geometry(N, a.rows);
     if (inverse) {
       hipLaunchKernelGGL(k_split_irfft_rows<E>, dim3(E::grid(g.lines)), dim3(E::kBlock), 0, s, a, g);
     } else {
@@ -109,20 +88,35 @@ struct LaunchRows {
   }
 };
 
-}  // namespace
+template <int N>
+struct LaunchRoundtrip {
+  static void run(const RowsArgs& a, hipStream_t s) { launch_rows_roundtrip<RowEngine<N>>(a, s); }
+};
 
-bool split_rfft_rows(const RowsArgs& a, bool inverse, hipStream_t s) {
-  // Odd halves are row lengths alone: 50, 54, 90, ... have them.
-  switch (a.n / 2) {
+// F<M>::run(args...) for half lengths M with an engine; false for the others. Odd halves are row
+// lengths alone: 50, 54, 90, ... have them.
+template <template <int> class F, class... Args>
+bool with_half(int m, Args&&... args) {
+  switch (m) {
 #define QH_SPLIT_CASE(N) \
   case N:                \
-    LaunchRows<N>::run(a, inverse, s); \
+    F<N>::run(args...);  \
     return true;
     QH_SPLIT_CASE(25) QH_SPLIT_CASE(27) QH_SPLIT_CASE(30) QH_SPLIT_CASE(45) QH_SPLIT_CASE(75)
     QH_SPLIT_CASE(81) QH_SPLIT_CASE(125) QH_SPLIT_CASE(135) QH_SPLIT_CASE(225) QH_SPLIT_CASE(243)
 #undef QH_SPLIT_CASE
-    default: return with_split<LaunchRows>(a.n / 2, a, inverse, s);
+    default: return with_split<F>(m, args...);
   }
+}
+
+}  // namespace
+
+bool split_rfft_rows(const RowsArgs& a, bool inverse, hipStream_t s) {
+  return with_half<LaunchRows>(a.n / 2, a, inverse, s);
+}
+
+bool split_rows_roundtrip(const RowsArgs& a, hipStream_t s) {
+  return with_half<LaunchRoundtrip>(a.n / 2, a, s);
 }
 
 }  // namespace qh

@@ -202,11 +202,9 @@ OdtSolver::OdtSolver(const OdtGrid& g, int count, const OdtConfig& c, int batch)
     a_.resize(nb * half_);
     hits_.resize(nb * half_);
     e_.resize(nb * half_);
-    x_[0].resize(nb * vol_);
     if (tv_) {
-      // FISTA's previous and prox-input iterates (Gerchberg-Papoulis updates x_[0] in place).
-      x_[1].resize(nb * vol_);
-      x_[2].resize(nb * vol_);
+      // FISTA's iterates and the prox input (Gerchberg-Papoulis works on the spectrum alone).
+      for (auto& x : x_) x.resize(nb * vol_);
       tv_state_ = std::make_unique<TvState>(g.nz, g.n, g.n, batch);
       tv_state_->set_exact(false);
       fgp_events_.resize(2 * c.iterations);
@@ -269,6 +267,28 @@ void OdtSolver::map(float2* fields, hipStream_t s, StageClock* clock, int first,
   mark(kNormalize);
 }
 
+// Gerchberg-Papoulis (src/cpu/odt.cpp:76-90) of nb volumes, from their spectra transformed back
+// along z and y (e_): x = max(x, 0), R2C, restore, C2R / N. x itself is formed only in the rows
+// that transform it on, and as the index at the end.
+void OdtSolver::solve_gp(int nb, float* out, hipStream_t s) {
+  const int n = g_.n;
+  const int nz = g_.nz;
+  const int h = n / 2 + 1;
+  const long rows = static_cast<long>(nb) * nz * n;
+  RealOp op;
+  op.out = RealOut::index;
+  op.a = 1.0f / static_cast<float>(vol_);
+  op.nm2 = nm2_;
+  op.inv_k02 = inv_k02_;
+  for (int it = 0; it < c_.iterations; ++it) {
+    rows_roundtrip(e_.get(), h, rows, n, op.a, s);
+    fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), false, 1.0f, 0, s);
+    z_roundtrip_restore(e_.get(), a_.get(), hits_.get(), nz, n, h, s, nb);
+    fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), true, 1.0f, 0, s);
+  }
+  irfft_rows(e_.get(), h, out, n, rows, n, op, s);
+}
+
 void OdtSolver::run_batch(float2* fields, long field_stride, int nb, float* out, hipStream_t s) {
   require(batchable(), "reconstruct: only the solves on half spectra batch");
   require(nb >= 1 && nb <= batch_, "reconstruct: batch beyond the solver's capacity");
@@ -285,6 +305,10 @@ void OdtSolver::run_batch(float2* fields, long field_stride, int nb, float* out,
               1.0f, 0, s);
   }
   fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), true, 1.0f, 0, s);
+  if (!tv_) {
+    solve_gp(nb, out, s);
+    return;
+  }
   RealOp first_op;
   first_op.a = inv;
   irfft_rows(e_.get(), h, x_[0].get(), n, rows, n, first_op, s);
@@ -305,14 +329,6 @@ void OdtSolver::run_batch(float2* fields, long field_stride, int nb, float* out,
     oo.inv_k02 = inv_k02_;
     irfft_rows(e_.get(), h, v, n, rows, n, oo, s);
   };
-  if (!tv_) {
-    for (int it = 0; it < c_.iterations; ++it) {
-      const bool last = it == c_.iterations - 1;
-      gradient_step(x_[0].get(), nullptr, RealIn::nonneg, 0.0f, last ? out : x_[0].get(),
-                    last ? RealOut::index : RealOut::scale);
-    }
-    return;
-  }
   // FISTA-TV as run() does it, every step over the batch; the TV prox takes the batch too.
   tv_state_->reset(s, nb);
   int cur = 0;
@@ -361,6 +377,12 @@ void OdtSolver::run(float2* fields, hipStream_t s, StageClock* clock, int first)
     // x = C2R(a) / N: the first z pass reads a and writes e, so a is kept.
     fft_lines(a_.get(), e_.get(), nz, lines_along(0, nz, n, h, h), true, 1.0f, 0, s);
     fft_lines(e_.get(), e_.get(), n, lines_along(1, nz, n, h, h), true, 1.0f, 0, s);
+    if (!tv_) {
+      solve_gp(1, out, s);
+      mark(kSolve);
+      mark(kFinish);
+      return;
+    }
     RealOp out_op;
     out_op.a = inv;
     irfft_rows(e_.get(), h, x_[0].get(), n, static_cast<long>(nz) * n, n, out_op, s);
@@ -380,17 +402,6 @@ void OdtSolver::run(float2* fields, hipStream_t s, StageClock* clock, int first)
       oo.inv_k02 = inv_k02_;
       irfft_rows(e_.get(), h, v, n, static_cast<long>(nz) * n, n, oo, s);
     };
-    if (!tv_) {
-      // Gerchberg-Papoulis (src/cpu/odt.cpp:76-90): x = max(x, 0), R2C, restore, C2R / N.
-      for (int it = 0; it < c_.iterations; ++it) {
-        const bool last = it == c_.iterations - 1;
-        gradient_step(x_[0].get(), nullptr, RealIn::nonneg, 0.0f, last ? out : x_[0].get(),
-                      last ? RealOut::index : RealOut::scale);
-      }
-      mark(kSolve);
-      mark(kFinish);
-      return;
-    }
     // FISTA-TV (src/cpu/odt.cpp:94-120): y = x + m (x - x_prev) is formed inside the R2C load.
     tv_state_->reset(s);
     int cur = 0;

@@ -141,6 +141,7 @@ class OdtSolver {
   bool timing_fgp() const { return time_fgp_; }
 
  private:
+  void solve_gp(int nb, float* out, hipStream_t s);
   void map(float2* fields, hipStream_t s, StageClock* clock, int first, bool fold, int slot = 0);
   OdtGrid g_;
   int count_;
