@@ -28,6 +28,7 @@
 #include "common.hpp"
 #include "fft.hpp"
 #include "fft_engine.hpp"
+#include "hostio.hpp"
 #include "tv.hpp"
 
 namespace qh {
@@ -52,8 +53,7 @@ BpmTables bpm_tables(int n, int nz, const qh_illumination* il, int count, const 
   t.step.assign(plane * count, float2{0.0f, 0.0f});
   t.last.assign(plane * count, float2{0.0f, 0.0f});
   t.q.assign(plane * count, 0.0f);
-  double q0 = 0;
-  for (int a = 0; a < count; ++a) {
+  parallel_for(count, [&](int a) {
     const double fiy = il[a].fy;
     const double fix = il[a].fx;
     const double fiz = std::sqrt(fm * fm - fiy * fiy - fix * fix);
@@ -77,8 +77,9 @@ BpmTables bpm_tables(int n, int nz, const qh_illumination* il, int count, const 
         t.q[i] = static_cast<float>(q);
       }
     }
-    q0 += static_cast<double>(t.q[a * plane]) * t.q[a * plane];
-  }
+  });
+  double q0 = 0;
+  for (int a = 0; a < count; ++a) q0 += static_cast<double>(t.q[a * plane]) * t.q[a * plane];
   t.lipschitz = static_cast<float>(nz * static_cast<double>(t.phase) * t.phase * q0 / count);
   return t;
 }
@@ -195,8 +196,7 @@ BpmModel::BpmModel(const BpmTables& t, int chunk, int checkpoint)
     // 8 n^2 nz bytes per illumination (384^2 x 384 with 81 illuminations: 37 GB, gradient
     // 184 -> about 130 ms against checkpoints every 16 slices). Otherwise checkpoints keep the
     // passes wide.
-    std::size_t free_bytes = 0, total_bytes = 0;
-    check(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo");
+    const std::size_t free_bytes = device_bytes_free();
     const std::size_t keep_all = static_cast<std::size_t>(plane_) *
                                  (5 * sizeof(float2) + sizeof(float) + sizeof(float2) * nz_);
     const std::size_t angles = static_cast<std::size_t>(chunk > 0 ? std::min(chunk, count_) : count_);
@@ -207,8 +207,7 @@ BpmModel::BpmModel(const BpmTables& t, int chunk, int checkpoint)
   if (chunk == 0) {
     // As many illuminations per pass as keep the adjoint's buffers within half the free
     // device memory (src/cuda/bpm.cu:225-232 sizes its chunks the same way).
-    std::size_t free_bytes = 0, total_bytes = 0;
-    check(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo");
+    const std::size_t free_bytes = device_bytes_free();
     const std::size_t per_angle =
         static_cast<std::size_t>(plane_) * (5 * sizeof(float2) + sizeof(float) +
                                             2 * sizeof(float2) * (nseg_ - 1) +

@@ -16,6 +16,7 @@
 
 #include "../../include/qoraholo_hip.h"
 #include "bpm.hpp"
+#include "call_memory.hpp"
 #include "fft.hpp"
 #include "pipeline.hpp"
 #include "hostio.hpp"
@@ -125,6 +126,7 @@ std::vector<std::array<float, 5>> device_sidebands(const float* holo, int count,
   if (dc_exclusion <= 0) dc_exclusion = static_cast<float>(n) / 8.0f;
   require_device();
   const hipStream_t s = call_stream();
+  const CallMemory memory(s);
   const std::size_t plane = static_cast<std::size_t>(n) * n;
   DeviceBuffer<float> dh(plane * count);
   DeviceBuffer<float2> half(static_cast<std::size_t>(count) * n * (n / 2 + 1));
@@ -259,6 +261,7 @@ namespace {
 void bpm_forward_call(const BpmTables& t, const float* x, const qh_bpm_options* o, qh_c64* out) {
   require_device();
   const hipStream_t s = call_stream();
+  const CallMemory memory(s);
   BpmModel m(t, o->chunk, o->checkpoint);
   const std::size_t vol = static_cast<std::size_t>(t.nz) * t.n * t.n;
   DeviceBuffer<float> dx(vol);
@@ -273,6 +276,7 @@ void bpm_vjp_call(const BpmTables& t, const float* x, const qh_c64* r, const qh_
                   float* grad) {
   require_device();
   const hipStream_t s = call_stream();
+  const CallMemory memory(s);
   BpmModel m(t, o->chunk, o->checkpoint);
   const std::size_t vol = static_cast<std::size_t>(t.nz) * t.n * t.n;
   DeviceBuffer<float> dx(vol), dg(vol);
@@ -288,6 +292,7 @@ void bpm_jvp_call(const BpmTables& t, const float* x, const float* h, const qh_b
                   qh_c64* out) {
   require_device();
   const hipStream_t s = call_stream();
+  const CallMemory memory(s);
   BpmModel m(t, o->chunk, o->checkpoint);
   const std::size_t vol = static_cast<std::size_t>(t.nz) * t.n * t.n;
   DeviceBuffer<float> dx(vol), dh(vol);
@@ -313,6 +318,7 @@ void bpm_reconstruct_call(const BpmTables& t, const qh_c64* fields, float* x,
                           double* loss) {
   require_device();
   const hipStream_t s = call_stream();
+  const CallMemory memory(s);
   BpmModel m(t, o->chunk, o->checkpoint);
   const std::size_t vol = static_cast<std::size_t>(t.nz) * t.n * t.n;
   DeviceBuffer<float> dx(vol);
@@ -437,6 +443,7 @@ int qh_hip_extract_fields(const float* holograms, int count, int n, const qh_cro
     require_fft(plan->out, "extract_fields");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const int m = plan->out;
     const std::size_t image = static_cast<std::size_t>(n) * n;
     DeviceBuffer<float> holo(count * image);
@@ -461,6 +468,7 @@ int qh_hip_unwrap(const float* wrapped, int nz, int ny, int nx, float* out) {
     require_fft(nx, "unwrap");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const std::size_t total = static_cast<std::size_t>(nz) * ny * nx;
     DeviceBuffer<float> psi(total);
     DeviceBuffer<float> phi(total);
@@ -481,6 +489,7 @@ int qh_hip_rytov(const qh_c64* ratio, int nz, int ny, int nx, qh_c64* out) {
     require_fft(nx, "rytov");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const std::size_t total = static_cast<std::size_t>(nz) * ny * nx;
     DeviceBuffer<float2> r(total);
     DeviceBuffer<float> psi(total);
@@ -507,33 +516,41 @@ int qh_hip_reconstruct(const qh_c64* fields, int count, int n, const qh_illumina
     require_device();
     const auto t0 = std::chrono::steady_clock::now();
     std::size_t free_before = 0, free_after = 0, total_mem = 0;
-    check(hipMemGetInfo(&free_before, &total_mem), "hipMemGetInfo");
     const hipStream_t s = call_stream();
+    // The timings report the memory that the call allocates.
+    std::unique_ptr<CallMemory> memory;
+    if (timings) {
+      check(hipMemGetInfo(&free_before, &total_mem), "hipMemGetInfo");
+    } else {
+      memory = std::make_unique<CallMemory>(s);
+    }
     OdtSolver solver(g, count, config_from(*options, *geometry));
     std::vector<float> il(2 * static_cast<std::size_t>(count));
     for (int a = 0; a < count; ++a) {
       il[2 * a] = illum[a].fy;
       il[2 * a + 1] = illum[a].fx;
     }
-    solver.set_illuminations(il.data());
+    solver.set_illuminations(il.data(), s);
     solver.time_fgp(timings != nullptr);
     const std::size_t plane = static_cast<std::size_t>(n) * n;
     DeviceBuffer<float2> f(plane * count);
     for (int len : {n, n / 2, g.nz}) fft_twiddles(len);
-    check(hipMemGetInfo(&free_after, &total_mem), "hipMemGetInfo");
+    if (timings) check(hipMemGetInfo(&free_after, &total_mem), "hipMemGetInfo");
     const double setup =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    StageClock clock(kOdtMarks + 3);
+    StageClock clock(timings ? kOdtMarks + 3 : 0);
     const int start = kOdtMarks, uploaded = kOdtMarks + 1, downloaded = kOdtMarks + 2;
-    clock.mark(start, s);
+    if (timings) clock.mark(start, s);
     upload(f.get(), fields, f.bytes(), s);
-    clock.mark(uploaded, s);
-    solver.run(f.get(), s, &clock, 0);
+    if (timings) clock.mark(uploaded, s);
+    solver.run(f.get(), s, timings ? &clock : nullptr, 0);
     const std::size_t vol = plane * g.nz;
     unsigned long long nfilled = 0;
-    download(ri, solver.index(), vol * sizeof(float), s);
-    download(&nfilled, solver.filled_device(), sizeof nfilled, s);
-    clock.mark(downloaded, s);
+    Downloads results;
+    results.add(&nfilled, solver.filled_device(), sizeof nfilled, s, true);
+    results.add(ri, solver.index(), vol * sizeof(float), s, vol * sizeof(float) <= (4u << 20));
+    results.finish();
+    if (timings) clock.mark(downloaded, s);
     check(hipStreamSynchronize(s), "reconstruct");
     if (filled) *filled = static_cast<double>(nfilled) / static_cast<double>(vol);
     if (timings) {
@@ -565,6 +582,7 @@ int qh_hip_map_kspace(const qh_c64* fields, int count, int n, const qh_illuminat
     require_fft(n, "map_kspace");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const OdtGrid g{grid->n, grid->nz, grid->df, grid->dfz, grid->fm2, grid->fna2, grid->gain};
     OdtSolver solver(g, count, OdtConfig{});
     std::vector<float> il(2 * static_cast<std::size_t>(count));
@@ -804,6 +822,7 @@ int qh_hip_fft_c2c(qh_c64* data, int d0, int d1, int d2, unsigned axes, int forw
     if (axes & 4u) require_fft(d2, "fft");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     DeviceBuffer<float2> d(static_cast<std::size_t>(d0) * d1 * d2);
     upload(d.get(), data, d.bytes(), s);
     fft3(d.get(), d0, d1, d2, axes, forward == 0, scale, s);
@@ -820,6 +839,7 @@ int qh_hip_rfft3(const float* x, int nz, int ny, int nx, qh_c64* out) {
     require_fft(nx / 2, "rfft3");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const std::size_t vol = static_cast<std::size_t>(nz) * ny * nx;
     const std::size_t half = static_cast<std::size_t>(nz) * ny * (nx / 2 + 1);
     DeviceBuffer<float> dx(vol);
@@ -839,6 +859,7 @@ int qh_hip_irfft3(const qh_c64* in, int nz, int ny, int nx, float scale, float* 
     require_fft(nx / 2, "irfft3");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const std::size_t vol = static_cast<std::size_t>(nz) * ny * nx;
     const std::size_t half = static_cast<std::size_t>(nz) * ny * (nx / 2 + 1);
     DeviceBuffer<float> dx(vol);
@@ -1061,6 +1082,7 @@ int qh_hip_tv_prox(const float* b, int nz, int ny, int nx, float lambda, int inn
             "tv_prox: bad arguments");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const std::size_t vol = static_cast<std::size_t>(nz) * ny * nx;
     DeviceBuffer<float> db(vol);
     DeviceBuffer<float> dx(vol);
@@ -1082,6 +1104,7 @@ int qh_hip_tv_prox_batch(const float* b, int batch, int nz, int ny, int nx, floa
             "tv_prox_batch: bad arguments (batch 1 to 65535)");
     require_device();
     const hipStream_t s = call_stream();
+    const CallMemory memory(s);
     const std::size_t vol = static_cast<std::size_t>(nz) * ny * nx;
     DeviceBuffer<float> db(vol * batch);
     DeviceBuffer<float> dx(vol * batch);

@@ -21,7 +21,8 @@ namespace {
 constexpr int kThreads = 256;
 
 std::mutex g_tables_mu;
-// (device, kind, n) -> table; kind 0: FFT twiddles, 1: DCT twiddles.
+// (device, kind, n) -> table; kind 0: FFT twiddles, 1: DCT twiddles, 2: the n floats of
+// neumann_terms.
 std::map<std::tuple<int, int, int>, DeviceBuffer<float2>> g_tables;
 
 const float2* table(int kind, int n) {
@@ -31,12 +32,17 @@ const float2* table(int kind, int n) {
   auto& buf = g_tables[{dev, kind, n}];
   if (buf.size() == 0) {
     std::vector<float2> h(n);
-    for (int t = 0; t < n; ++t) {
+    for (int t = 0; kind == 2 && t < n; ++t) {
+      const float v = 2.0f * cosf(kPi * static_cast<float>(t) / static_cast<float>(n));
+      (t % 2 == 0 ? h[t / 2].x : h[t / 2].y) = v;
+    }
+    for (int t = 0; kind != 2 && t < n; ++t) {
       // kind 0: exp(-2 pi i t / n); kind 1: exp(-i pi t / (2 n)). Evaluated in double.
       const double a = kind == 0 ? 2.0 * M_PI * t / static_cast<double>(n)
                                  : M_PI * t / (2.0 * static_cast<double>(n));
       h[t] = {static_cast<float>(std::cos(a)), static_cast<float>(-std::sin(a))};
     }
+    const CallMemory::Outside kept;
     DeviceBuffer<float2> d(n);
     check(hipMemcpy(d.get(), h.data(), n * sizeof(float2), hipMemcpyHostToDevice), "upload twiddles");
     buf = std::move(d);
@@ -592,6 +598,7 @@ bool fft_supported(int n) {
 
 const float2* fft_twiddles(int n) { return table(0, n); }
 const float2* dct_twiddles(int n) { return table(1, n); }
+const float* neumann_terms(int n) { return reinterpret_cast<const float*>(table(2, n)); }
 
 Lines lines_along(int axis, int d0, int d1, int d2, long pitch) {
   switch (axis) {

@@ -19,6 +19,8 @@ bool fft_supported(int n);
 const float2* fft_twiddles(int n);
 // Device table exp(-i pi k / (2 n)), k in [0, n): the DCT-II twiddles (Makhoul).
 const float2* dct_twiddles(int n);
+// Device table 2 cos(pi k / n) in float, k in [0, n): the terms of the Neumann eigenvalues.
+const float* neumann_terms(int n);
 
 // Lines of a 3D array: line l starts at (l / inner) * outer + (l % inner) * inner_stride and
 // its elements are `stride` apart. Units are elements (float2 for complex arrays).

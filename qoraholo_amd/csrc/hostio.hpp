@@ -1,13 +1,15 @@
 // Host ingest and egress. Copies between pageable host memory (numpy arrays, callers' buffers)
-// and the device go through two pinned staging buffers of the calling thread, chunk by chunk:
+// and the device go through rings of pinned staging slots of the calling thread, chunk by chunk:
 // the host side of each chunk is spread over a small pool of copy threads and overlaps the DMA
-// of the neighbouring chunk. A plain hipMemcpy from pageable memory stages through the
-// runtime's own buffers with one host thread and reaches about a fifth of the PCIe rate.
+// of the neighbouring chunks. A plain hipMemcpy from pageable memory stages through the
+// runtime's own buffers with one host thread: 25.7 MB take 754 us in and 1560 us out that way,
+// 1 MB 46 and 65 us; the DMA alone 476 and 27 us, the host copy 190 and 14 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <deque>
 #include <functional>
 
 namespace qh {
@@ -30,5 +32,23 @@ void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 // Pageable host dst <- device src, after the work already queued on s. Returns with dst
 // complete.
 void download(void* dst, const void* src, std::size_t bytes, hipStream_t s);
+
+// Several downloads whose DMAs queue up behind each other: add() returns with the copies queued
+// as far as the staging slots go, finish() with every dst complete.
+class Downloads {
+ public:
+  // alone: nothing is queued behind it on s before finish().
+  void add(void* dst, const void* src, std::size_t bytes, hipStream_t s, bool alone = false);
+  void finish();
+
+ private:
+  void retire();
+  struct Part {
+    int slot;
+    char* dst;
+    std::size_t bytes;
+  };
+  std::deque<Part> parts_;
+};
 
 }  // namespace qh

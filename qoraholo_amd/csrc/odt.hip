@@ -12,6 +12,7 @@
 
 #include "common.hpp"
 #include "fft.hpp"
+#include "hostio.hpp"
 #include "runtime.hpp"
 #include "stages.hpp"
 
@@ -214,13 +215,17 @@ OdtSolver::OdtSolver(const OdtGrid& g, int count, const OdtConfig& c, int batch)
   }
 }
 
-void OdtSolver::set_illuminations(const float* illum) {
+void OdtSolver::set_illuminations(const float* illum, hipStream_t s) {
   std::vector<float4> il(count_);
   for (int a = 0; a < count_; ++a) {
     const float fy = illum[2 * a];
     const float fx = illum[2 * a + 1];
     // fiz on the host in float, as the reference evaluates it (src/cpu/odt.cpp:141-144).
     il[a] = {fy, fx, std::sqrt(g_.fm2 - fy * fy - fx * fx), 0.0f};
+  }
+  if (s) {
+    upload(illum_.get(), il.data(), illum_.bytes(), s);
+    return;
   }
   check(hipMemcpy(illum_.get(), il.data(), count_ * sizeof(float4), hipMemcpyHostToDevice),
         "upload illuminations");

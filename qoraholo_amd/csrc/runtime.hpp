@@ -9,6 +9,8 @@
 #include <utility>
 #include <vector>
 
+#include "call_memory.hpp"
+
 namespace qh {
 
 // Errors the C-ABI maps to status codes: invalid arguments, misuse, out-of-memory and device
@@ -51,23 +53,31 @@ class DeviceBuffer {
   ~DeviceBuffer() { release(); }
   DeviceBuffer(const DeviceBuffer&) = delete;
   DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-  DeviceBuffer(DeviceBuffer&& o) noexcept : p_(std::exchange(o.p_, nullptr)), n_(std::exchange(o.n_, 0)) {}
+  DeviceBuffer(DeviceBuffer&& o) noexcept
+      : p_(std::exchange(o.p_, nullptr)), n_(std::exchange(o.n_, 0)), call_(o.call_) {}
   DeviceBuffer& operator=(DeviceBuffer&& o) noexcept {
     if (this != &o) {
       release();
       p_ = std::exchange(o.p_, nullptr);
       n_ = std::exchange(o.n_, 0);
+      call_ = o.call_;
     }
     return *this;
   }
+  // From the calling thread's CallMemory where there is one.
   void resize(std::size_t n) {
     release();
     if (n == 0) return;
-    check(hipMalloc(reinterpret_cast<void**>(&p_), n * sizeof(T)), "hipMalloc");
+    call_ = CallMemory::current();
+    p_ = static_cast<T*>(call_ ? call_->take(n * sizeof(T)) : device_alloc(n * sizeof(T)));
     n_ = n;
   }
   void release() {
-    if (p_) (void)hipFree(p_);
+    if (p_ && call_) {
+      call_->give(p_);
+    } else if (p_) {
+      (void)hipFree(p_);
+    }
     p_ = nullptr;
     n_ = 0;
   }
@@ -78,6 +88,7 @@ class DeviceBuffer {
  private:
   T* p_ = nullptr;
   std::size_t n_ = 0;
+  CallMemory* call_ = nullptr;
 };
 
 template <class T>
@@ -96,6 +107,11 @@ class PinnedBuffer {
   PinnedBuffer(const PinnedBuffer&) = delete;
   PinnedBuffer& operator=(const PinnedBuffer&) = delete;
   PinnedBuffer(PinnedBuffer&& o) noexcept : p_(std::exchange(o.p_, nullptr)), n_(std::exchange(o.n_, 0)) {}
+  PinnedBuffer& operator=(PinnedBuffer&& o) noexcept {
+    std::swap(p_, o.p_);
+    std::swap(n_, o.n_);
+    return *this;
+  }
   T* get() const { return p_; }
   std::size_t size() const { return n_; }
 
@@ -121,6 +137,10 @@ class Stream {
 class Event {
  public:
   Event() { check(hipEventCreate(&e_), "hipEventCreate"); }
+  explicit Event(bool timing) {
+    check(hipEventCreateWithFlags(&e_, timing ? hipEventDefault : hipEventDisableTiming),
+          "hipEventCreate");
+  }
   ~Event() {
     if (e_) (void)hipEventDestroy(e_);
   }

@@ -14,12 +14,6 @@ double ms_between(std::chrono::steady_clock::time_point a, std::chrono::steady_c
   return std::chrono::duration<double, std::milli>(b - a).count();
 }
 
-std::size_t free_device_bytes() {
-  std::size_t free_b = 0, total_b = 0;
-  check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-  return free_b;
-}
-
 // A reconstruction slot: a Pipeline of the geometry with its background fields set.
 class ReconWorker final : public SlotWorker {
  public:
@@ -86,7 +80,7 @@ class BpmWorker final : public SlotWorker {
 
 Server::Server(std::size_t budget_bytes, int max_slots)
     : budget_(budget_bytes), max_slots_(std::max(1, max_slots)) {
-  if (budget_ == 0) budget_ = free_device_bytes() / 10 * 9;
+  if (budget_ == 0) budget_ = device_bytes_free() / 10 * 9;
   dispatcher_ = std::thread([this] { dispatch_loop(); });
 }
 
@@ -157,11 +151,11 @@ int Server::add_kind(Kind kind, std::function<std::unique_ptr<SlotWorker>()> mak
   // lock), so the change in free memory is this slot's alone; running slots allocate nothing.
   std::lock_guard<std::mutex> lock(mu_);
   check(hipDeviceSynchronize(), "Server::add_geometry");
-  const std::size_t before = free_device_bytes();
+  const std::size_t before = device_bytes_free();
   auto slot = std::make_unique<Slot>();
   slot->pipeline = g->make();
   check(hipDeviceSynchronize(), "Server::add_geometry");
-  const std::size_t after = free_device_bytes();
+  const std::size_t after = device_bytes_free();
   slot->bytes = before > after ? before - after : 0;
   g->slot_bytes = std::max<std::size_t>(slot->bytes, 1);
   if (slot->bytes > budget_) {

@@ -74,8 +74,8 @@ class Unwrapper {
   DeviceBuffer<float> phi_;
   DeviceBuffer<double2> partial_;
   DeviceBuffer<float2> shift_;  // per image: congruence constant c, border shift
-  DeviceBuffer<float> eig_y_;   // 2 cos(pi k / ny), host-evaluated in float
-  DeviceBuffer<float> eig_x_;
+  const float* eig_y_;  // neumann_terms(ny), (nx)
+  const float* eig_x_;
 };
 
 // ---- ODT solver (src/cpu/odt.cpp:124-242 on the device) ----
@@ -108,7 +108,8 @@ class OdtSolver {
  public:
   // `batch`: the requests run_batch takes at once (the solves on half spectra).
   OdtSolver(const OdtGrid& g, int count, const OdtConfig& c, int batch = 1);
-  void set_illuminations(const float* illum_host);  // (count, 2) fy, fx
+  // (count, 2) fy, fx; on s, or at once without a stream.
+  void set_illuminations(const float* illum_host, hipStream_t s = nullptr);
   // fields: (count, n, n) complex on the device, overwritten by their spectra. The index volume
   // (nz, n, n) is left in index(). Marks go to clock[first + OdtMark] when given.
   void run(float2* fields, hipStream_t s, StageClock* clock = nullptr, int first = 0);

@@ -251,22 +251,14 @@ Unwrapper::Unwrapper(int count, int ny, int nx)
       nblk_(std::max(1, std::min(64, static_cast<int>((static_cast<long>(ny) * nx + 255) / 256)))),
       phi_(static_cast<std::size_t>(count) * ny * nx),
       partial_(static_cast<std::size_t>(count) * nblk_),
-      shift_(count),
-      eig_y_(ny),
-      eig_x_(nx) {
+      shift_(count) {
   require(fft_supported(ny) && fft_supported(nx), "unwrap: image sides must factor into 2, 3, 5");
-  const auto upload = [](DeviceBuffer<float>& d, int n) {
-    // 2 cos(pi k / n) in float on the host, the terms of the Neumann eigenvalue.
-    std::vector<float> h(n);
-    for (int k = 0; k < n; ++k) h[k] = 2.0f * cosf(kPi * static_cast<float>(k) / static_cast<float>(n));
-    check(hipMemcpy(d.get(), h.data(), n * sizeof(float), hipMemcpyHostToDevice), "upload eigenvalues");
-  };
-  upload(eig_y_, ny);
-  upload(eig_x_, nx);
+  eig_y_ = neumann_terms(ny);
+  eig_x_ = neumann_terms(nx);
 }
 
 std::size_t Unwrapper::bytes() const {
-  return phi_.bytes() + partial_.bytes() + shift_.bytes() + eig_y_.bytes() + eig_x_.bytes();
+  return phi_.bytes() + partial_.bytes() + shift_.bytes();
 }
 
 void Unwrapper::solve(const float* psi, hipStream_t s, bool border, int images) {
@@ -281,7 +273,7 @@ void Unwrapper::solve(const float* psi, hipStream_t s, bool border, int images) 
     if (!forward) {
       ColArgs c{phi, static_cast<long>(images) * nx_, ny_, nx_,
                 std::max(1, std::min(16, 2048 / ny_)), fft_factors(ny_), fft_twiddles(ny_),
-                dct_twiddles(ny_), eig_y_.get(), eig_x_.get(), 1.0f / static_cast<float>(ny_)};
+                dct_twiddles(ny_), eig_y_, eig_x_, 1.0f / static_cast<float>(ny_)};
       const std::size_t lds = (2 * ny_ + 2 * static_cast<std::size_t>(c.lines_per_block) * ny_) * sizeof(float2);
       const unsigned grid = static_cast<unsigned>((c.lines + c.lines_per_block - 1) / c.lines_per_block);
       hipLaunchKernelGGL(k_dct_cols_poisson, dim3(grid), dim3(kThreads), lds, s, c);

@@ -196,6 +196,40 @@ def test_reconstruction_matches_oracle(device, oracle, qh, rytov_fields, case):
     assert filled == want_filled
 
 
+@pytest.mark.parametrize("n,nz", [(30, 20), (50, 32), (64, 48), (72, 36), (96, 40), (192, 16)])
+def test_gp_row_roundtrip_matches_oracle(device, oracle, qh, n, nz):
+    """Gerchberg-Papoulis over the engines of its row round trip: row halves 15 (LDS), 25 and 36
+    (two groups), 32, 48 and 96 (four-step), with z sides of other engines."""
+    illum = qh.circular_scan(5, 0.9, geom(qh))
+    rng = np.random.default_rng(n)
+    fields = (rng.standard_normal((5, n, n)) + 1j * rng.standard_normal((5, n, n))).astype(np.complex64)
+    fields *= np.float32(0.1)
+    got, filled = qh.reconstruct(fields, illum, geom(qh), nz=nz, iterations=3, return_filled=True)
+    want, want_filled = oracle.reconstruct(fields, illum, GEOM, nz=nz, iterations=3)
+    assert contrast_error(got, want, GEOM[1]) < TOL
+    assert filled == want_filled
+
+
+def test_calls_of_several_threads_share_device_memory(device, qh):
+    """Calls of different sizes from several threads at once, which hand each other the blocks of
+    their buffers: the results of the same calls one after another."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    def call(i):
+        n = (32, 48, 64, 80)[i % 4]
+        rng = np.random.default_rng(i)
+        f = (rng.standard_normal((5, n, n)) + 1j * rng.standard_normal((5, n, n))).astype(np.complex64)
+        illum = qh.circular_scan(5, 0.9, geom(qh))
+        kind = dict(solver="tv", iterations=2) if i % 3 == 0 else dict(iterations=i % 3)
+        return qh.reconstruct(f * np.float32(0.1), illum, geom(qh), **kind), qh.rytov(f)
+
+    want = [call(i) for i in range(24)]
+    with ThreadPoolExecutor(4) as ex:
+        got = list(ex.map(call, range(24)))
+    for (a, b), (c, d) in zip(got, want):
+        assert np.array_equal(a, c) and np.array_equal(b, d)
+
+
 def test_tv_at_256_matches_oracle(device, oracle, qh):
     # The full-size transforms (256-point z lines, 128-point packed rows) and FGP strips.
     g = (0.532, 1.337, 1.2, 0.11)
