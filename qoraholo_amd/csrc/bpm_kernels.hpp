@@ -93,6 +93,21 @@ constexpr int mid_group() {
   }
 }
 
+// Whether the adjoint rows load their operands, from memory that no recent kernel has touched
+// (the envelopes), before the first transform: up to 192, where that fits the registers of four
+// waves per SIMD (adjoint of 96 slices of 128^2 with 9 illuminations 1370 -> 1275 us, with 25 1535
+// -> 1466 us; 64 of 192^2 with 49 2055 -> 2000 us; of 256^2 with 49 3077 -> 3139 us). The other
+// kernels, whose operands the caches hold, gained nothing by it or lost waves to the registers
+// (columns at 256: 2317 -> 2715 us).
+template <class E>
+constexpr bool operands_ahead() {
+  if constexpr (requires { E::kMatrix; }) {  // the four-step engine
+    return E::N <= 192;
+  } else {
+    return false;
+  }
+}
+
 // Rows (line l = b n + y, element i at l n + i): inverse x transform of T, envelope, screen,
 // forward x transform. in == null: the unit envelope of the first slice. out == null: store the
 // envelope only.
@@ -307,21 +322,28 @@ k_bpm_rows_adj(Args a) {
   E e(a.g);
   const int n = a.g.n;
   e.load([&](long l, int i) { return a.in[l * n + i]; });
-  e.first(true);
   // Operands of a bin: the screen t and the stored envelope w.
   struct Ops {
     float2 t, w;
   };
-  e.template mid_loaded<mid_group<E>()>(
-      [&](long l, int k) {
-        return Ops{a.screen[line_in_plane<E>(l, n) * n + k], a.w[l * n + k]};
-      },
-      [&](long l, int k, float2& v, Ops o) {
-        const float2 b = cscale(v, a.inv);
-        const float2 tw = cmul(o.t, o.w);
-        a.p[l * n + k] = a.phase * (tw.x * b.y - tw.y * b.x);
-        v = cmul(cconj(o.t), b);
-      });
+  const auto operands = [&](long l, int k) {
+    return Ops{a.screen[line_in_plane<E>(l, n) * n + k], a.w[l * n + k]};
+  };
+  const auto term = [&](long l, int k, float2& v, Ops o) {
+    const float2 b = cscale(v, a.inv);
+    const float2 tw = cmul(o.t, o.w);
+    a.p[l * n + k] = a.phase * (tw.x * b.y - tw.y * b.x);
+    v = cmul(cconj(o.t), b);
+  };
+  if constexpr (operands_ahead<E>()) {
+    Ops o[E::kBins];
+    e.bins([&](int i, long l, int k, float2&) { o[i] = operands(l, k); });
+    e.first(true);
+    e.bins([&](int i, long l, int k, float2& v) { term(l, k, v, o[i]); });
+  } else {
+    e.first(true);
+    e.template mid_loaded<mid_group<E>()>(operands, term);
+  }
   if (a.out == nullptr) return;
   e.second(false);
   e.store2([&](long l, int m, float2 v) { a.out[l * n + m] = v; });

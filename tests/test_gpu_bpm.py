@@ -116,6 +116,14 @@ def test_two_group_lengths_match_oracle(device, qh, oracle, nz, n):
     assert rel_l2(qh.bpm_vjp(x, r, il, g), oracle.bpm_vjp(x, r, il, GEOM)) < 2e-5
 
 
+@pytest.mark.parametrize("nz,n", [(3, 96), (2, 128), (2, 192), (2, 256)])
+def test_adjoint_rows_match_oracle(device, qh, oracle, nz, n):
+    """The adjoint's rows on both sides of the length up to which they load operands ahead."""
+    g, il, _, x = case(qh, nz, n, count=3)
+    r = residual_pattern(3, n)
+    assert rel_l2(qh.bpm_vjp(x, r, il, g), oracle.bpm_vjp(x, r, il, GEOM)) < 2e-5
+
+
 @pytest.mark.parametrize("nz,n,count", [(1, 32, 3), (2, 36, 1), (5, 40, 3), (4, 48, 3), (3, 50, 2),
                                         (3, 54, 2), (4, 60, 3), (5, 64, 270)])
 def test_plane_march_matches_slices_and_oracle(device, qh, oracle, nz, n, count):
