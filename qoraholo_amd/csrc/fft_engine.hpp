@@ -92,7 +92,9 @@ struct RegLines {
   __device__ RegLines(const LineGeom& g, int nb) { init<true>(g, nb); }
   // The block's own LINES lines, numbered from 0, with LDS of the caller's (kLds and kTw values);
   // table is exp(-2 pi i t / N). The caller synchronises before the first transform.
-  static constexpr int kBins = N1;  // bins a thread holds after a transform
+  static constexpr int kBins = N1;     // bins a thread holds after a transform
+  static constexpr int kSamples = N2;  // samples j + kFirst u of threads j < kFirst before it (v)
+  static constexpr int kFirst = N1;
   __device__ RegLines(float2* lds, float2* lds_table, const float2* table) : t(lds), tw(lds_table) {
     fill(table);
     l = line;

@@ -12,6 +12,7 @@
 
 #include "common.hpp"
 #include "fft.hpp"
+#include "gp_plane.hpp"
 #include "hostio.hpp"
 #include "runtime.hpp"
 #include "stages.hpp"
@@ -273,25 +274,29 @@ void OdtSolver::map(float2* fields, hipStream_t s, StageClock* clock, int first,
 }
 
 // Gerchberg-Papoulis (src/cpu/odt.cpp:76-90) of nb volumes, from their spectra transformed back
-// along z and y (e_): x = max(x, 0), R2C, restore, C2R / N. x itself is formed only in the rows
-// that transform it on, and as the index at the end.
+// along z (e_): x = max(x, 0), R2C, restore, C2R / N. x itself is formed only within the rows or
+// planes that transform it on, and as the index at the end.
 void OdtSolver::solve_gp(int nb, float* out, hipStream_t s) {
   const int n = g_.n;
   const int nz = g_.nz;
   const int h = n / 2 + 1;
-  const long rows = static_cast<long>(nb) * nz * n;
+  const long planes = static_cast<long>(nb) * nz;
+  const Lines columns = lines_along(1, nb * nz, n, h, h);
   RealOp op;
   op.out = RealOut::index;
   op.a = 1.0f / static_cast<float>(vol_);
   op.nm2 = nm2_;
   op.inv_k02 = inv_k02_;
   for (int it = 0; it < c_.iterations; ++it) {
-    rows_roundtrip(e_.get(), h, rows, n, op.a, s);
-    fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), false, 1.0f, 0, s);
+    if (!gp_plane(e_.get(), planes, n, op.a, s)) {
+      fft_lines(e_.get(), e_.get(), n, columns, true, 1.0f, 0, s);
+      rows_roundtrip(e_.get(), h, planes * n, n, op.a, s);
+      fft_lines(e_.get(), e_.get(), n, columns, false, 1.0f, 0, s);
+    }
     z_roundtrip_restore(e_.get(), a_.get(), hits_.get(), nz, n, h, s, nb);
-    fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), true, 1.0f, 0, s);
   }
-  irfft_rows(e_.get(), h, out, n, rows, n, op, s);
+  fft_lines(e_.get(), e_.get(), n, columns, true, 1.0f, 0, s);
+  irfft_rows(e_.get(), h, out, n, planes * n, n, op, s);
 }
 
 void OdtSolver::run_batch(float2* fields, long field_stride, int nb, float* out, hipStream_t s) {
@@ -309,11 +314,11 @@ void OdtSolver::run_batch(float2* fields, long field_stride, int nb, float* out,
     fft_lines(a_.get() + b * half_, e_.get() + b * half_, nz, lines_along(0, nz, n, h, h), true,
               1.0f, 0, s);
   }
-  fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), true, 1.0f, 0, s);
   if (!tv_) {
     solve_gp(nb, out, s);
     return;
   }
+  fft_lines(e_.get(), e_.get(), n, lines_along(1, nb * nz, n, h, h), true, 1.0f, 0, s);
   RealOp first_op;
   first_op.a = inv;
   irfft_rows(e_.get(), h, x_[0].get(), n, rows, n, first_op, s);
@@ -381,13 +386,13 @@ void OdtSolver::run(float2* fields, hipStream_t s, StageClock* clock, int first)
   if (real_) {
     // x = C2R(a) / N: the first z pass reads a and writes e, so a is kept.
     fft_lines(a_.get(), e_.get(), nz, lines_along(0, nz, n, h, h), true, 1.0f, 0, s);
-    fft_lines(e_.get(), e_.get(), n, lines_along(1, nz, n, h, h), true, 1.0f, 0, s);
     if (!tv_) {
       solve_gp(1, out, s);
       mark(kSolve);
       mark(kFinish);
       return;
     }
+    fft_lines(e_.get(), e_.get(), n, lines_along(1, nz, n, h, h), true, 1.0f, 0, s);
     RealOp out_op;
     out_op.a = inv;
     irfft_rows(e_.get(), h, x_[0].get(), n, static_cast<long>(nz) * n, n, out_op, s);

@@ -210,6 +210,20 @@ def test_gp_row_roundtrip_matches_oracle(device, oracle, qh, n, nz):
     assert filled == want_filled
 
 
+@pytest.mark.parametrize("n,nz", [(64, 2), (96, 6), (128, 4), (128, 30)])
+def test_gp_planes_match_oracle(device, oracle, qh, n, nz):
+    """Gerchberg-Papoulis on planes that one block takes through both axes: white fields, so that
+    the bins 0 and n/2 of a row, which share a column, carry as much as the others."""
+    illum = qh.circular_scan(4, 0.9, geom(qh))
+    rng = np.random.default_rng(n + nz)
+    fields = (rng.standard_normal((4, n, n)) + 1j * rng.standard_normal((4, n, n))).astype(np.complex64)
+    fields *= np.float32(0.1)
+    for iterations in (1, 4):
+        got = qh.reconstruct(fields, illum, geom(qh), nz=nz, iterations=iterations)
+        want, _ = oracle.reconstruct(fields, illum, GEOM, nz=nz, iterations=iterations)
+        assert contrast_error(got, want, GEOM[1]) < TOL
+
+
 def test_calls_of_several_threads_share_device_memory(device, qh):
     """Calls of different sizes from several threads at once, which hand each other the blocks of
     their buffers: the results of the same calls one after another."""
