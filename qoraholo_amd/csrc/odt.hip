@@ -12,6 +12,7 @@
 
 #include "common.hpp"
 #include "fft.hpp"
+#include "gp_complex.hpp"
 #include "gp_plane.hpp"
 #include "hostio.hpp"
 #include "runtime.hpp"
@@ -156,26 +157,6 @@ __global__ void k_fold_half(const float2* potential, const std::uint16_t* counts
   if (threadIdx.x == 0 && block_count > 0) atomicAdd(filled, static_cast<unsigned long long>(block_count));
 }
 
-__global__ void k_gp_nonneg(float2* p, long total) {
-  const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const float re = p[i].x;
-  p[i] = {re < 0.0f ? 0.0f : re, 0.0f};
-}
-
-__global__ void k_gp_restore_measured(float2* p, const float2* measured,
-                                      const std::uint16_t* counts, long total) {
-  const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  if (counts[i] > 0) p[i] = measured[i];
-}
-
-__global__ void k_index_complex(const float2* p, float* ri, long total, float nm2, float inv_k02) {
-  const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  ri[i] = index_from_potential(p[i].x, p[i].y, nm2, inv_k02);
-}
-
 }  // namespace
 
 OdtSolver::OdtSolver(const OdtGrid& g, int count, const OdtConfig& c, int batch)
@@ -212,7 +193,7 @@ OdtSolver::OdtSolver(const OdtGrid& g, int count, const OdtConfig& c, int batch)
       fgp_events_.resize(2 * c.iterations);
     }
   } else if (c.iterations > 0) {
-    measured_.resize(vol_);
+    work_.resize(vol_);
   }
 }
 
@@ -233,7 +214,7 @@ void OdtSolver::set_illuminations(const float* illum, hipStream_t s) {
 }
 
 std::size_t OdtSolver::bytes() const {
-  std::size_t b = illum_.bytes() + potential_.bytes() + counts_.bytes() + measured_.bytes() +
+  std::size_t b = illum_.bytes() + potential_.bytes() + counts_.bytes() + work_.bytes() +
                   a_.bytes() + hits_.bytes() + e_.bytes() + ri_.bytes() + filled_.bytes();
   for (const auto& x : x_) b += x.bytes();
   if (tv_state_) b += tv_state_->bytes();
@@ -441,28 +422,23 @@ void OdtSolver::run(float2* fields, hipStream_t s, StageClock* clock, int first)
     return;
   }
 
-  // Complex path (src/cpu/odt.cpp:208-241): plain inverse, or GP on full spectra.
-  float2* p = potential_.get();
-  if (c_.iterations > 0) {
-    check(hipMemcpyAsync(measured_.get(), p, vol_ * sizeof(float2), hipMemcpyDeviceToDevice, s),
-          "copy measured");
-    fft3(p, nz, n, n, 0b111u, true, inv, s);
-    for (int it = 0; it < c_.iterations; ++it) {
-      hipLaunchKernelGGL(k_gp_nonneg, dim3(blocks_for(vol_)), dim3(256), 0, s, p, vol_);
-      check_launch("gp_nonneg");
-      fft3(p, nz, n, n, 0b111u, false, 1.0f, s);
-      hipLaunchKernelGGL(k_gp_restore_measured, dim3(blocks_for(vol_)), dim3(256), 0, s, p,
-                         measured_.get(), counts_.get(), vol_);
-      check_launch("gp_restore");
-      fft3(p, nz, n, n, 0b111u, true, inv, s);
-    }
-  } else {
-    fft3(p, nz, n, n, 0b111u, true, inv, s);
+  // Complex path (src/cpu/odt.cpp:208-241): plain inverse, or GP on full spectra. The volume goes
+  // through the axes as z, y, x inverse and x, y, z forward, so that what happens between two
+  // transforms along one axis takes one pass with them.
+  float2* const measured = potential_.get();
+  float2* const p = c_.iterations > 0 ? work_.get() : measured;
+  const long rows = static_cast<long>(nz) * n;
+  const Lines columns = lines_along(1, nz, n, n, n);
+  fft_lines(measured, p, nz, lines_along(0, nz, n, n, n), true, 1.0f, 0, s);
+  fft_lines(p, p, n, columns, true, 1.0f, 0, s);
+  for (int it = 0; it < c_.iterations; ++it) {
+    gp_complex_rows(p, rows, n, inv, s);
+    fft_lines(p, p, n, columns, false, 1.0f, 0, s);
+    gp_complex_z(p, measured, counts_.get(), nz, static_cast<long>(n) * n, s);
+    fft_lines(p, p, n, columns, true, 1.0f, 0, s);
   }
   mark(kSolve);
-  hipLaunchKernelGGL(k_index_complex, dim3(blocks_for(vol_)), dim3(256), 0, s, p, out, vol_,
-                     nm2_, inv_k02_);
-  check_launch("index");
+  gp_complex_index(p, rows, n, inv, nm2_, inv_k02_, out, s);
   mark(kFinish);
 }
 

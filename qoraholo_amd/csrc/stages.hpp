@@ -156,7 +156,7 @@ class OdtSolver {
   DeviceBuffer<float4> illum_;
   DeviceBuffer<float2> potential_;
   DeviceBuffer<std::uint16_t> counts_;
-  DeviceBuffer<float2> measured_;
+  DeviceBuffer<float2> work_;  // the volume of a solve on full spectra
   DeviceBuffer<float2> a_;
   DeviceBuffer<std::uint8_t> hits_;
   DeviceBuffer<float2> e_;

@@ -224,6 +224,22 @@ def test_gp_planes_match_oracle(device, oracle, qh, n, nz):
         assert contrast_error(got, want, GEOM[1]) < TOL
 
 
+@pytest.mark.parametrize("n,nz", [(30, 24), (50, 36), (64, 50), (96, 32), (128, 6), (256, 4)])
+def test_gp_complex_passes_match_oracle(device, oracle, qh, n, nz):
+    """Gerchberg-Papoulis on full spectra, and the plain inverse, over the engines of their x and
+    z passes: lengths in LDS (30, 24, 6), of two groups and four-step."""
+    illum = qh.circular_scan(4, 0.9, geom(qh))
+    rng = np.random.default_rng(n + nz)
+    fields = (rng.standard_normal((4, n, n)) + 1j * rng.standard_normal((4, n, n))).astype(np.complex64)
+    fields *= np.float32(0.1)
+    for iterations in (0, 1, 3):
+        kind = dict(nz=nz, iterations=iterations, gp_transform="c2c")
+        got, filled = qh.reconstruct(fields, illum, geom(qh), return_filled=True, **kind)
+        want, want_filled = oracle.reconstruct(fields, illum, GEOM, **kind)
+        assert contrast_error(got, want, GEOM[1]) < TOL
+        assert filled == want_filled
+
+
 def test_calls_of_several_threads_share_device_memory(device, qh):
     """Calls of different sizes from several threads at once, which hand each other the blocks of
     their buffers: the results of the same calls one after another."""
