@@ -6,11 +6,13 @@
 // of exp(i (psi - phi)) in double, reduced in a fixed order. The DCTs follow Makhoul: reorder,
 // complex FFT, twiddle exp(-i pi k / 2n); the inverse is V_k = exp(i pi k / 2n)(X_k - i X_{n-k}),
 // inverse FFT, reorder back, / n (reference src/cpu/fft.cpp:101-133, src/cpu/unwrap.cpp:11-82).
+// Sides with a register engine take dct.hip; the kernels here serve the others.
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
 #include "common.hpp"
+#include "dct.hpp"
 #include "fft.hpp"
 #include "runtime.hpp"
 #include "stages.hpp"
@@ -24,15 +26,10 @@ constexpr int kThreads = 256;
 __global__ void k_divergence(const float* psi, float* rho, long total, int ny, int nx) {
   const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= total) return;
-  const int x = static_cast<int>(i % nx);
-  const int y = static_cast<int>((i / nx) % ny);
-  const float p = psi[i];
-  float r = 0.0f;
-  if (x + 1 < nx) r += wrap_phase(psi[i + 1] - p);
-  if (x > 0) r -= wrap_phase(p - psi[i - 1]);
-  if (y + 1 < ny) r += wrap_phase(psi[i + nx] - p);
-  if (y > 0) r -= wrap_phase(p - psi[i - nx]);
-  rho[i] = r;
+  const long plane = static_cast<long>(ny) * nx;
+  const long image = i / plane;
+  const int at = static_cast<int>(i - image * plane);
+  rho[i] = wrapped_divergence(psi + image * plane, at / nx, at % nx, ny, nx);
 }
 
 struct DctArgs {
@@ -266,9 +263,14 @@ void Unwrapper::solve(const float* psi, hipStream_t s, bool border, int images) 
   const long plane = static_cast<long>(ny_) * nx_;
   const long total = plane * images;
   float* phi = phi_.get();
-  hipLaunchKernelGGL(k_divergence, dim3(blocks_for(total)), dim3(256), 0, s, psi, phi, total, ny_, nx_);
-  check_launch("divergence");
-  for (int pass = 0; pass < 2; ++pass) {
+  const bool engines = dct_supported(ny_, nx_);
+  if (engines) {
+    dct_poisson(psi, phi, images, ny_, nx_, s);
+  } else {
+    hipLaunchKernelGGL(k_divergence, dim3(blocks_for(total)), dim3(256), 0, s, psi, phi, total, ny_, nx_);
+    check_launch("divergence");
+  }
+  for (int pass = 0; !engines && pass < 2; ++pass) {
     const bool forward = pass == 0;
     if (!forward) {
       ColArgs c{phi, static_cast<long>(images) * nx_, ny_, nx_,

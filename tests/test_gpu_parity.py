@@ -139,6 +139,21 @@ def test_unwrap_matches_oracle_and_known_answer(device, oracle, qh):
         assert np.max(np.abs(got[z] - truth[z] - offset)) < 2e-3
 
 
+@pytest.mark.parametrize("ny,nx", [(32, 50), (64, 36), (48, 512), (250, 32), (384, 60), (30, 64),
+                                   (96, 6)])
+def test_unwrap_engines_match_oracle(device, oracle, qh, ny, nx):
+    """Cosine transforms over the engines of both axes (four-step, two groups), and images with a
+    side that has none (30, 6). Phases beyond pi with noise, three images of which each is its own."""
+    from test_oracle import wrap
+
+    rng = np.random.default_rng(ny + nx)
+    psi = wrap(smooth_phase(3, ny, nx) + rng.standard_normal((3, ny, nx)).astype(np.float32) * np.float32(0.3))
+    psi = psi.astype(np.float32)
+    got = qh.unwrap(psi)
+    assert rel_l2(got, oracle.unwrap(psi)) < TOL
+    assert np.array_equal(qh.unwrap(psi[1]), got[1])
+
+
 def test_rytov_matches_oracle(device, oracle, qh):
     illum = qh.circular_scan(5, 0.8, geom(qh))
     ratio = qh.forward_fields(cell(qh), illum, geom(qh), 64)
