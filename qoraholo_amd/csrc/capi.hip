@@ -547,8 +547,12 @@ int qh_hip_reconstruct(const qh_c64* fields, int count, int n, const qh_illumina
     const std::size_t vol = plane * g.nz;
     unsigned long long nfilled = 0;
     Downloads results;
-    results.add(&nfilled, solver.filled_device(), sizeof nfilled, s, true);
-    results.add(ri, solver.index(), vol * sizeof(float), s, vol * sizeof(float) <= (4u << 20));
+    // The count goes ahead of a small volume (behind it, 15 us of a 64^3 call), and behind a large
+    // one, whose host copies would wait for all of it with the stream.
+    const bool small = vol * sizeof(float) <= kStagingSlot;
+    if (small) results.add(&nfilled, solver.filled_device(), sizeof nfilled, s, true);
+    results.add(ri, solver.index(), vol * sizeof(float), s, small);
+    if (!small) results.add(&nfilled, solver.filled_device(), sizeof nfilled, s, true);
     results.finish();
     if (timings) clock.mark(downloaded, s);
     check(hipStreamSynchronize(s), "reconstruct");

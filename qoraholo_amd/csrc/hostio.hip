@@ -21,9 +21,7 @@ namespace qh {
 
 namespace {
 
-// Staging slot: a copy into it takes about half the time of its DMA (37 of 82 us), so that the
-// first chunk's copy is all the DMA waits for and the last chunk's all that follows it.
-constexpr std::size_t kChunk = std::size_t(4) << 20;
+constexpr std::size_t kChunk = kStagingSlot;
 constexpr int kSlots = 4;  // of each direction
 // Host copies are split into parts of at least this size.
 constexpr std::size_t kMinPart = std::size_t(1) << 19;
