@@ -62,10 +62,12 @@ __device__ __forceinline__ float primal_value(float b, float lambda, float rz, f
 
 // 1 / max(1, sqrt(norm2)) from the hardware's reciprocal square root y. EXACT: g = n y corrected
 // once is the nearest float to sqrt(n), and y corrected once against that the nearest to its
-// reciprocal: the bits of 1.0f / sqrtf(n) for every float n from 1 up to the last 128 before
-// overflow (all of them compared on the device), in 8 operations instead of the compiler's 25. The
-// bounds keep the limits of the division: 0 for an infinite norm, whose residuals are NaN; a NaN
-// norm counts as below one, as in norm2 > 1 ? ... : 1.
+// reciprocal, except where every mantissa bit of the root is set: there the correction ends on the
+// tie between two floats and rounds to the even one, and the nearest is the next (the one exception
+// to a reciprocal corrected with fused operations). With it these are the bits of 1.0f / sqrtf(n)
+// for every float n from 1 to infinity (all 2^30 compared on the device), in 11 operations instead
+// of the compiler's 25. The bounds keep the limits of the division: 0 for an infinite norm, whose
+// residuals are NaN; a NaN norm counts as below one, as in norm2 > 1 ? ... : 1.
 template <bool EXACT>
 __device__ __forceinline__ float ball_scale(float norm2) {
   const float n = fmaxf(norm2, 1.0f);
@@ -74,7 +76,9 @@ __device__ __forceinline__ float ball_scale(float norm2) {
   const float h = 0.5f * y;
   if constexpr (EXACT) {
     const float root = fmaf(fmaf(-g, g, n), h, g);
-    return fmaxf(fmaf(fmaf(-root, y, 1.0f), y, y), 0.0f);
+    const float even = fmaf(fmaf(-root, y, 1.0f), y, y);
+    const unsigned up = __builtin_amdgcn_frexp_mantf(root) == 0x1.fffffep-1f ? 1u : 0u;
+    return fmaxf(__uint_as_float(__float_as_uint(even) + up), 0.0f);
   } else {
     return fmaf(h, fmaxf(fmaf(-g, y, 1.0f), -1.0f), y);
   }

@@ -348,6 +348,64 @@ def test_tv_tile_edges_match_oracle(device, oracle, shape, inner):
     assert np.max(np.abs(got - want)) < 1e-6
 
 
+def test_tv_projection_rounds_as_division_and_root(device):
+    """One step on volumes whose dual norms fall on every octave from 1 up, against the same
+    float32 operations in numpy: the projection's scale has the bits of 1 / sqrt(n). lambda is the
+    float nearest to 1/12, so that the step is 1 and a dual component a difference of b. Random
+    differences cover n; cells of one high voxel cover the n whose root has every mantissa bit set
+    (0x407ffffe and 0x407fffff, and those 4^k larger), which a reciprocal corrected once misses."""
+    from qoraholo_amd import _native
+
+    lam = np.float32(1) / np.float32(12)
+    assert np.float32(12) * lam == 1
+    one = np.float32(1)
+    rng = np.random.default_rng(2)
+
+    def norm2(qz, qy, qx):
+        return (qz * qz + qy * qy) + qx * qx
+
+    # Cells: a high voxel h and its upper neighbours h - q, on a grid on which differences are exact.
+    grid = np.float32(2.0**-22)
+    h = (rng.integers(5 << 20, 11 << 19, 1 << 18) * grid).astype(np.float32)
+    low = (rng.integers(0, 1 << 20, (2, h.size)) * grid).astype(np.float32)
+    qz, qy = h - low[0], h - low[1]
+    qx = (np.round(np.sqrt(4.0 - qz.astype(np.float64)**2 - qy.astype(np.float64)**2) / grid)
+          * grid).astype(np.float32)
+    bits = norm2(qz, qy, qx).view(np.uint32)
+    hit = np.flatnonzero(((bits == 0x407ffffe) | (bits == 0x407fffff)) & (qx > 0) & (qx <= h))
+    assert hit.size >= 256
+    hit = hit[:256]
+    cells = np.zeros((32, 32, 64), np.float32)
+    for i, c in enumerate(hit):
+        z, y, x = 4 * (i // 128), 4 * (i // 16 % 8), 4 * (i % 16)
+        cells[z, y, x], cells[z + 1, y, x] = h[c], low[0][c]
+        cells[z, y + 1, x], cells[z, y, x + 1] = low[1][c], h[c] - qx[c]
+    spread = rng.random((64, 96, 128), np.float32) * np.float32(3)
+
+    for b in [cells * np.float32(2.0**k) for k in (0, 1, 5, 20)] + [spread, spread * np.float32(7)]:
+        q = [np.zeros_like(b) for _ in range(3)]
+        for a in range(3):
+            lo = tuple(slice(None, -1) if i == a else slice(None) for i in range(3))
+            hi = tuple(slice(1, None) if i == a else slice(None) for i in range(3))
+            q[a][lo] = b[lo] - b[hi]
+        n = norm2(*q)
+        scale = one / np.sqrt(np.maximum(n, one))
+        s = np.zeros_like(b)
+        for a in range(3):
+            p = q[a] * scale
+            s = s + p
+            below = np.zeros_like(p)
+            hi = tuple(slice(1, None) if i == a else slice(None) for i in range(3))
+            lo = tuple(slice(None, -1) if i == a else slice(None) for i in range(3))
+            below[hi] = p[lo]
+            s = s - below
+        want = np.maximum(b - lam * s, np.float32(0))
+        got = np.empty_like(b)
+        _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *b.shape, float(lam), 1, 1,
+                                                   _native.ptr(got)))
+        assert np.array_equal(got, want)
+
+
 def test_tv_infinities_and_nans_stay_where_the_oracle_has_them(device, oracle):
     """One voxel that is infinite or NaN, inside and on the faces and tile seams."""
     from qoraholo_amd import _native
