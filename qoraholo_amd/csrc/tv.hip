@@ -176,7 +176,7 @@ struct StepArgs {
 // The march, unrolled over T + 1 planes: the r and p a stage hands on take the registers of the
 // plane it has done with, so the register sets rotate through the T stages and the loads, and after
 // T + 1 planes are back in place (a rolled loop moves 7 floats a point and stage back by v_mov). The
-// unrolled planes are numbered U = 0 .. T.
+// unrolled planes are numbered U = 0 .. T; without steps two planes, for two exchange buffers.
 //
 // QUADS: ny is a multiple of 4. Otherwise the rows of the last quad are stored column by column
 // like the others (h floats a column for h rows), which takes accesses of 4 bytes. FIRST: the first
@@ -187,11 +187,19 @@ struct StepMarch {
   static constexpr int HL = T + (FINAL ? 1 : 0);  // planes in front of a chunk
   static constexpr int S = T + (FINAL ? 1 : 0);   // stages that exchange rows
   static constexpr int TS = T > 0 ? T : 1;
-  static constexpr int kUnroll = T + 1;
+  static constexpr int kUnroll = T > 0 ? T + 1 : 2;
   // Row exchange buffers: planes that follow one another use different ones, as a wave may be one
-  // barrier ahead of its neighbours, never a plane.
+  // barrier ahead of its neighbours, never a plane. With a single buffer a wave could overwrite the
+  // row of a plane that the next wave has yet to read.
   static constexpr int kBufs = kUnroll % 2 == 0 ? 2 : 3;
   static constexpr int buf(int u) { return u == kUnroll - 1 && kBufs == 3 ? 2 : u % 2; }
+  static constexpr bool bufs_alternate() {
+    for (int u = 0; u < kUnroll; ++u) {
+      if (buf(u) == buf((u + 1) % kUnroll) || buf(u) >= kBufs) return false;
+    }
+    return true;
+  }
+  static_assert(bufs_alternate(), "consecutive planes exchange rows through different buffers");
 
   struct Lds {
     float ry[kBufs][S][NW + 1][64];  // r_y of the last row of wave w at w + 1; zero at 0

@@ -348,6 +348,22 @@ def test_tv_tile_edges_match_oracle(device, oracle, shape, inner):
     assert np.max(np.abs(got - want)) < 1e-6
 
 
+@pytest.mark.parametrize("shape", [(64, 32, 64), (90, 120, 60), (33, 62, 130)])
+def test_tv_output_pass_equals_oracle(device, oracle, shape):
+    """Single steps, whose output is formed by a pass without steps: many planes in a chunk, rows of
+    every quad exchanged on each. The device rounds every operation in the order of the oracle's
+    float expressions, so the bits are the same."""
+    from qoraholo_amd import _native
+
+    rng = np.random.default_rng(shape[0])
+    b = (rng.standard_normal(shape) * 0.3 + 0.3).astype(np.float32)
+    for inner in (1, 2):
+        got = np.empty_like(b)
+        _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *shape, 0.05, inner, 0,
+                                                   _native.ptr(got)))
+        assert np.array_equal(got, oracle.tv_prox(b, 0.05, inner)), inner
+
+
 def test_tv_projection_rounds_as_division_and_root(device):
     """One step on volumes whose dual norms fall on every octave from 1 up, against the same
     float32 operations in numpy: the projection's scale has the bits of 1 / sqrt(n). lambda is the
