@@ -53,9 +53,10 @@ def fgp_traffic(kernel: str):
 
 
 def fgp_passes(inner: int) -> list[int]:
-    """FGP steps of each pass of one prox call: as few passes of at most four steps as it needs, of
-    nearly equal length, the longer ones first (TvState::prox)."""
-    passes = (inner + 3) // 4
+    """FGP steps of each pass of one prox call: as few passes of at most four steps as it needs, with
+    the output, which the last pass forms, as one step more; of nearly equal length, the longer ones
+    first (TvState::prox)."""
+    passes = inner // 4 + 1
     return [inner // passes + (k < inner % passes) for k in range(passes)]
 
 

@@ -141,7 +141,9 @@ struct Window {
 // a wave's quad (a row of r_y and one of z per wave and stage through LDS), z neighbours from the
 // registers of the plane before. Every step makes one column, row and plane on either side of the
 // tile invalid, so tiles overlap by kHalo columns and rows on each side and a chunk of planes
-// starts T planes early. FINAL adds a stage that forms max(b - lambda L(p_{k+T}), 0).
+// starts T planes early. FINAL adds a stage that forms max(b - lambda L(p_{k+T}), 0), which takes
+// one more of each on the lower side (L reads p at x - 1, y - 1 and z - 1): T + FINAL of them lie
+// within kHalo, so that a pass with the output has at most three steps.
 //
 // Eight waves of up to 256 registers make one block per CU. Twelve waves (48 rows a tile) leave 168
 // registers, which T = 3 just fits and the other passes spill: 209 against 220 us for a 256^3 pass
@@ -185,6 +187,7 @@ template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
 struct StepMarch {
   static constexpr int NW = kWaves;
   static constexpr int HL = T + (FINAL ? 1 : 0);  // planes in front of a chunk
+  static_assert(HL <= kHalo, "the points a tile writes are out of reach of its edges");
   static constexpr int S = T + (FINAL ? 1 : 0);   // stages that exchange rows
   static constexpr int TS = T > 0 ? T : 1;
   static constexpr int kUnroll = T > 0 ? T + 1 : 2;
@@ -505,7 +508,7 @@ void launch_steps(StepArgs a, hipStream_t s, int batch, bool exact) {
 template <int T>
 void launch_steps_of(const StepArgs& a, hipStream_t s, int batch, bool exact) {
   if (a.x) {
-    launch_steps<T, false, true>(a, s, batch, exact);
+    if constexpr (T < kMaxSteps) launch_steps<T, false, true>(a, s, batch, exact);
   } else if (T >= 3 && a.first) {
     // The first of several passes, of 3 or 4 steps: without p_{k-1} at all (256^3: 193 against 200 us
     // for 3 steps, 219 against 240 us for 4; 384^3: 529 against 550 us for 3).
@@ -515,9 +518,10 @@ void launch_steps_of(const StepArgs& a, hipStream_t s, int batch, bool exact) {
   }
 }
 
-// `steps` FGP steps in one pass; with x set, the prox output after them (0 steps: of p_k). Only
-// whole quads have kernels with fused arithmetic.
+// `steps` FGP steps in one pass (up to kMaxSteps); with x set, the prox output after them (up to
+// kMaxSteps - 1; 0 steps: of p_k). Only whole quads have kernels with fused arithmetic.
 void fgp_steps(int steps, const StepArgs& a, hipStream_t s, int batch, bool exact) {
+  require(steps + (a.x ? 1 : 0) <= kMaxSteps, "tv: too many steps in a pass");
   switch (steps) {
     case 0: launch_steps<0, true, true>(a, s, batch, exact); break;
     case 1: launch_steps_of<1>(a, s, batch, exact); break;
@@ -564,8 +568,8 @@ void TvState::reset(hipStream_t s, int batch) {
 std::size_t TvState::bytes() const { return owned_.bytes(); }
 
 // tv_prox of the reference (src/cpu/tv.cpp:7-44): r <- p, `inner` FGP steps, out = primal(p).
-// The steps go in as few passes as they need, the last of which forms the output. The dual
-// iterates rotate through four buffers: a pass of T steps reads p_k and p_{k-1} (r is formed
+// The steps go in as few passes as they need, the last of which forms the output and counts it as
+// a step more. The dual iterates rotate through four buffers: a pass of T steps reads p_k and p_{k-1} (r is formed
 // inside it) and writes p_{k+T-1} and p_{k+T} to buffers nobody reads in that pass; the last pass
 // skips p_{k+T-1}, which the next call does not read (its first step uses r = p). The prox leaves
 // p in buffer cur_ for the next call.
@@ -578,7 +582,9 @@ void TvState::prox(const float* b, float* out, float lambda, int inner, hipStrea
   const bool apart = out + vol_ * batch_ <= b || b + vol_ * batch_ <= out;
   const bool joined = fused_ && apart && inner > 0;
   const int most = fused_ ? kMaxSteps : 1;
-  const int passes = (inner + most - 1) / most;
+  // The output takes the place of a step: passes = ceil((inner + 1) / most), whose nearly equal
+  // shares of the steps leave the last at most `most` - 1.
+  const int passes = (inner + (joined ? 1 : 0) + most - 1) / most;
   StepArgs a{};
   a.b = b;
   a.vol = vol_;

@@ -348,6 +348,42 @@ def test_tv_tile_edges_match_oracle(device, oracle, shape, inner):
     assert np.max(np.abs(got - want)) < 1e-6
 
 
+@pytest.mark.parametrize("shape", [(7, 60, 130), (40, 49, 113), (12, 96, 64), (9, 32, 200)])
+@pytest.mark.parametrize("inner", [3, 4, 7, 8, 12, 15, 16, 20])
+def test_tv_output_at_tile_seams_equals_oracle(device, oracle, shape, inner):
+    """The output on the first columns and rows of a tile, which reads the dual one point further
+    down than the steps of its pass: step counts around the multiples of four, several tiles in x,
+    y or both, duals far from zero at the seams. The device rounds every operation in the order of
+    the oracle's float expressions, so the bits are the same, in passes and in single steps."""
+    from qoraholo_amd import _native
+
+    rng = np.random.default_rng(shape[2] + inner)
+    b = (rng.standard_normal(shape) * 0.3 + 0.3).astype(np.float32)
+    want = oracle.tv_prox(b, 0.1, inner)
+    for fused in (1, 0):
+        got = np.empty_like(b)
+        _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *shape, 0.1, inner, fused,
+                                                   _native.ptr(got)))
+        assert np.array_equal(got, want), fused
+
+
+@pytest.mark.parametrize("inner", [4, 8])
+def test_tv_warm_dual_at_tile_seams_matches_oracle(device, oracle, qh, inner):
+    """FISTA-TV over three iterations, whose later proxes start from the dual of the one before, on
+    planes of several tiles. The contrast is at most 0.03 here and its float arithmetic (transforms,
+    steps) rounds at 1e-6 of it, so that each side is within the rounding of an index between 1 and
+    2, two units of 2^-23, and they differ by at most four: an output formed from a wrong dual at the
+    seams is 5 (inner 4) and 15 times (inner 8) further off."""
+    illum = qh.circular_scan(6, 0.9, geom(qh))
+    rng = np.random.default_rng(inner)
+    fields = (rng.standard_normal((6, 72, 72)) + 1j * rng.standard_normal((6, 72, 72))).astype(np.complex64)
+    kind = dict(nz=24, iterations=3, solver="tv", tv_inner=inner, tv_weight=0.1)
+    got = qh.reconstruct(fields, illum, geom(qh), **kind)
+    want, _ = oracle.reconstruct(fields, illum, GEOM, **kind)
+    assert np.max(np.abs(want - GEOM[1])) < 0.03
+    assert np.max(np.abs(got.astype(np.float64) - want)) < 4 * 2.0**-23
+
+
 @pytest.mark.parametrize("shape", [(64, 32, 64), (90, 120, 60), (33, 62, 130)])
 def test_tv_output_pass_equals_oracle(device, oracle, shape):
     """Single steps, whose output is formed by a pass without steps: many planes in a chunk, rows of
