@@ -52,24 +52,25 @@ def fgp_traffic(kernel: str):
     return float(m.group(1)) if m else None
 
 
-def fgp_passes(inner: int) -> list[int]:
-    """FGP steps of each pass of one prox call: as few passes of at most four steps as it needs, with
-    the output, which the last pass forms, as one step more; of nearly equal length, the longer ones
-    first (TvState::prox)."""
-    passes = inner // 4 + 1
-    return [inner // passes + (k < inner % passes) for k in range(passes)]
+def fgp_passes(inner: int, voxels: int) -> tuple[list[int], bool]:
+    """FGP steps of each pass of one prox call, and whether the last forms the output: as few passes
+    of at most four steps as it needs, with the output as one step more where the last forms it; of
+    nearly equal length, the longer ones first (TvState::prox)."""
+    joined = not (inner % 4 == 0 and voxels >= 1 << 22)
+    passes = (inner + joined + 3) // 4
+    return [inner // passes + (k < inner % passes) for k in range(passes)], joined
 
 
-def fgp_pass_volumes(inner: int) -> list[int]:
+def fgp_pass_volumes(inner: int, voxels: int) -> list[int]:
     """Volumes (b, dual components, output) each FGP launch of one prox call must read and write.
     A pass of T steps reads b and p_k (3), plus p_{k-1} (3) except in the first (r = p there); it
     writes p_{k+T-1} (3; not the last pass, nor one of a single step) and p_{k+T} (3), the last
-    pass the output as well."""
+    pass the output as well where it forms it."""
     out = []
-    steps = fgp_passes(inner)
+    steps, joined = fgp_passes(inner, voxels)
     for k, t in enumerate(steps):
         last = k + 1 == len(steps)
-        out.append(1 + 3 + (3 if k else 0) + 3 + (1 if last else 3 if t > 1 else 0))
+        out.append(1 + 3 + (3 if k else 0) + 3 + (int(joined) if last else 3 if t > 1 else 0))
     return out
 
 
@@ -80,7 +81,7 @@ def reconstruction_bytes(count: int, holo: int, n: int, nz: int, iterations: int
     one write of its array however many passes it takes. Front end as the algorithmic model of
     the reference's stages (hologram R2C, crop, inverse, ratio, unwrap, Rytov, 2D FFT); mapping
     with uint16 hit counts; per outer iteration the five transform kernels (momentum fused into
-    the first, the data restore into the z pass) and the FGP passes (the last forms the output)."""
+    the first, the data restore into the z pass) and the FGP passes and the output."""
     a, nh, m = count, holo, n
     v = nz * n * n
     h = nz * n * (n // 2 + 1)
@@ -97,7 +98,8 @@ def reconstruction_bytes(count: int, holo: int, n: int, nz: int, iterations: int
              + 10 * v + 9 * h                            # Hermitian data and hits
              + 8 * h + 4 * v)                            # initial C2R
     transforms = (8 * v + 8 * h) + 16 * h + 25 * h + 16 * h + (8 * h + 4 * v)
-    prox = sum(fgp_pass_volumes(inner)) * 4 * v
+    # An output that no FGP pass forms is written from b and the dual (3).
+    prox = (sum(fgp_pass_volumes(inner, v)) + (0 if fgp_passes(inner, v)[1] else 5)) * 4 * v
     return int(front + iterations * (transforms + prox))
 
 
@@ -862,7 +864,7 @@ def main() -> int:
     launches = max(1, t["fgp_launches"])
     steps_per_launch = t["fgp_steps"] / launches
     kernel = "fgp_steps"
-    passes = fgp_pass_volumes(INNER)
+    passes = fgp_pass_volumes(INNER, N ** 3)
     assert len(passes) * ITERATIONS == launches, (passes, launches)
     # What the launches must move: per pass b and the dual iterates it reads, the iterates it
     # writes and the output (10, 13 and 11 volumes for the passes of 4, 3 and 3 steps).

@@ -83,7 +83,7 @@ typedef struct {
 
 /* src/backends.hpp:31-42 (OdtTimings), device event intervals in milliseconds, plus the summed
  * duration of the FGP dual-step kernels, the steps and the kernel passes they took (up to four
- * steps per pass, the last of which forms the output; FISTA-TV only). */
+ * steps per pass, the last of which may form the output as well; FISTA-TV only). */
 typedef struct {
   size_t bytes;
   double setup;

@@ -568,8 +568,8 @@ void TvState::reset(hipStream_t s, int batch) {
 std::size_t TvState::bytes() const { return owned_.bytes(); }
 
 // tv_prox of the reference (src/cpu/tv.cpp:7-44): r <- p, `inner` FGP steps, out = primal(p).
-// The steps go in as few passes as they need, the last of which forms the output and counts it as
-// a step more. The dual iterates rotate through four buffers: a pass of T steps reads p_k and p_{k-1} (r is formed
+// The steps go in as few passes as they need, the last of which forms the output where that leaves
+// it at most three steps. The dual iterates rotate through four buffers: a pass of T steps reads p_k and p_{k-1} (r is formed
 // inside it) and writes p_{k+T-1} and p_{k+T} to buffers nobody reads in that pass; the last pass
 // skips p_{k+T-1}, which the next call does not read (its first step uses r = p). The prox leaves
 // p in buffer cur_ for the next call.
@@ -580,10 +580,16 @@ void TvState::prox(const float* b, float* out, float lambda, int inner, hipStrea
   // An output that overlaps b is written only by a pass without steps: the stages of the others
   // read b beyond their own points, its last stage at them alone.
   const bool apart = out + vol_ * batch_ <= b || b + vol_ * batch_ <= out;
-  const bool joined = fused_ && apart && inner > 0;
+  // Step counts that are multiples of four: passes of four steps and one of the output alone move
+  // the fewest bytes; in small volumes, where a plane's latency bounds a pass, the output counts as
+  // a step more and the shares are smaller. A FISTA iteration of 4 / 8 / 20 steps this way and that:
+  // 479 / 751 / 1570 against 560 / 807 / 1627 us at 256^3, 216 / 340 / 711 against 251 / 362 / 742
+  // at 192^3, 233 / 405 / 919 against 286 / 412 / 896 at 162^3, 114 / 176 / 361 against 121 / 169 /
+  // 350 at 128^3, 58 / 88 / 176 against 56 / 82 / 169 at 64^3.
+  constexpr long kLarge = 1L << 22;
+  const bool whole = inner % kMaxSteps == 0 && vol_ * batch_ >= kLarge;
+  const bool joined = fused_ && apart && inner > 0 && !whole;
   const int most = fused_ ? kMaxSteps : 1;
-  // The output takes the place of a step: passes = ceil((inner + 1) / most), whose nearly equal
-  // shares of the steps leave the last at most `most` - 1.
   const int passes = (inner + (joined ? 1 : 0) + most - 1) / most;
   StepArgs a{};
   a.b = b;

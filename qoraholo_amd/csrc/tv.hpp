@@ -14,8 +14,8 @@ void fill(float* d, long n, float v, hipStream_t s);
 
 // Dual state of the TV prox, kept across calls (FISTA warm start): four rotating dual buffers
 // of three components each. Steps run up to four per pass, the last of which forms the output
-// (set_fused(false) runs them one per pass and the output in a kernel of its own, for
-// comparisons; the results are the same bits).
+// where it has at most three (set_fused(false) runs them one per pass and the output in a kernel
+// of its own, for comparisons; the results are the same bits).
 class TvState {
  public:
   // The dual buffers in device memory of its own, for up to `batch` volumes proxed together.

@@ -367,6 +367,20 @@ def test_tv_output_at_tile_seams_equals_oracle(device, oracle, shape, inner):
         assert np.array_equal(got, want), fused
 
 
+@pytest.mark.parametrize("shape,inner", [((300, 120, 120), 4), ((300, 120, 120), 8), ((272, 126, 124), 8)])
+def test_tv_whole_passes_of_large_volumes_equal_oracle(device, oracle, shape, inner):
+    """Volumes from 2^22 voxels up, whose step counts that are multiples of four take passes of four
+    steps and one of the output alone; rows in whole groups of four and not."""
+    from qoraholo_amd import _native
+
+    rng = np.random.default_rng(inner)
+    b = (rng.standard_normal(shape) * 0.3 + 0.3).astype(np.float32)
+    got = np.empty_like(b)
+    _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *shape, 0.1, inner, 1,
+                                               _native.ptr(got)))
+    assert np.array_equal(got, oracle.tv_prox(b, 0.1, inner))
+
+
 @pytest.mark.parametrize("inner", [4, 8])
 def test_tv_warm_dual_at_tile_seams_matches_oracle(device, oracle, qh, inner):
     """FISTA-TV over three iterations, whose later proxes start from the dual of the one before, on
