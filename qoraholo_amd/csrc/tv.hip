@@ -14,7 +14,8 @@
 // and 4 rows share no line they write. With plain rows a tile of 64 columns wrote parts of lines
 // and the 256^3 pass of three steps took 290-350 us against 220 us (a kernel that only moves the
 // same data in that pattern took 326 us cut at 58 columns, 231 us cut at 48, and 186-202 us in
-// quads).
+// quads). Planes of the dual hold whole quads: rows past the last of the volume are zero and stay
+// zero.
 //
 // Per prox of 10 steps, output included (4 + 3 + 3 steps), against two steps per pass and a kernel
 // for the output before: 671 against 837 us at 256^3, 1131 against 2635 us at 320^3, 1952 against
@@ -162,6 +163,7 @@ struct StepArgs {
   float* p_last;       // out: p_{k+T}, or null
   float* x;            // out with FINAL: the prox output
   long vol;
+  long dual_plane, dual_vol;  // floats of a plane and of a component of the dual
   int nz, ny, nx;
   float lambda;
   float step;
@@ -180,9 +182,10 @@ struct StepArgs {
 // T + 1 planes are back in place (a rolled loop moves 7 floats a point and stage back by v_mov). The
 // unrolled planes are numbered U = 0 .. T; without steps two planes, for two exchange buffers.
 //
-// QUADS: ny is a multiple of 4. Otherwise the rows of the last quad are stored column by column
-// like the others (h floats a column for h rows), which takes accesses of 4 bytes. FIRST: the first
-// pass of a prox, which needs no p_{k-1}.
+// QUADS: planes of the dual hold whole quads. Otherwise (a fixed workspace without room for them)
+// they end with the volume's last row, and the rows of the last quad are stored column by column like
+// the others (h floats a column for h rows), which takes accesses of 4 bytes: 206 against 128 us for a
+// prox of 10 steps at 90^3, 590 against 359 us at 270^2 x 90. FIRST: the first pass of a prox, which needs no p_{k-1}.
 template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
 struct StepMarch {
   static constexpr int NW = kWaves;
@@ -225,11 +228,20 @@ struct StepMarch {
   // plane, loaded a plane ahead.
   float pk[3][kRows], pm[3][kRows], bb[kRows];
 
+  // Floats of a plane and of a component of the dual, and bytes of the wave's quad in a plane. The
+  // fused form only runs on volumes whose rows fill their quads: the dual has the volume's own planes
+  // there, and the fewer values to hold are worth 2% (256^3: 16.33 against 16.72 ms a request).
+  __device__ __forceinline__ long dual_plane() const { return EXACT ? a.dual_plane : plane; }
+  __device__ __forceinline__ long dual_vol() const { return EXACT ? a.dual_vol : a.vol; }
+  __device__ __forceinline__ int dual_bytes() const {
+    return 4 * a.nx * (EXACT && QUADS && rows > 0 ? kRows : rows);
+  }
+
   __device__ __forceinline__ void load_dual(float (&v)[3][kRows], const float* p, long at,
                                             bool on) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const Window q(p + c * a.vol + at, 4 * rows * a.nx, on);
+      const Window q(p + c * dual_vol() + at, dual_bytes(), on);
       if constexpr (QUADS) {
         q.load4(v[c], xq);
       } else {
@@ -239,10 +251,10 @@ struct StepMarch {
     }
   }
   __device__ __forceinline__ void load(int f) {
-    const long at = static_cast<long>(min(f, a.nz - 1)) * plane + wave_row;
-    load_dual(pk, a.p_k, at, true);
-    if constexpr (!FIRST) load_dual(pm, a.p_km1, at, a.first == 0);
-    const Window b(a.b + at, 4 * rows * a.nx, true);
+    const long z = static_cast<long>(min(f, a.nz - 1));
+    load_dual(pk, a.p_k, z * dual_plane() + wave_row, true);
+    if constexpr (!FIRST) load_dual(pm, a.p_km1, z * dual_plane() + wave_row, a.first == 0);
+    const Window b(a.b + z * plane + wave_row, 4 * rows * a.nx, true);
 #pragma unroll
     for (int j = 0; j < kRows; ++j) bb[j] = b.load(xr + 4u * static_cast<unsigned>(j * a.nx));
   }
@@ -250,10 +262,10 @@ struct StepMarch {
   // Component-wise rows of p on plane z, where that is the tile's to write.
   __device__ __forceinline__ void store(float* p, int z, const float (&v)[kRows][3]) {
     const bool on = p != nullptr && wave_on && z >= z0 && z < z1;
-    const long at = static_cast<long>(max(z, 0)) * plane + wave_row;
+    const long at = static_cast<long>(max(z, 0)) * dual_plane() + wave_row;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const Window q(p + c * a.vol + at, 4 * rows * a.nx, on);
+      const Window q(p + c * dual_vol() + at, dual_bytes(), on);
       if constexpr (QUADS) {
         const float r[kRows] = {v[0][c], v[1][c], v[2][c], v[3][c]};
         q.stream4(r, xq_out);
@@ -378,10 +390,11 @@ __global__ void __launch_bounds__(kWaves * 64)
   // Volume blockIdx.y of a batch of volumes that lie one after another.
   const long batch = static_cast<long>(blockIdx.y);
   a.b += batch * a.vol;
-  a.p_k += 3 * batch * a.vol;
-  if (a.p_km1) a.p_km1 += 3 * batch * a.vol;
-  if (a.p_prev) a.p_prev += 3 * batch * a.vol;
-  if (a.p_last) a.p_last += 3 * batch * a.vol;
+  const long duals = 3 * batch * (EXACT ? a.dual_vol : a.vol);
+  a.p_k += duals;
+  if (a.p_km1) a.p_km1 += duals;
+  if (a.p_prev) a.p_prev += duals;
+  if (a.p_last) a.p_last += duals;
   if (a.x) a.x += batch * a.vol;
   M m{a, lds};
   // The wave index is uniform across the wave: as a scalar it keeps the row arithmetic, the
@@ -405,7 +418,7 @@ __global__ void __launch_bounds__(kWaves * 64)
   m.wave_row = m.rows > 0 ? static_cast<long>(m.yw) * a.nx : 0;
   const bool in_x = x >= 0 && x < a.nx;
   const bool out_x = in_x && x >= tx * a.tile_x && x < (tx + 1) * a.tile_x;
-  m.xq = in_x ? 4u * static_cast<unsigned>(x * m.rows) : kOutside;
+  m.xq = in_x ? 4u * static_cast<unsigned>(x * (QUADS && EXACT ? kRows : m.rows)) : kOutside;
   m.xr = in_x ? 4u * static_cast<unsigned>(x) : kOutside;
   m.xq_out = out_x ? m.xq : kOutside;
   m.xr_out = out_x ? m.xr : kOutside;
@@ -481,6 +494,10 @@ int step_chunk(int steps, int halo, int turn, long tiles, int nz) {
   return best;
 }
 
+// Rows of a plane of the dual that holds whole quads.
+long whole_quads(int ny) { return (static_cast<long>(ny) + kRows - 1) / kRows * kRows; }
+
+// Volumes whose rows do not fill their last quad round every operation, as their results always have.
 template <int T, bool FIRST, bool FINAL>
 void launch_steps(StepArgs a, hipStream_t s, int batch, bool exact) {
   const auto cut = [](int n, int width, int& own, int& halo) {
@@ -496,9 +513,9 @@ void launch_steps(StepArgs a, hipStream_t s, int batch, bool exact) {
   const int chunks = (a.nz + a.zlen - 1) / a.zlen;
   const dim3 grid(static_cast<unsigned>(tiles * chunks), static_cast<unsigned>(batch));
   const dim3 block(kWaves * 64);
-  if (a.ny % kRows != 0) {
+  if (a.dual_plane != whole_quads(a.ny) * a.nx) {
     hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, false, true>), grid, block, 0, s, a);
-  } else if (exact) {
+  } else if (exact || a.ny % kRows != 0) {
     hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, true, true>), grid, block, 0, s, a);
   } else {
     hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, true, false>), grid, block, 0, s, a);
@@ -519,7 +536,7 @@ void launch_steps_of(const StepArgs& a, hipStream_t s, int batch, bool exact) {
 }
 
 // `steps` FGP steps in one pass (up to kMaxSteps); with x set, the prox output after them (up to
-// kMaxSteps - 1; 0 steps: of p_k). Only whole quads have kernels with fused arithmetic.
+// kMaxSteps - 1; 0 steps: of p_k).
 void fgp_steps(int steps, const StepArgs& a, hipStream_t s, int batch, bool exact) {
   require(steps + (a.x ? 1 : 0) <= kMaxSteps, "tv: too many steps in a pass");
   switch (steps) {
@@ -535,8 +552,8 @@ void fgp_steps(int steps, const StepArgs& a, hipStream_t s, int batch, bool exac
 // Floats of one dual buffer (three components per volume of the batch, one volume's after
 // another's), rounded up to 256 bytes so that every buffer of a workspace starts 256-byte
 // aligned.
-std::size_t dual_floats(int nz, int ny, int nx, int batch = 1) {
-  const std::size_t three = 3 * static_cast<std::size_t>(nz) * ny * nx * batch;
+std::size_t dual_floats(int nz, long rows, int nx, int batch = 1) {
+  const std::size_t three = 3 * static_cast<std::size_t>(nz) * rows * nx * batch;
   return (three + 63) / 64 * 64;
 }
 
@@ -545,23 +562,25 @@ std::size_t dual_floats(int nz, int ny, int nx, int batch = 1) {
 std::size_t TvState::workspace_floats(int nz, int ny, int nx) { return 4 * dual_floats(nz, ny, nx); }
 
 TvState::TvState(int nz, int ny, int nx, int batch)
-    : nz_(nz), ny_(ny), nx_(nx), vol_(static_cast<long>(nz) * ny * nx), cap_(batch),
-      owned_(4 * dual_floats(nz, ny, nx, std::max(batch, 1))) {
+    : nz_(nz), ny_(ny), nx_(nx), vol_(static_cast<long>(nz) * ny * nx), rows_(whole_quads(ny)),
+      cap_(batch), owned_(4 * dual_floats(nz, rows_, nx, std::max(batch, 1))) {
   require(batch >= 1 && batch <= 65535, "tv: the batch must be 1 to 65535");
-  const std::size_t stride = dual_floats(nz, ny, nx, batch);
+  const std::size_t stride = dual_floats(nz, rows_, nx, batch);
   for (int i = 0; i < 4; ++i) p_[i] = owned_.get() + i * stride;
 }
 
-TvState::TvState(int nz, int ny, int nx, float* workspace)
-    : nz_(nz), ny_(ny), nx_(nx), vol_(static_cast<long>(nz) * ny * nx) {
-  const std::size_t stride = dual_floats(nz, ny, nx);
+TvState::TvState(int nz, int ny, int nx, float* workspace, std::size_t floats)
+    : nz_(nz), ny_(ny), nx_(nx), vol_(static_cast<long>(nz) * ny * nx), rows_(whole_quads(ny)) {
+  require(workspace_floats(nz, ny, nx) <= floats, "tv: the workspace is too small");
+  if (4 * dual_floats(nz, rows_, nx) > floats) rows_ = ny;
+  const std::size_t stride = dual_floats(nz, rows_, nx);
   for (int i = 0; i < 4; ++i) p_[i] = workspace + i * stride;
 }
 
 void TvState::reset(hipStream_t s, int batch) {
   require(batch >= 1 && batch <= cap_, "tv: batch beyond the state's capacity");
   batch_ = batch;
-  fill(p_[0], 3 * vol_ * batch, 0.0f, s);
+  fill(p_[0], 3 * nz_ * rows_ * nx_ * batch, 0.0f, s);
   cur_ = 0;
 }
 
@@ -594,6 +613,8 @@ void TvState::prox(const float* b, float* out, float lambda, int inner, hipStrea
   StepArgs a{};
   a.b = b;
   a.vol = vol_;
+  a.dual_plane = rows_ * nx_;
+  a.dual_vol = nz_ * a.dual_plane;
   a.nz = nz_;
   a.ny = ny_;
   a.nx = nx_;

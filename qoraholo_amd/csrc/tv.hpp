@@ -20,9 +20,9 @@ class TvState {
  public:
   // The dual buffers in device memory of its own, for up to `batch` volumes proxed together.
   TvState(int nz, int ny, int nx, int batch = 1);
-  // The dual buffers in `workspace` (workspace_floats(nz, ny, nx) floats of device memory,
-  // 256-byte aligned, not owned: it must outlive the state).
-  TvState(int nz, int ny, int nx, float* workspace);
+  // The dual buffers in `workspace` (`floats` of device memory, at least workspace_floats(nz, ny,
+  // nx), 256-byte aligned, not owned: it must outlive the state).
+  TvState(int nz, int ny, int nx, float* workspace, std::size_t floats);
   static std::size_t workspace_floats(int nz, int ny, int nx);
   // Zero duals for the next `batch` volumes (at most the capacity), which every prox until the
   // next reset takes together: b and out then hold that many volumes one after another.
@@ -42,6 +42,7 @@ class TvState {
  private:
   int nz_, ny_, nx_;
   long vol_;
+  long rows_;      // of a plane of the dual: ny, in whole groups of four where the buffers have room
   int cap_ = 1;    // volumes the buffers hold
   int batch_ = 1;  // volumes of the current solve
   DeviceBuffer<float> owned_;

@@ -61,7 +61,7 @@ int qh_hip_tv_prox_dev_noalloc(const float* b, int nz, int ny, int nx, float lam
     require(TvState::workspace_floats(nz, ny, nx) <= kScratchFloats,
             "tv_prox_dev_noalloc: dual buffers exceed the scratch array");
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    TvState state(nz, ny, nx, device_scratch());
+    TvState state(nz, ny, nx, device_scratch(), kScratchFloats);
     state.set_fused(fused != 0);
     state.reset(s);  // the dual starts at zero: the array keeps the last call's contents
     state.prox(b, x, lambda, inner, s);

@@ -63,6 +63,28 @@ def test_noalloc_prox_in_place(device):
         assert np.array_equal(bd.cpu().numpy().view(np.uint32), want.view(np.uint32)), shape
 
 
+@pytest.mark.parametrize("shape,inner", [((128, 127, 129), 10), ((3000, 1, 500), 3), ((700, 5, 450), 4)])
+def test_noalloc_prox_without_room_for_whole_groups_of_rows(device, shape, inner):
+    """Volumes near the limit whose row count is no multiple of four: the fixed array holds their
+    dual only without the rows that would fill the last group. The allocating call has that room."""
+    import torch
+    from qoraholo_amd import _native
+
+    lib = _native.lib()
+    rows = -(-shape[1] // 4) * 4
+    assert np.prod(shape) <= MAX_VOXELS < shape[0] * rows * shape[2]
+    rng = np.random.default_rng(shape[1])
+    b = (rng.standard_normal(shape) * 0.2 + 0.3).astype(np.float32)
+    want = _prox_allocating(lib, _native, b, 0.05, inner, 1)
+    bd = torch.from_numpy(b).cuda()
+    xd = torch.empty_like(bd)
+    _native.check(lib.qh_hip_tv_prox_dev_noalloc(
+        _native.ptr(bd.data_ptr()), *shape, 0.05, inner, 1, _native.ptr(xd.data_ptr()),
+        _native.ptr(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    assert np.array_equal(xd.cpu().numpy(), want)
+
+
 def test_noalloc_prox_refuses_volumes_above_the_limit(device):
     import torch
     from qoraholo_amd import _native
