@@ -46,14 +46,6 @@ std::string& last_error() {
 
 namespace {
 
-// Per-thread stream of the per-call entry points, so calls from different host threads run
-// independently.
-hipStream_t call_stream() {
-  thread_local std::unique_ptr<Stream> s;
-  if (!s) s = std::make_unique<Stream>();
-  return s->get();
-}
-
 void require_device() {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess || n < 1) throw DeviceError("no HIP device available");

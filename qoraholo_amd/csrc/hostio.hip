@@ -13,6 +13,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "runtime.hpp"
@@ -125,22 +126,24 @@ CopyPool& pool() {
 
 // The calling thread's pinned slots and what marks their last DMA: slots 0 .. kSlots - 1 upload,
 // the others download. A slot grows to what it is used for, so that a thread's small calls pin
-// little. Transfers of one slot are marked by their stream alone (an event after each is 10 us of a
-// small call); several in a row by events.
+// little. Transfers of one slot on the thread's own stream are marked by that stream alone (an event
+// after each is 10 us of a small call); several in a row, and all on other streams, which may be
+// destroyed before the slot is used again, by the slot's event.
 struct Staging {
+  std::unique_ptr<Stream> own;  // call_stream()
   PinnedBuffer<char> memory[2 * kSlots];
   Event done[2 * kSlots]{Event(false), Event(false), Event(false), Event(false),
                          Event(false), Event(false), Event(false), Event(false)};
   enum class Mark { none, event, stream };
   Mark mark[2 * kSlots] = {};
-  hipStream_t stream[2 * kSlots] = {};
   int up = 0;
   int down = 0;
 
+  // An error is reported once: the slot is free after it.
   void wait(int i) {
-    if (mark[i] == Mark::event) check(hipEventSynchronize(done[i].get()), "hipEventSynchronize");
-    if (mark[i] == Mark::stream) check(hipStreamSynchronize(stream[i]), "hipStreamSynchronize");
-    mark[i] = Mark::none;
+    const Mark m = std::exchange(mark[i], Mark::none);
+    if (m == Mark::event) check(hipEventSynchronize(done[i].get()), "hipEventSynchronize");
+    if (m == Mark::stream) check(hipStreamSynchronize(own->get()), "hipStreamSynchronize");
   }
   // Slot i, its last DMA over, with room for `bytes`.
   char* slot(int i, std::size_t bytes) {
@@ -152,9 +155,9 @@ struct Staging {
     return memory[i].get();
   }
   void queued(int i, hipStream_t s, bool alone) {
-    if (!alone) done[i].record(s);
-    mark[i] = alone ? Mark::stream : Mark::event;
-    stream[i] = s;
+    const bool by_stream = alone && own && s == own->get();
+    if (!by_stream) done[i].record(s);
+    mark[i] = by_stream ? Mark::stream : Mark::event;
   }
 };
 
@@ -195,6 +198,12 @@ void parallel_for(int parts, const std::function<void(int)>& part) {
     return;
   }
   pool().run(parts, part);
+}
+
+hipStream_t call_stream() {
+  Staging& st = staging();
+  if (!st.own) st.own = std::make_unique<Stream>();
+  return st.own->get();
 }
 
 void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s) {

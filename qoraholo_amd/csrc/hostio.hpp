@@ -29,6 +29,10 @@ void host_copy(void* dst, const void* src, std::size_t bytes);
 // done.
 void parallel_for(int parts, const std::function<void(int)>& part);
 
+// Per-thread stream of the per-call entry points, so calls from different host threads run
+// independently. It lives as long as the thread's staging slots.
+hipStream_t call_stream();
+
 // Device dst <- pageable host src. Returns once src may be reused; the DMA of the last chunks
 // may still be in flight on s, ahead of any later work on s.
 void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s);
@@ -41,8 +45,8 @@ void download(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 // as far as the staging slots go, finish() with every dst complete.
 class Downloads {
  public:
-  // alone: next to nothing is queued behind it on s before finish(), so that it is waited for with
-  // the stream and needs no event.
+  // alone: next to nothing is queued behind it on s before finish(), so that on call_stream() it is
+  // waited for with the stream and needs no event.
   void add(void* dst, const void* src, std::size_t bytes, hipStream_t s, bool alone = false);
   void finish();
 

@@ -185,7 +185,8 @@ struct StepArgs {
 // QUADS: planes of the dual hold whole quads. Otherwise (a fixed workspace without room for them)
 // they end with the volume's last row, and the rows of the last quad are stored column by column like
 // the others (h floats a column for h rows), which takes accesses of 4 bytes: 206 against 128 us for a
-// prox of 10 steps at 90^3, 590 against 359 us at 270^2 x 90. FIRST: the first pass of a prox, which needs no p_{k-1}.
+// prox of 10 steps at 90^3, 590 against 359 us at 270^2 x 90. FIRST: the first pass of a prox, which
+// needs no p_{k-1}.
 template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
 struct StepMarch {
   static constexpr int NW = kWaves;

@@ -266,3 +266,21 @@ def test_batched_and_single_geometries_mix(device, qh, mixed):
         ri, _, _ = server.wait(rid)
         assert np.array_equal(ri, mixed[k][1]), k
     assert server.stats()["failed"] == 0
+
+
+def test_calls_after_a_batched_server_has_gone(device, qh, mixed):
+    """A batched slot uploads its backgrounds through the staging of the thread that builds it, on a
+    stream of its own. Calls of that thread, which take the same staging slots in turn, go on when
+    the slot and its stream no longer exist, and a second server's stream may have taken its place."""
+    d, alone = mixed[0]
+    assert d.bg.nbytes <= 4 << 20
+    field = (np.arange(3 * 64 * 64) % 17).reshape(3, 64, 64).astype(np.complex64)
+    want = qh.rytov(field + 1)
+    for _ in range(2):
+        server = qh.Server(max_slots=1)
+        gid = server.add_geometry(d.count, d.size, illuminations=d.illum, geometry=d.geom,
+                                  backgrounds=d.bg, max_batch=2, **d.kw)
+        assert np.array_equal(server.wait(server.submit(gid, d.holo))[0], alone)
+        del server
+        for _ in range(6):
+            assert np.array_equal(qh.rytov(field + 1), want)
