@@ -22,10 +22,21 @@ namespace qh {
 
 namespace {
 
-constexpr std::size_t kChunk = kStagingSlot;
 constexpr int kSlots = 4;  // of each direction
-// Host copies are split into parts of at least this size.
+// Chunks of transfers that take several: two slots in turn. A DMA of 4 MB leaves a gap of a seventh
+// of its time to the next one (128 / 256 MB in and out: 7.0 / 13.0 ms in chunks of 4 MB, 5.5 / 10.7 of
+// 8, 5.4 / 10.4 of 16), and the first and last host copy of a smaller transfer wait for less in
+// smaller chunks (24 MB: 1.21 ms of 8, 1.27 to 1.33 of 16).
+constexpr std::size_t kLarge = std::size_t(128) << 20;
+constexpr std::size_t kLargeChunk = std::size_t(16) << 20;
+constexpr std::size_t chunk_of(std::size_t bytes) {
+  return bytes > kLarge ? kLargeChunk : kStagingSlot;
+}
+// Host copies are split over threads, into parts of at least kMinPart, from where that pays for waking
+// them (calls that move 1 / 1.25 / 1.5 MB in and out: 162 / 180 / 180 us by two threads, 137 / 158 /
+// 200 us by one).
 constexpr std::size_t kMinPart = std::size_t(1) << 19;
+constexpr std::size_t kMinSplit = 3 * kMinPart;
 
 int usable_cpus() {
   cpu_set_t set;
@@ -150,7 +161,7 @@ struct Staging {
     wait(i);
     if (memory[i].size() < bytes) {
       memory[i] = PinnedBuffer<char>();
-      memory[i] = PinnedBuffer<char>(std::clamp(std::bit_ceil(bytes), std::size_t(1) << 16, kChunk));
+      memory[i] = PinnedBuffer<char>(std::max(std::bit_ceil(bytes), std::size_t(1) << 16));
     }
     return memory[i].get();
   }
@@ -160,6 +171,13 @@ struct Staging {
     mark[i] = by_stream ? Mark::stream : Mark::event;
   }
 };
+
+// The next slot of a ring at `at`: of all slots, or of two for a transfer in several chunks.
+int next_slot(int& at, bool several) {
+  const int i = at % (several ? 2 : kSlots);
+  at = (i + 1) % kSlots;
+  return i;
+}
 
 Staging& staging() {
   thread_local std::unique_ptr<Staging> s;
@@ -176,7 +194,7 @@ int host_copy_threads() {
 
 void host_copy(void* dst, const void* src, std::size_t bytes) {
   const int threads = host_copy_threads();
-  if (bytes < 2 * kMinPart || threads == 1) {
+  if (bytes < kMinSplit || threads == 1) {
     std::memcpy(dst, src, bytes);
     return;
   }
@@ -210,14 +228,14 @@ void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s) {
   Staging& st = staging();
   auto* d = static_cast<char*>(dst);
   const auto* h = static_cast<const char*>(src);
-  for (std::size_t off = 0; off < bytes; off += kChunk) {
-    const std::size_t len = std::min(kChunk, bytes - off);
-    const int i = st.up;
-    st.up = (st.up + 1) % kSlots;
+  const std::size_t chunk = chunk_of(bytes);
+  for (std::size_t off = 0; off < bytes; off += chunk) {
+    const std::size_t len = std::min(chunk, bytes - off);
+    const int i = next_slot(st.up, bytes > chunk);
     char* const slot = st.slot(i, len);
     host_copy(slot, h + off, len);
     check(hipMemcpyAsync(d + off, slot, len, hipMemcpyHostToDevice, s), "upload");
-    st.queued(i, s, bytes <= kChunk);
+    st.queued(i, s, bytes <= chunk);
   }
 }
 
@@ -225,11 +243,13 @@ void Downloads::add(void* dst, const void* src, std::size_t bytes, hipStream_t s
   Staging& st = staging();
   auto* h = static_cast<char*>(dst);
   const auto* d = static_cast<const char*>(src);
-  for (std::size_t off = 0; off < bytes; off += kChunk) {
-    const std::size_t len = std::min(kChunk, bytes - off);
-    if (static_cast<int>(parts_.size()) == kSlots) retire();
-    const int i = kSlots + st.down;
-    st.down = (st.down + 1) % kSlots;
+  const std::size_t chunk = chunk_of(bytes);
+  for (std::size_t off = 0; off < bytes; off += chunk) {
+    const std::size_t len = std::min(chunk, bytes - off);
+    const int i = kSlots + next_slot(st.down, bytes > chunk);
+    while (std::any_of(parts_.begin(), parts_.end(), [&](const Part& p) { return p.slot == i; })) {
+      retire();
+    }
     check(hipMemcpyAsync(st.slot(i, len), d + off, len, hipMemcpyDeviceToHost, s), "download");
     st.queued(i, s, alone);
     parts_.push_back({i, h + off, len});
@@ -249,7 +269,7 @@ void Downloads::finish() {
 
 void download(void* dst, const void* src, std::size_t bytes, hipStream_t s) {
   Downloads d;
-  d.add(dst, src, bytes, s, bytes <= kChunk);
+  d.add(dst, src, bytes, s, bytes <= kStagingSlot);
   d.finish();
 }
 

@@ -14,9 +14,10 @@
 
 namespace qh {
 
-// Size of a staging slot: a copy into it takes about half the time of its DMA (37 of 82 us), so that
-// the first chunk's copy is all the DMA waits for and the last chunk's all that follows it.
-inline constexpr std::size_t kStagingSlot = std::size_t(4) << 20;
+// Transfers up to this size go through one staging slot: a copy into it takes about half the time of
+// its DMA, so that the first chunk's copy is all the DMA of a larger transfer waits for and the last
+// chunk's all that follows it.
+inline constexpr std::size_t kStagingSlot = std::size_t(8) << 20;
 
 // Threads a host copy is spread over (the caller included): half the CPUs this process may
 // run on, at most 8.

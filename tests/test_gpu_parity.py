@@ -255,6 +255,21 @@ def test_gp_complex_passes_match_oracle(device, oracle, qh, n, nz):
         assert filled == want_filled
 
 
+def test_host_transfers_of_every_chunking_are_whole(device):
+    """Transfers below and from the sizes where the host copy is split (1.5 MB), where a transfer
+    takes several chunks (above 8 MB) and larger ones (above 128 MB), in an order in which slots
+    grow: the output without steps is max(b, 0), bit for bit."""
+    from qoraholo_amd import _native
+
+    rng = np.random.default_rng(3)
+    for nz in (1, 191, 192, 1024, 1025, 2049, 16384, 16385, 17500, 1, 1025):
+        b = rng.random((nz, 4, 512), np.float32) - np.float32(0.5)
+        got = np.empty_like(b)
+        _native.check(_native.lib().qh_hip_tv_prox(_native.ptr(b), *b.shape, 0.05, 0, 1,
+                                                   _native.ptr(got)))
+        assert np.array_equal(got, np.maximum(b, 0)), nz
+
+
 def test_calls_of_several_threads_share_device_memory(device, qh):
     """Calls of different sizes from several threads at once, which hand each other the blocks of
     their buffers: the results of the same calls one after another."""
