@@ -11,106 +11,14 @@
 #include "gp_complex.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
-#include "common.hpp"
-#include "fft.hpp"
-#include "fft_engine.hpp"
-#include "runtime.hpp"
-#include "split_lines.hpp"
+#include "gp_complex_kernels.hpp"
 
 namespace qh {
 
 namespace {
 
-struct RowArgs {
-  LineGeom g;
-  float2* p;
-  float scale;
-};
-
-struct IndexArgs {
-  LineGeom g;
-  const float2* p;
-  float scale;
-  float nm2;
-  float inv_k02;
-  float* ri;
-};
-
-struct ZLineArgs {
-  LineGeom g;
-  float2* p;
-  const float2* measured;
-  const std::uint16_t* counts;
-  long plane;
-};
-
-template <class E>
-__global__ void __launch_bounds__(E::kBlock) k_gp_rows(RowArgs a) {
-  E e(a.g);
-  const long n = a.g.n;
-  e.load([&](long l, int i) { return a.p[l * n + i]; });
-  e.first(true);
-  e.mid([&](long, int, float2& v) {
-    const float x = v.x * a.scale;
-    v = {x < 0.0f ? 0.0f : x, 0.0f};
-  });
-  e.second(false);
-  e.store2([&](long l, int k, float2 v) { a.p[l * n + k] = v; });
-}
-
-template <class E>
-__global__ void __launch_bounds__(E::kBlock) k_gp_index(IndexArgs a) {
-  E e(a.g);
-  const long n = a.g.n;
-  e.load([&](long l, int i) { return a.p[l * n + i]; });
-  e.first(true);
-  e.store1([&](long l, int x, float2 v) {
-    const float2 p = cscale(v, a.scale);
-    a.ri[l * n + x] = index_from_potential(p.x, p.y, a.nm2, a.inv_k02);
-  });
-}
-
-// Most bins are not measured: their counts come first (ahead of the transform where the engine
-// numbers its bins) and the measured values only where they say so.
-template <class E>
-__global__ void __launch_bounds__(E::kBlock) k_gp_z(ZLineArgs a) {
-  E e(a.g);
-  e.load([&](long l, int i) { return a.p[i * a.plane + l]; });
-  if constexpr (requires { E::kBins; }) {
-    std::uint16_t c[E::kBins];
-    e.bins([&](int i, long l, int k, float2&) { c[i] = a.counts[k * a.plane + l]; });
-    e.first(false);
-    e.bins([&](int i, long l, int k, float2& v) {
-      if (c[i] > 0) v = a.measured[k * a.plane + l];
-    });
-  } else {
-    e.first(false);
-    e.mid([&](long l, int k, float2& v) {
-      if (a.counts[k * a.plane + l] > 0) v = a.measured[k * a.plane + l];
-    });
-  }
-  e.second(true);
-  e.store2([&](long l, int i, float2 v) { a.p[i * a.plane + l] = v; });
-}
-
-template <class E>
-void launch(RowArgs a, unsigned grid, std::size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL(k_gp_rows<E>, dim3(grid), dim3(E::kBlock), lds, s, a);
-}
-template <class E>
-void launch(IndexArgs a, unsigned grid, std::size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL(k_gp_index<E>, dim3(grid), dim3(E::kBlock), lds, s, a);
-}
-template <class E>
-void launch(ZLineArgs a, unsigned grid, std::size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL(k_gp_z<E>, dim3(grid), dim3(E::kBlock), lds, s, a);
-}
-
-// Rows: about 256 threads a block. Adjacent lines: 16, a whole 128-byte segment of each block row.
-template <class A>
-constexpr bool kAdjacent = std::is_same_v<A, ZLineArgs>;
+using namespace gp;
 
 constexpr int floor_pow2(int v) { return v < 2 ? 1 : 2 * floor_pow2(v / 2); }
 
@@ -121,16 +29,6 @@ void launch_reg(const A& a, hipStream_t s) {
   using E = RegLines<N1, N2, kAdjacent<A>, kLines * kT>;
   launch<E>(a, E::grid(a.g.lines), 0, s);
 }
-
-template <int N>
-struct Split {
-  template <class A>
-  static void run(const A& a, hipStream_t s) {
-    constexpr int kT = SplitLines<N, false, 1>::T;
-    using E = SplitLines<N, kAdjacent<A>, kAdjacent<A> ? 16 : std::max(1, 256 / kT)>;
-    launch<E>(a, E::grid(a.g.lines), 0, s);
-  }
-};
 
 template <class A>
 void run(A a, const char* what, hipStream_t s) {
@@ -146,7 +44,7 @@ void run(A a, const char* what, hipStream_t s) {
     case 384: launch_reg<16, 24>(a, s); break;
     case 512: launch_reg<32, 16>(a, s); break;
     default: {
-      if (with_split<Split>(a.g.n, a, s)) break;
+      if (split(a, s)) break;
       using E = LdsLines<!kAdjacent<A>>;
       a.g.lines_per_block = E::lines_per_block(a.g.n);
       launch<E>(a, E::grid(a.g.lines, a.g.lines_per_block), E::dynamic_lds(a.g.n), s);
