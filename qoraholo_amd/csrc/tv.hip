@@ -163,7 +163,6 @@ struct StepArgs {
   float* p_last;       // out: p_{k+T}, or null
   float* x;            // out with FINAL: the prox output
   long vol;
-  long dual_plane, dual_vol;  // floats of a plane and of a component of the dual
   int nz, ny, nx;
   float lambda;
   float step;
@@ -175,6 +174,7 @@ struct StepArgs {
   int halo_x, halo_y;    // kHalo, or 0 where one tile holds the volume's side
   int to_index;          // the output as refractive index
   float nm2, inv_k02;
+  long dual_plane, dual_vol;  // floats of a plane and of a component of the dual
 };
 
 // The march, unrolled over T + 1 planes: the r and p a stage hands on take the registers of the
@@ -182,12 +182,18 @@ struct StepArgs {
 // T + 1 planes are back in place (a rolled loop moves 7 floats a point and stage back by v_mov). The
 // unrolled planes are numbered U = 0 .. T; without steps two planes, for two exchange buffers.
 //
-// QUADS: planes of the dual hold whole quads. Otherwise (a fixed workspace without room for them)
-// they end with the volume's last row, and the rows of the last quad are stored column by column like
-// the others (h floats a column for h rows), which takes accesses of 4 bytes: 206 against 128 us for a
-// prox of 10 steps at 90^3, 590 against 359 us at 270^2 x 90. FIRST: the first pass of a prox, which
-// needs no p_{k-1}.
-template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
+// FIRST: the first pass of a prox, which needs no p_{k-1}.
+//
+// ROWS: how the volume's rows fill the quads of the dual. whole: ny is a multiple of 4. filled: the
+// dual's planes hold the rest of the last quad as well (a variant of its own: the sizes that then
+// differ between the dual and b are values to hold, 2% of a 256^3 request, 16.72 against 16.33 ms).
+// cut: the dual's planes end with the volume's last row (a fixed workspace without room for more), and
+// the rows of the last quad are stored column by column like the others (h floats a column for h
+// rows), which takes accesses of 4 bytes: 206 against 128 us for a prox of 10 steps at 90^3, 590
+// against 359 us at 270^2 x 90.
+enum class Rows { whole, filled, cut };
+
+template <int T, bool FIRST, bool FINAL, Rows ROWS, bool EXACT>
 struct StepMarch {
   static constexpr int NW = kWaves;
   static constexpr int HL = T + (FINAL ? 1 : 0);  // planes in front of a chunk
@@ -229,13 +235,15 @@ struct StepMarch {
   // plane, loaded a plane ahead.
   float pk[3][kRows], pm[3][kRows], bb[kRows];
 
-  // Floats of a plane and of a component of the dual, and bytes of the wave's quad in a plane. The
-  // fused form only runs on volumes whose rows fill their quads: the dual has the volume's own planes
-  // there, and the fewer values to hold are worth 2% (256^3: 16.33 against 16.72 ms a request).
-  __device__ __forceinline__ long dual_plane() const { return EXACT ? a.dual_plane : plane; }
-  __device__ __forceinline__ long dual_vol() const { return EXACT ? a.dual_vol : a.vol; }
+  // Floats of a plane and of a component of the dual, and bytes of the wave's quad in a plane.
+  __device__ __forceinline__ long dual_plane() const {
+    return ROWS == Rows::filled ? a.dual_plane : plane;
+  }
+  __device__ __forceinline__ long dual_vol() const {
+    return ROWS == Rows::filled ? a.dual_vol : a.vol;
+  }
   __device__ __forceinline__ int dual_bytes() const {
-    return 4 * a.nx * (EXACT && QUADS && rows > 0 ? kRows : rows);
+    return ROWS == Rows::filled && rows > 0 ? 4 * kRows * a.nx : 4 * rows * a.nx;
   }
 
   __device__ __forceinline__ void load_dual(float (&v)[3][kRows], const float* p, long at,
@@ -243,7 +251,7 @@ struct StepMarch {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const Window q(p + c * dual_vol() + at, dual_bytes(), on);
-      if constexpr (QUADS) {
+      if constexpr (ROWS != Rows::cut) {
         q.load4(v[c], xq);
       } else {
 #pragma unroll
@@ -253,9 +261,11 @@ struct StepMarch {
   }
   __device__ __forceinline__ void load(int f) {
     const long z = static_cast<long>(min(f, a.nz - 1));
-    load_dual(pk, a.p_k, z * dual_plane() + wave_row, true);
-    if constexpr (!FIRST) load_dual(pm, a.p_km1, z * dual_plane() + wave_row, a.first == 0);
-    const Window b(a.b + z * plane + wave_row, 4 * rows * a.nx, true);
+    const long at = z * plane + wave_row;
+    const long dual_at = z * dual_plane() + wave_row;
+    load_dual(pk, a.p_k, dual_at, true);
+    if constexpr (!FIRST) load_dual(pm, a.p_km1, dual_at, a.first == 0);
+    const Window b(a.b + at, 4 * rows * a.nx, true);
 #pragma unroll
     for (int j = 0; j < kRows; ++j) bb[j] = b.load(xr + 4u * static_cast<unsigned>(j * a.nx));
   }
@@ -267,7 +277,7 @@ struct StepMarch {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const Window q(p + c * dual_vol() + at, dual_bytes(), on);
-      if constexpr (QUADS) {
+      if constexpr (ROWS != Rows::cut) {
         const float r[kRows] = {v[0][c], v[1][c], v[2][c], v[3][c]};
         q.stream4(r, xq_out);
       } else {
@@ -383,19 +393,19 @@ struct StepMarch {
   }
 };
 
-template <int T, bool FIRST, bool FINAL, bool QUADS, bool EXACT>
+template <int T, bool FIRST, bool FINAL, Rows ROWS, bool EXACT>
 __global__ void __launch_bounds__(kWaves * 64)
     __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) k_fgp_steps(StepArgs a) {
-  using M = StepMarch<T, FIRST, FINAL, QUADS, EXACT>;
+  using M = StepMarch<T, FIRST, FINAL, ROWS, EXACT>;
   __shared__ typename M::Lds lds;
   // Volume blockIdx.y of a batch of volumes that lie one after another.
   const long batch = static_cast<long>(blockIdx.y);
   a.b += batch * a.vol;
-  const long duals = 3 * batch * (EXACT ? a.dual_vol : a.vol);
-  a.p_k += duals;
-  if (a.p_km1) a.p_km1 += duals;
-  if (a.p_prev) a.p_prev += duals;
-  if (a.p_last) a.p_last += duals;
+  const long dual_vol = ROWS == Rows::filled ? a.dual_vol : a.vol;
+  a.p_k += 3 * batch * dual_vol;
+  if (a.p_km1) a.p_km1 += 3 * batch * dual_vol;
+  if (a.p_prev) a.p_prev += 3 * batch * dual_vol;
+  if (a.p_last) a.p_last += 3 * batch * dual_vol;
   if (a.x) a.x += batch * a.vol;
   M m{a, lds};
   // The wave index is uniform across the wave: as a scalar it keeps the row arithmetic, the
@@ -419,7 +429,7 @@ __global__ void __launch_bounds__(kWaves * 64)
   m.wave_row = m.rows > 0 ? static_cast<long>(m.yw) * a.nx : 0;
   const bool in_x = x >= 0 && x < a.nx;
   const bool out_x = in_x && x >= tx * a.tile_x && x < (tx + 1) * a.tile_x;
-  m.xq = in_x ? 4u * static_cast<unsigned>(x * (QUADS && EXACT ? kRows : m.rows)) : kOutside;
+  m.xq = in_x ? 4u * static_cast<unsigned>(x * (ROWS == Rows::filled ? kRows : m.rows)) : kOutside;
   m.xr = in_x ? 4u * static_cast<unsigned>(x) : kOutside;
   m.xq_out = out_x ? m.xq : kOutside;
   m.xr_out = out_x ? m.xr : kOutside;
@@ -515,11 +525,13 @@ void launch_steps(StepArgs a, hipStream_t s, int batch, bool exact) {
   const dim3 grid(static_cast<unsigned>(tiles * chunks), static_cast<unsigned>(batch));
   const dim3 block(kWaves * 64);
   if (a.dual_plane != whole_quads(a.ny) * a.nx) {
-    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, false, true>), grid, block, 0, s, a);
-  } else if (exact || a.ny % kRows != 0) {
-    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, true, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, Rows::cut, true>), grid, block, 0, s, a);
+  } else if (a.ny % kRows != 0) {
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, Rows::filled, true>), grid, block, 0, s, a);
+  } else if (exact) {
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, Rows::whole, true>), grid, block, 0, s, a);
   } else {
-    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, true, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_fgp_steps<T, FIRST, FINAL, Rows::whole, false>), grid, block, 0, s, a);
   }
 }
 
