@@ -98,7 +98,9 @@ constexpr int mid_group() {
 // waves per SIMD (adjoint of 96 slices of 128^2 with 9 illuminations 1370 -> 1275 us, with 25 1535
 // -> 1466 us; 64 of 192^2 with 49 2055 -> 2000 us; of 256^2 with 49 3077 -> 3139 us). The other
 // kernels, whose operands the caches hold, gained nothing by it or lost waves to the registers
-// (columns at 256: 2317 -> 2715 us).
+// (columns at 256: 2317 -> 2715 us). Nor did the two-group lines, whose threads hold more bins: a
+// gradient at 72^2 x 48 1.22 -> 1.25 ms, at 120^2 1.58 -> 1.57, at 160^2 2.00 -> 2.26, at 240^2 2.96
+// -> 3.35.
 template <class E>
 constexpr bool operands_ahead() {
   if constexpr (requires { E::kMatrix; }) {  // the four-step engine

@@ -137,7 +137,11 @@ __global__ void __launch_bounds__(P::kBlock) k_gp_plane(PlaneArgs a) {
   }
 }
 
-// f.template operator()<P>() with the engines of side n; false for other sides.
+// f.template operator()<P>() with the engines of side n; false for other sides. Both engines of a
+// side here take the same number of threads. Those of 72, 80, 90, 108 and 120 do not (72: 324 for
+// the columns, 648 for the rows), and 100 (1000 for both) has not been tried: these sides go through
+// the three launches, at about the time of their neighbours (an iteration at 72^3 / 80^3 / 96^3 22 /
+// 23 / 23 us, at 100^3 / 108^3 / 120^3 / 128^3 33 / 32 / 38 / 33 us).
 template <class F>
 bool with_plane(int n, F f) {
   switch (n) {

@@ -1,7 +1,7 @@
 // Host ingest and egress. Copies between pageable host memory (numpy arrays, callers' buffers)
 // and the device go through rings of pinned staging slots of the calling thread, chunk by chunk:
 // the host side of each chunk is spread over a small pool of copy threads and overlaps the DMA
-// of the neighbouring chunks. A plain hipMemcpy from pageable memory stages through the
+// of the neighbouring chunk. A plain hipMemcpy from pageable memory stages through the
 // runtime's own buffers with one host thread: 25.7 MB take 754 us in and 1560 us out that way,
 // 1 MB 46 and 65 us; the DMA alone 476 and 27 us, the host copy 190 and 14 us.
 #pragma once

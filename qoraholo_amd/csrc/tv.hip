@@ -19,10 +19,13 @@
 //
 // Per prox of 10 steps, output included (4 + 3 + 3 steps), against two steps per pass and a kernel
 // for the output before: 671 against 837 us at 256^3, 1131 against 2635 us at 320^3, 1952 against
-// 3183 us at 384^3, 158 against 184 us at 128^3 and 73 against 131 us at 64^3. What bounds it: a
-// middle pass moves its 13 volumes at 4-5 TB/s with the halo re-reads (a device copy reaches 4.9),
-// a first or last pass of four stages is near its vector work (42 instructions a point and step,
-// and only 24 of 32 rows and 56 of 64 columns of a tile are its own).
+// 3183 us at 384^3, 158 against 184 us at 128^3 and 73 against 131 us at 64^3. What bounds it: the
+// middle pass moves 978 MB with the halo re-reads, at 4.6 TB/s (a device copy reaches 4.9). The first
+// and last are bound by neither traffic nor vector work alone: of their 206 and 222 us the 722 and 820
+// MB would take 147 and 167, and the vector units of the CUs that hold a block (220 of 256 at 256^3)
+// are busy 64 and 52% of the cycles (48% in the middle pass; 33 instructions a point and step in the
+// first, 47 in its exact form, and only 24 of 32 rows and 56 of 64 columns of a tile are its own). Two
+// waves a SIMD hide the one behind the other in part.
 #include <algorithm>
 #include <atomic>
 

@@ -316,6 +316,10 @@ def test_tv_prox_partial_tiles(device, oracle):
     assert np.max(np.abs(got - want)) < 1e-6
 
 
+# Passes are of up to four steps now, in tiles of 64 columns by 32 rows whatever the row width: what
+# the text below says of pairs of steps, floats per lane, x tiles and chunk lengths is of the kernels
+# these sizes were chosen for. They still cover sides within one tile and over several, row counts
+# that fill the last group of four and that do not, and one to three passes.
 @pytest.mark.parametrize("shape,inner", [((62, 60, 60), 10), ((40, 33, 130), 7), ((70, 128, 100), 4),
                                          ((33, 77, 256), 5), ((256, 256, 256), 10),
                                          ((20, 30, 300), 3), ((44, 50, 128), 6),
@@ -505,6 +509,8 @@ def test_tv_infinities_and_nans_stay_where_the_oracle_has_them(device, oracle):
                                        err_msg=f"{value} at {at}")
 
 
+# As above: sides within one tile and over several, with the output in the last pass and alone (the
+# 256^3 batch), in passes of several steps and of one.
 @pytest.mark.parametrize("shape,inner,batch", [((9, 20, 64), 5, 3), ((16, 16, 128), 4, 3),
                                                ((20, 30, 300), 3, 3), ((12, 18, 302), 5, 3),
                                                ((40, 64, 256), 4, 3), ((256, 256, 256), 4, 2)])

@@ -18,6 +18,7 @@ def _prox_allocating(lib, native, b, lam, inner, fused):
     return x
 
 
+# Passes are of up to four steps now: 5 steps are 3 + 2, and 4 steps of a small volume 2 + 2.
 def test_noalloc_prox_equals_allocating_prox(device):
     import torch
     from qoraholo_amd import _native
