@@ -137,16 +137,18 @@ CopyPool& pool() {
 
 // The calling thread's pinned slots and what marks their last DMA: slots 0 .. kSlots - 1 upload,
 // the others download. A slot grows to what it is used for, so that a thread's small calls pin
-// little. Transfers of one slot on the thread's own stream are marked by that stream alone (an event
-// after each is 10 us of a small call); several in a row, and all on other streams, which may be
-// destroyed before the slot is used again, by the slot's event.
+// little. Transfers of one slot on the thread's own stream, or on that of a StagedStream, are marked by
+// the stream alone (an event after each is 10 us of a small call); several in a row, and all on other
+// streams, which may be destroyed before the slot is used again, by the slot's event.
 struct Staging {
-  std::unique_ptr<Stream> own;  // call_stream()
+  std::unique_ptr<Stream> own;    // call_stream()
+  hipStream_t staged = nullptr;   // of the thread's StagedStream
   PinnedBuffer<char> memory[2 * kSlots];
   Event done[2 * kSlots]{Event(false), Event(false), Event(false), Event(false),
                          Event(false), Event(false), Event(false), Event(false)};
   enum class Mark { none, event, stream };
   Mark mark[2 * kSlots] = {};
+  hipStream_t stream[2 * kSlots] = {};
   int up = 0;
   int down = 0;
 
@@ -154,7 +156,7 @@ struct Staging {
   void wait(int i) {
     const Mark m = std::exchange(mark[i], Mark::none);
     if (m == Mark::event) check(hipEventSynchronize(done[i].get()), "hipEventSynchronize");
-    if (m == Mark::stream) check(hipStreamSynchronize(own->get()), "hipStreamSynchronize");
+    if (m == Mark::stream) check(hipStreamSynchronize(stream[i]), "hipStreamSynchronize");
   }
   // Slot i, its last DMA over, with room for `bytes`.
   char* slot(int i, std::size_t bytes) {
@@ -166,9 +168,16 @@ struct Staging {
     return memory[i].get();
   }
   void queued(int i, hipStream_t s, bool alone) {
-    const bool by_stream = alone && own && s == own->get();
+    const bool by_stream = alone && ((own && s == own->get()) || (staged && s == staged));
     if (!by_stream) done[i].record(s);
     mark[i] = by_stream ? Mark::stream : Mark::event;
+    stream[i] = s;
+  }
+  // s has been waited for.
+  void settled(hipStream_t s) {
+    for (int i = 0; i < 2 * kSlots; ++i) {
+      if (mark[i] == Mark::stream && stream[i] == s) mark[i] = Mark::none;
+    }
   }
 };
 
@@ -222,6 +231,15 @@ hipStream_t call_stream() {
   Staging& st = staging();
   if (!st.own) st.own = std::make_unique<Stream>();
   return st.own->get();
+}
+
+StagedStream::StagedStream(hipStream_t s) : s_(s), outer_(std::exchange(staging().staged, s)) {}
+StagedStream::~StagedStream() {
+  // Settled also after an error: the stream does not run on past it.
+  (void)hipStreamSynchronize(s_);
+  Staging& st = staging();
+  if (!(st.own && s_ == st.own->get())) st.settled(s_);
+  st.staged = outer_;
 }
 
 void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s) {

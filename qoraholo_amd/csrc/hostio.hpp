@@ -34,6 +34,21 @@ void parallel_for(int parts, const std::function<void(int)>& part);
 // independently. It lives as long as the thread's staging slots.
 hipStream_t call_stream();
 
+// While it lives, small transfers of the calling thread on s are waited for with the stream, as on
+// call_stream(), instead of an event each. It waits for s when it ends, so that the staging keeps
+// nothing of a stream that may be destroyed then.
+class StagedStream {
+ public:
+  explicit StagedStream(hipStream_t s);
+  ~StagedStream();
+  StagedStream(const StagedStream&) = delete;
+  StagedStream& operator=(const StagedStream&) = delete;
+
+ private:
+  hipStream_t s_;
+  hipStream_t outer_;
+};
+
 // Device dst <- pageable host src. Returns once src may be reused; the DMA of the last chunks
 // may still be in flight on s, ahead of any later work on s.
 void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s);
@@ -46,8 +61,8 @@ void download(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 // as far as the staging slots go, finish() with every dst complete.
 class Downloads {
  public:
-  // alone: next to nothing is queued behind it on s before finish(), so that on call_stream() it is
-  // waited for with the stream and needs no event.
+  // alone: next to nothing is queued behind it on s before finish(), so that on call_stream() and
+  // a StagedStream it is waited for with the stream and needs no event.
   void add(void* dst, const void* src, std::size_t bytes, hipStream_t s, bool alone = false);
   void finish();
 

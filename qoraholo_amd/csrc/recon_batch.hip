@@ -114,6 +114,7 @@ void ReconBatch::run(const float* const* inputs, float* const* outputs, int nb) 
   const hipStream_t s = stream_.get();
   const std::size_t stack = static_cast<std::size_t>(count_) * n_ * n_;
   const std::size_t vol = static_cast<std::size_t>(solver_.nz()) * solver_.n() * solver_.n();
+  const StagedStream staged(s);
   for (int b = 0; b < nb; ++b) upload(holo_.get() + b * stack, inputs[b], stack * sizeof(float), s);
   if (graphs_ok_) {
     graphs_[nb - 1]->launch(s);
