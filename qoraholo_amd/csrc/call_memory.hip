@@ -4,6 +4,7 @@
 #include <mutex>
 
 #include "runtime.hpp"
+#include "thread_end.hpp"
 
 namespace qh {
 
@@ -146,7 +147,8 @@ std::size_t device_bytes_free() {
 }
 
 CallMemory::CallMemory(hipStream_t s) : s_(s), device_(current_device()), outer_(current_call()) {
-  thread_local ThreadMark mark;
+  thread_local PerThread<ThreadMark> mark;
+  mark.get();
   current_call() = this;
 }
 

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "runtime.hpp"
+#include "thread_end.hpp"
 
 namespace qh {
 
@@ -189,9 +190,8 @@ int next_slot(int& at, bool several) {
 }
 
 Staging& staging() {
-  thread_local std::unique_ptr<Staging> s;
-  if (!s) s = std::make_unique<Staging>();
-  return *s;
+  thread_local PerThread<Staging> s;
+  return s.get();
 }
 
 }  // namespace

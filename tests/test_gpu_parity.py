@@ -255,6 +255,28 @@ def test_gp_complex_passes_match_oracle(device, oracle, qh, n, nz):
         assert filled == want_filled
 
 
+def test_process_may_exit_right_after_threads_made_calls(device):
+    """Threads release their staging and the last one the pool when they end, which is after they
+    have been joined: a process that exits then ends with status 0, whether the release has run, is
+    under way or never starts."""
+    import subprocess
+    import sys
+
+    code = """
+import sys, numpy as np, qoraholo_amd as qh
+from concurrent.futures import ThreadPoolExecutor
+f = np.ones((9, 128, 128), np.complex64)
+with ThreadPoolExecutor(8) as ex:
+    out = list(ex.map(lambda _: qh.rytov(f), range(32)))
+print("joined", len(out), flush=True)
+"""
+    root = str(__import__("pathlib").Path(__file__).resolve().parent.parent)
+    done = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True,
+                          timeout=100)
+    assert done.stdout.strip() == "joined 32"
+    assert done.returncode == 0, done.stderr[-500:]
+
+
 def test_host_transfers_of_every_chunking_are_whole(device):
     """Transfers below and from the sizes where the host copy is split (1.5 MB), where a transfer
     takes several chunks (above 8 MB) and larger ones (above 128 MB), in an order in which slots

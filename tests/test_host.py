@@ -258,3 +258,44 @@ def test_field_ratio_matches_oracle_bitwise(qh, oracle, count, bcount, shape):
     want = oracle.field_ratio(s, b)
     assert got.shape == want.shape
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def test_threads_release_what_they_hold_before_the_process_ends_or_not_at_all(tmp_path):
+    """What a thread keeps of the device (PerThread) against a runtime that exit() takes down: the
+    process may return from main before the thread's release has begun, during it and after it."""
+    import shutil
+    import subprocess
+    from pathlib import Path
+
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    csrc = Path(__file__).resolve().parent.parent / "qoraholo_amd" / "csrc"
+    (tmp_path / "main.cpp").write_text(r"""
+#include <atomic>
+#include <cstdlib>
+#include <thread>
+#include <unistd.h>
+#include "thread_end.hpp"
+struct Runtime { std::atomic<bool> alive{true}; ~Runtime() { alive = false; usleep(60000); } };
+Runtime runtime;
+struct Held {
+  ~Held() {
+    for (int i = 0; i < 10; ++i) {
+      usleep(2000);
+      if (!runtime.alive) _exit(1);
+    }
+  }
+};
+int main(int, char** argv) {
+  static std::atomic<bool> used{false};
+  std::thread([] { thread_local qh::PerThread<Held> held; held.get(); used = true; }).detach();
+  while (!used) usleep(10);
+  usleep(std::atoi(argv[1]));
+  return 0;
+}
+""")
+    exe = tmp_path / "main"
+    subprocess.run(["g++", "-std=c++20", "-O1", "-pthread", f"-I{csrc}", "-x", "c++",
+                    str(tmp_path / "main.cpp"), str(csrc / "thread_end.hip"), "-o", str(exe)], check=True)
+    for wait_us in (0, 300, 5000, 19000, 21000, 50000):
+        assert subprocess.run([str(exe), str(wait_us)], timeout=20).returncode == 0, wait_us
