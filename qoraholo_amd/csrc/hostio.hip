@@ -23,8 +23,12 @@ namespace qh {
 
 namespace {
 
-constexpr int kSlots = 4;  // of each direction
-// Chunks of transfers that take several: two slots in turn. A DMA of 4 MB leaves a gap of a seventh
+// Staging slots: two that transfers in several chunks take in turn, either way, and four in turn for
+// the single chunks of each direction.
+constexpr int kPair = 2;
+constexpr int kRing = 4;
+constexpr int kSlots = kPair + 2 * kRing;
+// Chunks of transfers that take several. A DMA of 4 MB leaves a gap of a seventh
 // of its time to the next one (128 / 256 MB in and out: 7.0 / 13.0 ms in chunks of 4 MB, 5.5 / 10.7 of
 // 8, 5.4 / 10.4 of 16), and the first and last host copy of a smaller transfer wait for less in
 // smaller chunks (24 MB: 1.21 ms of 8, 1.27 to 1.33 of 16).
@@ -136,20 +140,21 @@ CopyPool& pool() {
   return p;
 }
 
-// The calling thread's pinned slots and what marks their last DMA: slots 0 .. kSlots - 1 upload,
-// the others download. A slot grows to what it is used for, so that a thread's small calls pin
-// little. Transfers of one slot on the thread's own stream, or on that of a StagedStream, are marked by
-// the stream alone (an event after each is 10 us of a small call); several in a row, and all on other
-// streams, which may be destroyed before the slot is used again, by the slot's event.
+// The calling thread's pinned slots and what marks their last DMA. A slot grows to what it is used
+// for, so that a thread's small calls pin little. Transfers of one slot on the thread's own stream, or
+// on that of a StagedStream, are marked by the stream alone (an event after each is 10 us of a small
+// call); several in a row, and all on other streams, which may be destroyed before the slot is used
+// again, by the slot's event.
 struct Staging {
-  std::unique_ptr<Stream> own;    // call_stream()
-  hipStream_t staged = nullptr;   // of the thread's StagedStream
-  PinnedBuffer<char> memory[2 * kSlots];
-  Event done[2 * kSlots]{Event(false), Event(false), Event(false), Event(false),
-                         Event(false), Event(false), Event(false), Event(false)};
+  std::unique_ptr<Stream> own;   // call_stream()
+  hipStream_t staged = nullptr;  // of the thread's StagedStream
+  PinnedBuffer<char> memory[kSlots];
+  Event done[kSlots]{Event(false), Event(false), Event(false), Event(false), Event(false),
+                     Event(false), Event(false), Event(false), Event(false), Event(false)};
   enum class Mark { none, event, stream };
-  Mark mark[2 * kSlots] = {};
-  hipStream_t stream[2 * kSlots] = {};
+  Mark mark[kSlots] = {};
+  hipStream_t stream[kSlots] = {};
+  int pair = 0;
   int up = 0;
   int down = 0;
 
@@ -174,20 +179,19 @@ struct Staging {
     mark[i] = by_stream ? Mark::stream : Mark::event;
     stream[i] = s;
   }
+  // The slot of the next chunk.
+  int next(bool several, bool download) {
+    if (several) return std::exchange(pair, (pair + 1) % kPair);
+    int& at = download ? down : up;
+    return kPair + (download ? kRing : 0) + std::exchange(at, (at + 1) % kRing);
+  }
   // s has been waited for.
   void settled(hipStream_t s) {
-    for (int i = 0; i < 2 * kSlots; ++i) {
+    for (int i = 0; i < kSlots; ++i) {
       if (mark[i] == Mark::stream && stream[i] == s) mark[i] = Mark::none;
     }
   }
 };
-
-// The next slot of a ring at `at`: of all slots, or of two for a transfer in several chunks.
-int next_slot(int& at, bool several) {
-  const int i = at % (several ? 2 : kSlots);
-  at = (i + 1) % kSlots;
-  return i;
-}
 
 Staging& staging() {
   thread_local PerThread<Staging> s;
@@ -249,7 +253,7 @@ void upload(void* dst, const void* src, std::size_t bytes, hipStream_t s) {
   const std::size_t chunk = chunk_of(bytes);
   for (std::size_t off = 0; off < bytes; off += chunk) {
     const std::size_t len = std::min(chunk, bytes - off);
-    const int i = next_slot(st.up, bytes > chunk);
+    const int i = st.next(bytes > chunk, false);
     char* const slot = st.slot(i, len);
     host_copy(slot, h + off, len);
     check(hipMemcpyAsync(d + off, slot, len, hipMemcpyHostToDevice, s), "upload");
@@ -264,7 +268,7 @@ void Downloads::add(void* dst, const void* src, std::size_t bytes, hipStream_t s
   const std::size_t chunk = chunk_of(bytes);
   for (std::size_t off = 0; off < bytes; off += chunk) {
     const std::size_t len = std::min(chunk, bytes - off);
-    const int i = kSlots + next_slot(st.down, bytes > chunk);
+    const int i = st.next(bytes > chunk, true);
     while (std::any_of(parts_.begin(), parts_.end(), [&](const Part& p) { return p.slot == i; })) {
       retire();
     }
