@@ -7,9 +7,10 @@
 //
 // The pool keeps at most kPoolBytes per process, frees blocks that kPoolCalls calls in a row did
 // not take, and is freed when an allocation of the library runs out of memory and when the last
-// thread that made calls ends. Blocks are handed over only after the stream that used them has been
-// waited for, so any thread and stream may take them. Other allocators of the process do not see the
-// pool: one that runs out (torch's, say) finds up to kPoolBytes less than before.
+// thread that made calls ends before the process does. Blocks are handed over only after the stream
+// that used them has been waited for, so any thread and stream may take them. Other allocators of the
+// process do not see the pool: one that runs out (torch's, say) finds up to kPoolBytes less than
+// before.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -542,10 +542,11 @@ template <int T>
 void launch_steps_of(const StepArgs& a, hipStream_t s, int batch, bool exact) {
   if (a.x) {
     if constexpr (T < kMaxSteps) launch_steps<T, false, true>(a, s, batch, exact);
-  } else if (T >= 3 && a.first) {
-    // The first of several passes, of 3 or 4 steps: without p_{k-1} at all (256^3: 193 against 200 us
-    // for 3 steps, 219 against 240 us for 4; 384^3: 529 against 550 us for 3).
-    launch_steps<T, T >= 3, false>(a, s, batch, exact);
+  } else if (T >= 2 && a.first) {
+    // The first of several passes, of 2 to 4 steps: without p_{k-1} at all (256^3: 193 against 200 us
+    // for 3 steps, 219 against 240 us for 4; 384^3: 529 against 550 us for 3; a prox of 2 + 2 steps at
+    // 128^3 79.5 against 81.5 us).
+    launch_steps<T, T >= 2, false>(a, s, batch, exact);
   } else {
     launch_steps<T, false, false>(a, s, batch, exact);
   }
